@@ -50,6 +50,37 @@ def test_forward_and_gradients_match_fp64_oracle(D, H, B):
         m.close()
 
 
+@pytest.mark.parametrize("D,H,B", [(1, 1, 5), (33, 40, 31), (18, 64, 129), (64, 128, 257), (20, 112, 128),
+                                   (65, 16, 100), (10, 129, 64)])
+def test_small_network_kernels_at_their_edges(D, H, B):
+    """Padding of inputs, units, groups of 32 and chunks of 128 samples, the
+    largest small network and the first sizes beyond it; a larger batch on the
+    same model first, whose rows must not show in the smaller one's sums."""
+    p, x, t = problem(D, H, B + 300, seed=7 * D + H + B)
+    m = GpuMlp(D, H, B + 300)
+    try:
+        m.set_params(p)
+        m.train(x, t, 2, 1e-3)
+        m.set_params(p)
+        y = m.forward(x[:B])
+        y64 = omlp.forward(p.astype(np.float64), x[:B].astype(np.float64), D, H)
+        assert np.allclose(y, y64, rtol=1e-5, atol=1e-5 * (1 + np.abs(y64).max()))
+        loss, g = m.loss_grad(x[:B], t[:B])
+        L64, g64 = omlp.loss_grad(p.astype(np.float64), x[:B].astype(np.float64), t[:B].astype(np.float64), D, H)
+        assert abs(loss - L64) <= 1e-5 * max(1.0, L64)
+        assert np.abs(g - g64).max() <= 2e-5 * np.abs(g64).max() + 1e-7
+        # One Adam step from zero moments moves each parameter by lr sign(g)
+        # where the gradient is well away from zero.
+        lr = 1e-3
+        curve = m.train(x[:B], t[:B], 1, lr)
+        assert curve[0] == np.float32(loss)
+        sure = np.abs(g64) > 1e-3 * np.abs(g64).max()
+        step = m.get_params().astype(np.float64) - p
+        assert np.abs(step + lr * np.sign(g64))[sure].max() <= 1e-3 * lr + 2.0 ** -23 * np.abs(p).max()
+    finally:
+        m.close()
+
+
 def test_training_reduces_loss_and_fits():
     rng = np.random.default_rng(3)
     X = rng.uniform(-2, 2, size=(4000, 6))
