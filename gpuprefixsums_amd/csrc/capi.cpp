@@ -96,8 +96,6 @@ void free_handle(gps_handle* h) {
     delete h;
 }
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 int check_scan_args(gps_handle* h, const void* in, const void* out, uint64_t n) {
     if (!h) return fail(GPS_ERR_INVALID, "null handle");
     if (int rc_ = gps::check_device(h)) return rc_;
@@ -132,9 +130,8 @@ int scan_u32(gps_handle* h, const uint32_t* in, uint32_t* out, uint64_t n, bool 
         return fail(GPS_ERR_UNSUPPORTED, "carries are offered by the CSDL tile and persistent schedules");
     const uint32_t tile = kernel_tile(shape, schedule);
     const uint32_t tiles = (uint32_t)((n + tile - 1) / tile);
-    const uint32_t vec_ok = aligned16(in) && aligned16(out);
     if (h->algo == GPS_ALGO_RTS) {
-        HIP_TRY(gps::launch_rts_u32(shape, inclusive, in, out, n, tiles, vec_ok, h->tile_sums, s));
+        HIP_TRY(gps::launch_rts_u32(shape, inclusive, in, out, n, tiles, h->tile_sums, s));
         return GPS_OK;
     }
     HIP_TRY(gps::before_epoch_launch(h, s));
@@ -143,7 +140,6 @@ int scan_u32(gps_handle* h, const uint32_t* in, uint32_t* out, uint64_t n, bool 
     p.out = out;
     p.n = n;
     p.num_tiles = tiles;
-    p.vec_ok = vec_ok;
     p.status = h->status;
     p.ticket = h->ticket;
     p.err = h->err;

@@ -11,8 +11,6 @@ using gps::hip_fail;
 
 namespace {
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 // The persistent segmented kernel unless the handle asks for one workgroup
 // per tile.
 bool seg_persistent(const gps_handle* h) { return h->schedule != GPS_SCHEDULE_TILE; }
@@ -65,7 +63,7 @@ int enqueue_segmented(gps_handle* h, const uint32_t* in, uint32_t* out, const ui
     if (n == 0) return GPS_OK;
     HIP_TRY(gps::before_epoch_launch(h, s));
     HIP_TRY(gps::launch_segscan_u32(seg_shape(h, n), inclusive, seg_persistent(h), in, out, offsets, num_segments, n,
-                                    aligned16(in) && aligned16(out), h->status, h->ticket, h->err, s));
+                                    h->status, h->ticket, h->err, s));
     return GPS_OK;
 }
 
@@ -96,11 +94,10 @@ int scan_fp(gps_handle* h, const void* in, float* out, uint64_t n, bool bf16, in
     if ((ia & (bf16 ? 1u : 3u)) || (oa & 3u)) return fail(GPS_ERR_INVALID, "misaligned buffer");
     if (n == 0) return GPS_OK;
     const gps::TileShape s = fp_shape(h, n, false);
-    const uint32_t vec_ok = ((ia & (bf16 ? 7u : 15u)) == 0) && ((oa & 15u) == 0);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
-    HIP_TRY(gps::launch_scan_fp(s, bf16, compensated, fp_persistent(h, n), in, out, n, vec_ok, h->status, h->ticket,
-                                h->err, st));
+    HIP_TRY(gps::launch_scan_fp(s, bf16, compensated, fp_persistent(h, n), in, out, n, h->status, h->ticket, h->err,
+                                st));
     return GPS_OK;
 }
 
@@ -132,10 +129,9 @@ int segscan_fp(gps_handle* h, const void* in, float* out, const uint64_t* offset
     if (n == 0) return GPS_OK;
     const bool persistent = segfp_persistent(h, n);
     const gps::TileShape s = persistent && h->size_adaptive ? gps::TileShape{1024, 8} : fp_shape(h, n, true);
-    const uint32_t vec_ok = ((ia & (bf16 ? 7u : 15u)) == 0) && ((oa & 15u) == 0);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
-    HIP_TRY(gps::launch_segscan_fp(s, bf16, compensated != 0, persistent, in, out, offsets, num_segments, n, vec_ok,
+    HIP_TRY(gps::launch_segscan_fp(s, bf16, compensated != 0, persistent, in, out, offsets, num_segments, n,
                                    h->status, h->ticket, h->err, st));
     return GPS_OK;
 }
@@ -226,8 +222,7 @@ int gps_segmented_graph_create(gps_handle* h, const uint32_t* d_in, uint32_t* d_
         // No re-arm check inside a capture: a graph node must not depend on
         // the host-side launch count (gps_reset re-arms explicitly).
         rc = n ? (gps::launch_segscan_u32(seg_shape(h, n), inclusive != 0, seg_persistent(h), d_in, d_out, d_offsets,
-                                          num_segments, n, aligned16(d_in) && aligned16(d_out), h->status,
-                                          h->ticket, h->err, s) == hipSuccess
+                                          num_segments, n, h->status, h->ticket, h->err, s) == hipSuccess
                       ? GPS_OK
                       : GPS_ERR_HIP)
                : GPS_OK;
@@ -318,7 +313,6 @@ int gps_estimate_occupancy(gps_handle* h, const uint32_t* d_in, uint32_t* d_out,
         p.out = d_out;
         p.n = n;
         p.num_tiles = (uint32_t)((n + tile - 1) / tile);
-        p.vec_ok = aligned16(d_in) && aligned16(d_out);
         p.status = h->status;
         p.ticket = h->ticket;
         p.err = h->err;

@@ -24,7 +24,6 @@ struct ScanParams {
     uint32_t* out;
     uint64_t n;
     uint32_t num_tiles;
-    uint32_t vec_ok;  // in and out are 16-byte aligned
     uint64_t* status;  // one word per tile
     uint64_t* ticket;  // (epoch << 32) | tickets taken
     uint32_t* err;     // device error bits (watchdogs)
@@ -136,7 +135,7 @@ hipError_t launch_csdldf_split_u32(TileShape s, bool inclusive, const ScanParams
 // Persistent decoupled-fallback scan (grid = resident workgroups).
 hipError_t launch_csdldf_pp_u32(TileShape s, bool inclusive, const ScanParams& p, hipStream_t stream);
 hipError_t launch_rts_u32(TileShape s, bool inclusive, const uint32_t* in, uint32_t* out, uint64_t n,
-                          uint32_t num_tiles, uint32_t vec_ok, uint32_t* tile_sums, hipStream_t stream);
+                          uint32_t num_tiles, uint32_t* tile_sums, hipStream_t stream);
 
 // Batched segmented scan in one launch: persistent (grid = resident
 // workgroups, pipelined) or one workgroup per tile.
@@ -145,7 +144,7 @@ bool seg_shape_supported(TileShape s, bool persistent);
 // stream capture, so the capture holds only the launch).
 hipError_t prepare_segscan_u32(TileShape s, bool inclusive, bool persistent);
 hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, const uint32_t* in, uint32_t* out,
-                              const uint64_t* offsets, uint64_t num_segments, uint64_t n, uint32_t vec_ok,
+                              const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                               uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream);
 
 // FP32 / BF16-input inclusive scans with FP32 output (2 status words per tile).
@@ -155,12 +154,12 @@ enum FpCarry : int { kFpPlain = 0, kFpPair = 1 };
 // persistent: resident workgroups loop over ticketed tiles, loading tile i+1
 // while tile i's lookback resolves (otherwise one workgroup per tile).
 hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, const void* in, float* out,
-                          uint64_t n, uint32_t vec_ok, uint64_t* status, uint64_t* ticket, uint32_t* err,
+                          uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
                           hipStream_t stream);
 // Batched segmented FP inclusive scan (one launch; same shapes as launch_scan_fp;
 // persistent as there).
 hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, const void* in, float* out,
-                             const uint64_t* offsets, uint64_t num_segments, uint64_t n, uint32_t vec_ok,
+                             const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                              uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream);
 
 // Member-wise scan of n 4-member uint32 structs (4 status words per tile).

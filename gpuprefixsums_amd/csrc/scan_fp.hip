@@ -162,7 +162,6 @@ struct FpParams {
     float* out;
     uint64_t n;
     uint32_t num_tiles;
-    uint32_t vec_ok;
     uint64_t* status;  // 2 words per tile
     uint64_t* ticket;
     uint32_t* err;
@@ -171,38 +170,61 @@ struct FpParams {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
+// Tile input and output as the uint32 tiles' (tile_u32.hpp): vectors from any
+// element address, outputs and partial FP32 inputs through a raw buffer that
+// ends at n, the ordinary load policy for inputs the Infinity Cache holds. A
+// BF16 buffer ends at the last whole dword; an odd last element is added.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef u16x4 u16x4_any __attribute__((aligned(2)));
+
+__device__ __forceinline__ f32x4 widen(u16x4 b) {
+    f32x4 x;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) x[c] = __builtin_bit_cast(float, (uint32_t)b[c] << 16);
+    return x;
+}
+
 template <bool BF16, int VEC>
-__device__ __forceinline__ void load_fp(f32x4 (&x)[VEC], const void* in, uint64_t base, uint64_t n, bool vec_path) {
-    if (vec_path) {
+__device__ __forceinline__ void load_fp(f32x4 (&x)[VEC], const void* in, uint64_t start, uint64_t n,
+                                        uint32_t tile_elems) {
+    const uint32_t valid = tile_valid(start, n, tile_elems), at = thread_offset<VEC>();
+    if (BF16) {
+        const uint16_t* const p = static_cast<const uint16_t*>(in) + start;
+        u16x4 d[VEC];
+        if (valid == tile_elems && 2u * n > kCachedBytes) {
+            const u16x4_any* const v = reinterpret_cast<const u16x4_any*>(p + at);
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            if (BF16) {
-                const u16x4 b = __builtin_nontemporal_load(reinterpret_cast<const u16x4*>(
-                    static_cast<const uint16_t*>(in) + base + (uint64_t)k * 256u));
+            for (int k = 0; k < VEC; ++k) d[k] = __builtin_nontemporal_load(v + k * 64);
+        } else {
+            const __amdgpu_buffer_rsrc_t r = raw_buffer(p, 2u * (valid & ~1u));
 #pragma unroll
-                for (int c = 0; c < 4; ++c) x[k][c] = __builtin_bit_cast(float, (uint32_t)b[c] << 16);
-            } else {
-                x[k] = __builtin_nontemporal_load(
-                    reinterpret_cast<const f32x4*>(static_cast<const float*>(in) + base + (uint64_t)k * 256u));
+            for (int k = 0; k < VEC; ++k)
+                d[k] = __builtin_bit_cast(u16x4, __builtin_amdgcn_raw_buffer_load_b64(r, 2u * at + k * 512u, 0, 0));
+            if (valid & 1u) {  // the element that fills half of the buffer's last dword
+                const uint16_t last = p[valid - 1u];
+#pragma unroll
+                for (int k = 0; k < VEC; ++k)
+#pragma unroll
+                    for (int c = 0; c < 4; c += 2) d[k][c] = at + k * 256u + c == valid - 1u ? last : d[k][c];
             }
         }
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) x[k] = widen(d[k]);
     } else {
+        u32x4 d[VEC];
+        load_tile<VEC>(d, static_cast<const uint32_t*>(in), start, n, tile_elems);
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-                float v = 0.f;
-                if (i < n) {
-                    if (BF16)
-                        v = __builtin_bit_cast(float, (uint32_t)static_cast<const uint16_t*>(in)[i] << 16);
-                    else
-                        v = static_cast<const float*>(in)[i];
-                }
-                x[k][c] = v;
-            }
-        }
+        for (int k = 0; k < VEC; ++k) x[k] = __builtin_bit_cast(f32x4, d[k]);
     }
+}
+
+template <int VEC>
+__device__ __forceinline__ void store_fp(float* out, const f32x4 (&x)[VEC], uint64_t start, uint64_t n,
+                                         uint32_t tile_elems) {
+    u32x4 d[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) d[k] = __builtin_bit_cast(u32x4, x[k]);
+    store_tile<VEC>(reinterpret_cast<uint32_t*>(out), d, 0u, start, n, tile_elems);
 }
 
 template <int BLOCK, int VEC, bool BF16, bool COMP>
@@ -219,11 +241,9 @@ __global__ __launch_bounds__(BLOCK) void scan_fp(FpParams p) {
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    const uint32_t tile = s_ticket[0], epoch = s_ticket[1];
-    const uint64_t base = thread_base<BLOCK, VEC>(tile);
-    const bool vec_path = p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n);
+    const uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]), epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     f32x4 x[VEC];
-    load_fp<BF16, VEC>(x, p.in, base, p.n, vec_path);
+    load_fp<BF16, VEC>(x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
 
     // Per vector: lane total (pair), wave exclusive scan -> lane carry L_k.
     ff lane_carry[VEC];
@@ -287,19 +307,7 @@ __global__ __launch_bounds__(BLOCK) void scan_fp(FpParams p) {
         }
         x[k] = y;
     }
-    if (vec_path) {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k)
-            __builtin_nontemporal_store(x[k], reinterpret_cast<f32x4*>(p.out + base + (uint64_t)k * 256u));
-    } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-                if (i < p.n) p.out[i] = x[k][c];
-            }
-    }
+    store_fp<VEC>(p.out, x, (uint64_t)tile * C::kTile, p.n, C::kTile);
 }
 
 // ---------------------------------------------------------------------------
@@ -408,12 +416,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
 
     f32x4 x[VEC], y[VEC];
-    load_fp<BF16, VEC>(x, p.in, thread_base<BLOCK, VEC>(tile), p.n, p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n));
+    load_fp<BF16, VEC>(x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
 
     while (true) {
         // Per vector: lane total, wave exclusive scan -> lane carry.
@@ -439,7 +447,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             s_ticket[2] = take_ticket(p.ticket, total_tickets).tile;
         }
         __syncthreads();
-        const uint32_t next = s_ticket[2];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
         const bool has_next = next < p.num_tiles;
 
         LookbackW2<Ops> lb;
@@ -448,8 +456,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             lb.issue(p.status, epoch);
         }
         if (has_next)
-            load_fp<BF16, VEC>(y, p.in, thread_base<BLOCK, VEC>(next), p.n,
-                               p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n));
+            load_fp<BF16, VEC>(y, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         if (wave == 0) {
             T prefix = Ops::zero();
             if (tile != 0) {
@@ -472,22 +479,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             }
             x[k] = o;
         }
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n)) {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-                __builtin_nontemporal_store(x[k], reinterpret_cast<f32x4*>(p.out + base + (uint64_t)k * 256u));
-        } else {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-                    if (i < p.n) p.out[i] = x[k][c];
-                }
-        }
+        store_fp<VEC>(p.out, x, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) x[k] = y[k];
         tile = next;
     }
@@ -543,7 +536,6 @@ struct SegFpParams {
     uint64_t num_segments;
     uint64_t n;
     uint32_t num_tiles;
-    uint32_t vec_ok;
     uint64_t* status;  // 2 words per tile
     uint64_t* ticket;
     uint32_t* err;
@@ -568,13 +560,11 @@ __global__ __launch_bounds__(BLOCK) void segscan_fp(SegFpParams p) {
     }
     for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[i] = 0u;
     __syncthreads();
-    const uint32_t tile = s_ticket[0], epoch = s_ticket[1];
+    const uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]), epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     const uint64_t a = (uint64_t)tile * C::kTile;
     const uint64_t b = a + C::kTile < p.n ? a + C::kTile : p.n;
-    const uint64_t base = thread_base<BLOCK, VEC>(tile);
-    const bool vec_path = p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n);
     f32x4 x[VEC];
-    load_fp<BF16, VEC>(x, p.in, base, p.n, vec_path);  // the head search overlaps these loads
+    load_fp<BF16, VEC>(x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);  // the head search overlaps these loads
 
     if (wave == 0) {
         const uint64_t s0 = find_first_segment(p.offsets, p.num_segments, a);
@@ -671,19 +661,7 @@ __global__ __launch_bounds__(BLOCK) void segscan_fp(SegFpParams p) {
         }
         x[k] = y;
     }
-    if (vec_path) {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k)
-            __builtin_nontemporal_store(x[k], reinterpret_cast<f32x4*>(p.out + base + (uint64_t)k * 256u));
-    } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-                if (i < p.n) p.out[i] = x[k][c];
-            }
-    }
+    store_fp<VEC>(p.out, x, (uint64_t)tile * C::kTile, p.n, C::kTile);
 }
 
 // Persistent, software-pipelined form of segscan_fp (the segscan_pp_u32
@@ -714,12 +692,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     }
     for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[0][i] = 0u;
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
 
     f32x4 x[VEC], y[VEC];
-    load_fp<BF16, VEC>(x, p.in, thread_base<BLOCK, VEC>(tile), p.n, p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n));
+    load_fp<BF16, VEC>(x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
     {
         const uint64_t lo = (uint64_t)tile * C::kTile;
         const uint64_t hi = lo + C::kTile < p.n ? lo + C::kTile : p.n;
@@ -793,7 +771,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         // the other head buffer was last read by the previous tile's output pass
         for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[cur ^ 1u][i] = 0u;
         __syncthreads();
-        const uint32_t next = s_ticket[2];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
         const bool has_next = next < p.num_tiles;
 
         LookbackW2<Ops> lb;
@@ -808,8 +786,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             mark_heads_by(s_heads[cur ^ 1u], p.offsets, p.num_segments, s0, lo, hi, next == 0, lane, kWave);
         }
         if (has_next)
-            load_fp<BF16, VEC>(y, p.in, thread_base<BLOCK, VEC>(next), p.n,
-                               p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n));
+            load_fp<BF16, VEC>(y, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         if (wave == 0) {
             ff prefix = {0.f, 0.f};
             if (need_lookback) {
@@ -838,22 +815,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             }
             x[k] = o;
         }
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n)) {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-                __builtin_nontemporal_store(x[k], reinterpret_cast<f32x4*>(p.out + base + (uint64_t)k * 256u));
-        } else {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-                    if (i < p.n) p.out[i] = x[k][c];
-                }
-        }
+        store_fp<VEC>(p.out, x, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) x[k] = y[k];
         tile = next;
         cur ^= 1u;
@@ -948,12 +911,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
 
     f32x4 x[VEC], y[VEC];
-    load_fp<BF16, VEC>(x, p.in, thread_base<BLOCK, VEC>(tile), p.n, p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n));
+    load_fp<BF16, VEC>(x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
 
     while (true) {
         // Lane total of the lane's consecutive run, then one pair wave scan.
@@ -983,7 +946,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             s_ticket[2] = take_ticket(p.ticket, total_tickets).tile;
         }
         __syncthreads();
-        const uint32_t next = s_ticket[2];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
         const bool has_next = next < p.num_tiles;
 
         LookbackW2<Ops> lb;
@@ -992,8 +955,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             lb.issue(p.status, epoch);
         }
         if (has_next)
-            load_fp<BF16, VEC>(y, p.in, thread_base<BLOCK, VEC>(next), p.n,
-                               p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n));
+            load_fp<BF16, VEC>(y, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         if (wave == 0) {
             T prefix = Ops::zero();
             if (tile != 0) {
@@ -1017,22 +979,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             x[q] = o;
         }
         blocked_to_striped<VEC>(x, slice);
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n)) {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-                __builtin_nontemporal_store(x[k], reinterpret_cast<f32x4*>(p.out + base + (uint64_t)k * 256u));
-        } else {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-                    if (i < p.n) p.out[i] = x[k][c];
-                }
-        }
+        store_fp<VEC>(p.out, x, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) x[k] = y[k];
         tile = next;
     }
@@ -1081,12 +1029,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     }
     for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[0][i] = 0u;
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
 
     f32x4 x[VEC], y[VEC];
-    load_fp<BF16, VEC>(x, p.in, thread_base<BLOCK, VEC>(tile), p.n, p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n));
+    load_fp<BF16, VEC>(x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
     {
         const uint64_t lo = (uint64_t)tile * C::kTile;
         const uint64_t hi = lo + C::kTile < p.n ? lo + C::kTile : p.n;
@@ -1152,7 +1100,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         // the other head buffer was last read by the previous tile's output pass
         for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[cur ^ 1u][i] = 0u;
         __syncthreads();
-        const uint32_t next = s_ticket[2];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
         const bool has_next = next < p.num_tiles;
 
         LookbackW2<Ops> lb;
@@ -1167,8 +1115,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             mark_heads_by(s_heads[cur ^ 1u], p.offsets, p.num_segments, s0, lo, hi, next == 0, lane, kWave);
         }
         if (has_next)
-            load_fp<BF16, VEC>(y, p.in, thread_base<BLOCK, VEC>(next), p.n,
-                               p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n));
+            load_fp<BF16, VEC>(y, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         if (wave == 0) {
             ff prefix = {0.f, 0.f};
             if (need_lookback) {
@@ -1217,22 +1164,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             }
         }
         blocked_to_striped<VEC>(x, slice);
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n)) {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-                __builtin_nontemporal_store(x[k], reinterpret_cast<f32x4*>(p.out + base + (uint64_t)k * 256u));
-        } else {
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-                    if (i < p.n) p.out[i] = x[k][c];
-                }
-        }
+        store_fp<VEC>(p.out, x, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) x[k] = y[k];
         tile = next;
         cur ^= 1u;
@@ -1280,7 +1213,7 @@ static hipError_t launch_fp_pp_carry(int carry, const FpParams& p, hipStream_t s
 }
 
 hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, const void* in, float* out,
-                          uint64_t n, uint32_t vec_ok, uint64_t* status, uint64_t* ticket, uint32_t* err,
+                          uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
                           hipStream_t stream) {
     const bool compensated = carry == kFpPair;
     FpParams p{};
@@ -1288,7 +1221,6 @@ hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, co
     p.out = out;
     p.n = n;
     p.num_tiles = (uint32_t)((n + s.tile() - 1) / s.tile());
-    p.vec_ok = vec_ok;
     p.status = status;
     p.ticket = ticket;
     p.err = err;
@@ -1330,7 +1262,7 @@ static hipError_t launch_segfp_pp(const SegFpParams& p, hipStream_t stream) {
 }
 
 hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, const void* in, float* out,
-                             const uint64_t* offsets, uint64_t num_segments, uint64_t n, uint32_t vec_ok,
+                             const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                              uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream) {
     SegFpParams p{};
     p.in = in;
@@ -1339,7 +1271,6 @@ hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool pers
     p.num_segments = num_segments;
     p.n = n;
     p.num_tiles = (uint32_t)((n + s.tile() - 1) / s.tile());
-    p.vec_ok = vec_ok;
     p.status = status;
     p.ticket = ticket;
     p.err = err;

@@ -26,8 +26,6 @@ struct TileFront {
     using C = TileCfg<BLOCK, VEC>;
     u32x4 d[VEC];
     uint32_t tile, epoch, wave_prefix, tile_total;
-    uint64_t base;
-    bool vec_path;
 
     __device__ __forceinline__ void run(const ScanParams& p, uint32_t* s_wave, uint32_t* s_ticket) {
         const uint32_t wave = wave_index();
@@ -43,14 +41,9 @@ struct TileFront {
             }
         }
         __syncthreads();
-        tile = s_ticket[0];
-        epoch = s_ticket[1];
-        base = thread_base<BLOCK, VEC>(tile);
-        vec_path = p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n);
-        if (vec_path)
-            load_vec<VEC>(d, p.in + base);
-        else
-            load_guarded<VEC>(d, p.in, base, p.n);
+        tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+        epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
+        load_tile<VEC>(d, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
         const uint32_t run_total = wave_scan_run<VEC, INCL>(d);
         if (lane_id() == 0) s_wave[wave] = run_total;
         __syncthreads();
@@ -58,10 +51,7 @@ struct TileFront {
     }
 
     __device__ __forceinline__ void store(const ScanParams& p, uint32_t add) {
-        if (vec_path)
-            store_vec<VEC>(p.out + base, d, add);
-        else
-            store_guarded<VEC>(p.out, d, add, base, p.n);
+        store_tile<VEC>(p.out, d, add, (uint64_t)tile * C::kTile, p.n, C::kTile);
     }
 };
 
@@ -148,17 +138,13 @@ csdl_pp_u32(ScanParams p) {
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
     if (threadIdx.x == 0) atomic_add_counter(p.occupancy, 1ull);
 
     u32x4 a[VEC], b[VEC];
-    const uint64_t base = thread_base<BLOCK, VEC>(tile);
-    if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n))
-        load_vec<VEC>(a, p.in + base);
-    else
-        load_guarded<VEC>(a, p.in, base, p.n);
+    load_tile<VEC>(a, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
 
     while (true) {
         const uint32_t run = wave_scan_run<VEC, INCL>(a);
@@ -180,7 +166,7 @@ csdl_pp_u32(ScanParams p) {
             s_ticket[2] = take_ticket(p.ticket, total_tickets).tile;
         }
         __syncthreads();
-        const uint32_t next = s_ticket[2];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
         const bool has_next = next < p.num_tiles;
 
         Lookback lb;
@@ -189,11 +175,7 @@ csdl_pp_u32(ScanParams p) {
             lb.issue(p.status, epoch);
         }
         if (has_next) {
-            const uint64_t next_base = thread_base<BLOCK, VEC>(next);
-            if (p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n))
-                load_vec<VEC>(b, p.in + next_base);
-            else
-                load_guarded<VEC>(b, p.in, next_base, p.n);
+            load_tile<VEC>(b, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         }
         if (wave == 0) {
             uint32_t prefix = tile == 0 ? s_carry : 0u;  // tile 0 starts from the carry-in
@@ -209,13 +191,8 @@ csdl_pp_u32(ScanParams p) {
         }
         __syncthreads();
         const uint32_t add = s_prefix + wave_prefix;
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n))
-            store_vec<VEC>(p.out + base, a, add);
-        else
-            store_guarded<VEC>(p.out, a, add, base, p.n);
+        store_tile<VEC>(p.out, a, add, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) a[k] = b[k];
         tile = next;
     }
@@ -262,7 +239,7 @@ template <int DW, int VEC, bool INCL>
 __global__ __launch_bounds__(64 * (DW + 1)) __attribute__((amdgpu_waves_per_eu(VEC >= 8 ? 4 : GPS_WAVES_PER_EU))) void
 csdl_cw_u32(ScanParams p) {
     constexpr uint32_t kWaveElems = 256u * VEC;
-    constexpr uint64_t kTile = (uint64_t)DW * kWaveElems;
+    constexpr uint32_t kTile = DW * kWaveElems;
     __shared__ uint32_t s_tot[2][DW];
     __shared__ uint32_t s_arrived[DW];
     __shared__ uint32_t s_ticket[2];
@@ -327,16 +304,10 @@ csdl_cw_u32(ScanParams p) {
 
     // ---- data waves ----
     if (!lds_wait_ge(&s_ticket_seq, 1u, p.err)) return;
-    uint32_t tile = s_ticket[0];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
     if (tile >= p.num_tiles) return;
     u32x4 a[VEC], b[VEC];
-    {
-        const uint64_t base = (uint64_t)tile * kTile + wave * kWaveElems + lane * 4u;
-        if (p.vec_ok && (uint64_t)(tile + 1u) * kTile <= p.n)
-            load_vec<VEC>(a, p.in + base);
-        else
-            load_guarded<VEC>(a, p.in, base, p.n);
-    }
+    load_tile<VEC>(a, p.in, (uint64_t)tile * kTile, p.n, kTile);
     for (uint32_t i = 0;; ++i) {
         const uint32_t run = wave_scan_run<VEC, INCL>(a);
         if (lane == 0) {
@@ -344,25 +315,16 @@ csdl_cw_u32(ScanParams p) {
             lds_release(&s_arrived[wave], i + 1u);
         }
         if (!lds_wait_ge(&s_ticket_seq, i + 2u, p.err)) return;
-        const uint32_t next = s_ticket[(i + 1u) & 1u];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[(i + 1u) & 1u]);
         const bool has_next = next < p.num_tiles;
         if (has_next) {
-            const uint64_t nb = (uint64_t)next * kTile + wave * kWaveElems + lane * 4u;
-            if (p.vec_ok && (uint64_t)(next + 1u) * kTile <= p.n)
-                load_vec<VEC>(b, p.in + nb);
-            else
-                load_guarded<VEC>(b, p.in, nb, p.n);
+            load_tile<VEC>(b, p.in, (uint64_t)next * kTile, p.n, kTile);
         }
         if (!lds_wait_ge(&s_prefix_seq, i + 1u, p.err)) return;
         const uint32_t wp = wave_sum(lane < wave ? s_tot[i & 1u][lane] : 0u);
         const uint32_t add = s_prefix[i & 1u] + wp;
-        const uint64_t base = (uint64_t)tile * kTile + wave * kWaveElems + lane * 4u;
-        if (p.vec_ok && (uint64_t)(tile + 1u) * kTile <= p.n)
-            store_vec<VEC>(p.out + base, a, add);
-        else
-            store_guarded<VEC>(p.out, a, add, base, p.n);
+        store_tile<VEC>(p.out, a, add, (uint64_t)tile * kTile, p.n, kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) a[k] = b[k];
         tile = next;
     }
@@ -522,14 +484,10 @@ __global__ __launch_bounds__(BLOCK) void csdldf_u32(ScanParams p) {
 
             // Workgroup-wide redundant reduction of tile j (always a full tile:
             // only the last tile is partial and it is nobody's predecessor).
-            const uint32_t j = s_fb_tile;
+            const uint32_t j = __builtin_amdgcn_readfirstlane(s_fb_tile);
             {
                 u32x4 fd[VEC];
-                const uint64_t fbase = thread_base<BLOCK, VEC>(j);
-                if (p.vec_ok)
-                    load_vec<VEC>(fd, p.in + fbase);
-                else
-                    load_guarded<VEC>(fd, p.in, fbase, p.n);
+                load_tile<VEC>(fd, p.in, (uint64_t)j * C::kTile, p.n, C::kTile);
                 const uint32_t ws = wave_sum(thread_sum<VEC>(fd));
                 if (lane == 0) s_red[wave] = ws;
             }
@@ -678,8 +636,8 @@ csdldf_pp_u32(ScanParams p) {
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
     if (threadIdx.x == 0) atomic_add_counter(p.occupancy, 1ull);
 
@@ -689,13 +647,7 @@ csdldf_pp_u32(ScanParams p) {
     if (threadIdx.x < 4) s_count[threadIdx.x] = 0;
 
     u32x4 a[VEC], b[VEC];
-    {
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n))
-            load_vec<VEC>(a, p.in + base);
-        else
-            load_guarded<VEC>(a, p.in, base, p.n);
-    }
+    load_tile<VEC, (VEC < 8)>(a, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
 
     // Set when the current tile's aggregate was published while the previous
     // tile stalled (stall-time prepublication, below).
@@ -721,14 +673,10 @@ csdldf_pp_u32(ScanParams p) {
             // period 2 keeps the plain order.)
             if (threadIdx.x == 0) s_ticket[2] = take_ticket(p.ticket, total_tickets).tile;
             __syncthreads();
-            next = s_ticket[2];
+            next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
             has_next = next < p.num_tiles;
             if (has_next) {
-                const uint64_t next_base = thread_base<BLOCK, VEC>(next);
-                if (p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n))
-                    load_vec<VEC>(b, p.in + next_base);
-                else
-                    load_guarded<VEC>(b, p.in, next_base, p.n);
+                load_tile<VEC, (VEC < 8)>(b, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
                 prefetched = true;
             }
             const bool pre_next = has_next && !is_stalled_tile(p, next);
@@ -761,7 +709,7 @@ csdldf_pp_u32(ScanParams p) {
                 s_ticket[2] = take_ticket(p.ticket, total_tickets).tile;
             }
             __syncthreads();
-            next = s_ticket[2];
+            next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
             has_next = next < p.num_tiles;
             prepublished = false;
         }
@@ -778,11 +726,7 @@ csdldf_pp_u32(ScanParams p) {
             w = idx >= 0 ? v : make_status(0u, kFlagIncl, epoch);
         }
         if (has_next && !prefetched) {
-            const uint64_t next_base = thread_base<BLOCK, VEC>(next);
-            if (p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n))
-                load_vec<VEC>(b, p.in + next_base);
-            else
-                load_guarded<VEC>(b, p.in, next_base, p.n);
+            load_tile<VEC, (VEC < 8)>(b, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         }
 
         while (true) {
@@ -832,18 +776,17 @@ csdldf_pp_u32(ScanParams p) {
             // Workgroup-wide redundant reduction of tile j (a full tile: only
             // the last tile is partial and it is nobody's predecessor), FB
             // vectors per round so that it fits beside the two live tiles.
-            const uint32_t j = s_fb_tile;
+            const uint32_t j = __builtin_amdgcn_readfirstlane(s_fb_tile);
             {
                 constexpr int FB = VEC < 2 ? VEC : 2;
-                const uint64_t fbase = thread_base<BLOCK, VEC>(j);
+                const u32x4_any* v =
+                    reinterpret_cast<const u32x4_any*>(p.in + (uint64_t)j * C::kTile + thread_offset<VEC>());
                 uint32_t tsum = 0;
 #pragma unroll 1
                 for (int c = 0; c < VEC; c += FB) {
                     u32x4 fd[FB];
-                    if (p.vec_ok)
-                        load_vec<FB>(fd, p.in + fbase + (uint64_t)c * 256u);
-                    else
-                        load_guarded<FB>(fd, p.in, fbase + (uint64_t)c * 256u, p.n);
+#pragma unroll
+                    for (int k = 0; k < FB; ++k) fd[k] = __builtin_nontemporal_load(v + (c + k) * 64);
                     tsum += thread_sum<FB>(fd);
                 }
                 const uint32_t ws = wave_sum(tsum);
@@ -897,13 +840,8 @@ csdldf_pp_u32(ScanParams p) {
         }
 
         const uint32_t add = s_prefix + wave_prefix;
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n))
-            store_vec<VEC>(p.out + base, a, add);
-        else
-            store_guarded<VEC>(p.out, a, add, base, p.n);
+        store_tile<VEC>(p.out, a, add, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) a[k] = b[k];
         tile = next;
     }
@@ -921,17 +859,12 @@ csdldf_pp_u32(ScanParams p) {
 // (ReduceThenScan.cuh:36-37); here the last tile is reduced over [.., n).
 // ---------------------------------------------------------------------------
 template <int BLOCK, int VEC>
-__global__ __launch_bounds__(BLOCK) void rts_reduce_u32(const uint32_t* in, uint64_t n, uint32_t vec_ok,
-                                                        uint32_t* tile_sums) {
+__global__ __launch_bounds__(BLOCK) void rts_reduce_u32(const uint32_t* in, uint64_t n, uint32_t* tile_sums) {
     using C = TileCfg<BLOCK, VEC>;
     __shared__ uint32_t s_red[C::kWaves];
     const uint32_t tile = blockIdx.x;
-    const uint64_t base = thread_base<BLOCK, VEC>(tile);
     u32x4 d[VEC];
-    if (vec_ok && tile_is_full<BLOCK, VEC>(tile, n))
-        load_vec<VEC>(d, in + base);
-    else
-        load_guarded<VEC>(d, in, base, n);
+    load_tile<VEC>(d, in, (uint64_t)tile * C::kTile, n, C::kTile);
     const uint32_t ws = wave_sum(thread_sum<VEC>(d));
     if (lane_id() == 0) s_red[threadIdx.x / kWave] = ws;
     __syncthreads();
@@ -952,15 +885,14 @@ __global__ __launch_bounds__(kSpineBlock) void rts_spine_u32(uint32_t* tile_sums
     const uint32_t wave = threadIdx.x / kWave;
     uint32_t carry = 0;
     for (uint32_t round = 0; round * C::kTile < num_tiles; ++round) {
-        const uint64_t base = thread_base<kSpineBlock, 1>(round);
         u32x4 d[1];
-        load_guarded<1>(d, tile_sums, base, num_tiles);
+        load_tile<1>(d, tile_sums, (uint64_t)round * C::kTile, num_tiles, C::kTile);
         const uint32_t run = wave_scan_run<1, false>(d);
         if (lane_id() == 0) s_wave[wave] = run;
         __syncthreads();
         uint32_t wave_prefix, total;
         combine_waves<C::kWaves>(s_wave, wave, wave_prefix, total);
-        store_guarded<1>(tile_sums, d, carry + wave_prefix, base, num_tiles);
+        store_tile<1>(tile_sums, d, carry + wave_prefix, (uint64_t)round * C::kTile, num_tiles, C::kTile);
         carry += total;
         __syncthreads();
     }
@@ -968,28 +900,20 @@ __global__ __launch_bounds__(kSpineBlock) void rts_spine_u32(uint32_t* tile_sums
 
 template <int BLOCK, int VEC, bool INCL>
 __global__ __launch_bounds__(BLOCK) void rts_downsweep_u32(const uint32_t* in, uint32_t* out, uint64_t n,
-                                                           uint32_t vec_ok, const uint32_t* tile_prefix) {
+                                                           const uint32_t* tile_prefix) {
     using C = TileCfg<BLOCK, VEC>;
     __shared__ uint32_t s_wave[C::kWaves];
     const uint32_t tile = blockIdx.x;
     const uint32_t wave = threadIdx.x / kWave;
-    const uint64_t base = thread_base<BLOCK, VEC>(tile);
-    const bool vec_path = vec_ok && tile_is_full<BLOCK, VEC>(tile, n);
     u32x4 d[VEC];
-    if (vec_path)
-        load_vec<VEC>(d, in + base);
-    else
-        load_guarded<VEC>(d, in, base, n);
+    load_tile<VEC>(d, in, (uint64_t)tile * C::kTile, n, C::kTile);
     const uint32_t run = wave_scan_run<VEC, INCL>(d);
     if (lane_id() == 0) s_wave[wave] = run;
     __syncthreads();
     uint32_t wave_prefix, total;
     combine_waves<C::kWaves>(s_wave, wave, wave_prefix, total);
     const uint32_t add = tile_prefix[tile] + wave_prefix;
-    if (vec_path)
-        store_vec<VEC>(out + base, d, add);
-    else
-        store_guarded<VEC>(out, d, add, base, n);
+    store_tile<VEC>(out, d, add, (uint64_t)tile * C::kTile, n, C::kTile);
 }
 
 // ---------------------------------------------------------------------------
@@ -1069,26 +993,19 @@ __global__ void validate_diff_kernel(const uint32_t* in, const uint32_t* scan, u
 // nontemporal): the practical read-n + write-n ceiling the scan is held to,
 // and the calibration kernel for HBM byte counters.
 template <int BLOCK, int VEC>
-__global__ __launch_bounds__(BLOCK) void copy_u32_kernel(const uint32_t* in, uint32_t* out, uint64_t n,
-                                                         uint32_t vec_ok) {
-    const uint32_t tile = blockIdx.x;
-    const uint64_t base = thread_base<BLOCK, VEC>(tile);
+__global__ __launch_bounds__(BLOCK) void copy_u32_kernel(const uint32_t* in, uint32_t* out, uint64_t n) {
+    constexpr uint32_t kTile = TileCfg<BLOCK, VEC>::kTile;
+    const uint64_t start = (uint64_t)blockIdx.x * kTile;
     u32x4 d[VEC];
-    if (vec_ok && tile_is_full<BLOCK, VEC>(tile, n)) {
-        load_vec<VEC>(d, in + base);
-        store_vec<VEC>(out + base, d, 0u);
-    } else {
-        load_guarded<VEC>(d, in, base, n);
-        store_guarded<VEC>(out, d, 0u, base, n);
-    }
+    load_tile<VEC>(d, in, start, n, kTile);
+    store_tile<VEC>(out, d, 0u, start, n, kTile);
 }
 
 hipError_t launch_copy_u32(const uint32_t* in, uint32_t* out, uint64_t n, hipStream_t stream) {
     if (!n) return hipSuccess;
     constexpr uint32_t kTile = TileCfg<256, 4>::kTile;
-    const uint32_t vec_ok = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
     hipLaunchKernelGGL((copy_u32_kernel<256, 4>), dim3((uint32_t)((n + kTile - 1) / kTile)), dim3(256), 0, stream,
-                       in, out, n, vec_ok);
+                       in, out, n);
     return hipGetLastError();
 }
 
@@ -1257,18 +1174,18 @@ hipError_t launch_csdldf_pp_u32(TileShape s, bool inclusive, const ScanParams& p
 }
 
 hipError_t launch_rts_u32(TileShape s, bool inclusive, const uint32_t* in, uint32_t* out, uint64_t n,
-                          uint32_t num_tiles, uint32_t vec_ok, uint32_t* tile_sums, hipStream_t stream) {
+                          uint32_t num_tiles, uint32_t* tile_sums, hipStream_t stream) {
 #define X(B, V)                                                                                           \
     if (s.block == B && s.vec == V) {                                                                     \
-        hipLaunchKernelGGL((rts_reduce_u32<B, V>), dim3(num_tiles), dim3(B), 0, stream, in, n, vec_ok,    \
+        hipLaunchKernelGGL((rts_reduce_u32<B, V>), dim3(num_tiles), dim3(B), 0, stream, in, n,    \
                            tile_sums);                                                                    \
         hipLaunchKernelGGL(rts_spine_u32, dim3(1), dim3(kSpineBlock), 0, stream, tile_sums, num_tiles);  \
         if (inclusive)                                                                                    \
             hipLaunchKernelGGL((rts_downsweep_u32<B, V, true>), dim3(num_tiles), dim3(B), 0, stream, in,  \
-                               out, n, vec_ok, (const uint32_t*)tile_sums);                               \
+                               out, n, (const uint32_t*)tile_sums);                               \
         else                                                                                              \
             hipLaunchKernelGGL((rts_downsweep_u32<B, V, false>), dim3(num_tiles), dim3(B), 0, stream, in, \
-                               out, n, vec_ok, (const uint32_t*)tile_sums);                               \
+                               out, n, (const uint32_t*)tile_sums);                               \
         return hipGetLastError();                                                                         \
     }
     GPS_SHAPES(X)

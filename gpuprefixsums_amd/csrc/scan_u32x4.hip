@@ -105,45 +105,17 @@ struct LookbackV4 {
     }
 };
 
-// Tile I/O: element (wave, k, lane) of tile t is struct
-// t * BLOCK * VEC + wave * 64 * VEC + k * 64 + lane.
+// Tile I/O: a tile of BLOCK * VEC structs is one of 4 * BLOCK * VEC uint32 in
+// the plain scan's layout, struct (wave, k, lane) its uint4 (wave, k, lane).
 template <int BLOCK, int VEC>
-__device__ __forceinline__ uint64_t v4_base(uint32_t tile, uint32_t wave, uint32_t lane) {
-    return (uint64_t)tile * ((uint64_t)BLOCK * VEC) + (uint64_t)wave * (64u * VEC) + lane;
+__device__ __forceinline__ void load_v4(u32x4 (&d)[VEC], const V4Params& p, uint32_t tile) {
+    constexpr uint32_t kElems = 4u * BLOCK * VEC;
+    load_tile<VEC>(d, p.in, (uint64_t)tile * kElems, 4u * p.n, kElems);
 }
-
 template <int BLOCK, int VEC>
-__device__ __forceinline__ void load_v4(u32x4 (&d)[VEC], const V4Params& p, uint32_t tile, uint32_t wave,
-                                        uint32_t lane) {
-    const uint64_t base = v4_base<BLOCK, VEC>(tile, wave, lane);
-    const u32x4* in4 = reinterpret_cast<const u32x4*>(p.in);
-    if ((uint64_t)(tile + 1u) * ((uint64_t)BLOCK * VEC) <= p.n) {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) d[k] = __builtin_nontemporal_load(in4 + base + (uint64_t)k * 64u);
-    } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            const uint64_t i = base + (uint64_t)k * 64u;
-            d[k] = i < p.n ? in4[i] : (u32x4){0u, 0u, 0u, 0u};
-        }
-    }
-}
-
-template <int BLOCK, int VEC>
-__device__ __forceinline__ void store_v4(const V4Params& p, const u32x4 (&d)[VEC], u32x4 add, uint32_t tile,
-                                         uint32_t wave, uint32_t lane) {
-    const uint64_t base = v4_base<BLOCK, VEC>(tile, wave, lane);
-    u32x4* out4 = reinterpret_cast<u32x4*>(p.out);
-    if ((uint64_t)(tile + 1u) * ((uint64_t)BLOCK * VEC) <= p.n) {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) __builtin_nontemporal_store(d[k] + add, out4 + base + (uint64_t)k * 64u);
-    } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            const uint64_t i = base + (uint64_t)k * 64u;
-            if (i < p.n) out4[i] = d[k] + add;
-        }
-    }
+__device__ __forceinline__ void store_v4(const V4Params& p, const u32x4 (&d)[VEC], u32x4 add, uint32_t tile) {
+    constexpr uint32_t kElems = 4u * BLOCK * VEC;
+    store_tile<VEC>(p.out, d, add, (uint64_t)tile * kElems, 4u * p.n, kElems);
 }
 
 // Scans the tile in registers: per vector and member, a DPP scan across the
@@ -197,9 +169,10 @@ __global__ __launch_bounds__(BLOCK) void csdl_u32x4(V4Params p) {
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    const uint32_t tile = s_ticket[0], epoch = s_ticket[1];
+    const uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]),
+                   epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     u32x4 d[VEC];
-    load_v4<BLOCK, VEC>(d, p, tile, wave, lane);
+    load_v4<BLOCK, VEC>(d, p, tile);
     u32x4 wave_prefix, tile_total;
     scan_v4<BLOCK, VEC, INCL>(d, s_wave, wave, lane, wave_prefix, tile_total);
 
@@ -220,8 +193,7 @@ __global__ __launch_bounds__(BLOCK) void csdl_u32x4(V4Params p) {
         }
     }
     __syncthreads();
-    store_v4<BLOCK, VEC>(p, d, (u32x4){s_prefix[0], s_prefix[1], s_prefix[2], s_prefix[3]} + wave_prefix, tile,
-                         wave, lane);
+    store_v4<BLOCK, VEC>(p, d, (u32x4){s_prefix[0], s_prefix[1], s_prefix[2], s_prefix[3]} + wave_prefix, tile);
 }
 
 // Persistent, software-pipelined form (the schedule of the plain CSDL scan's
@@ -248,13 +220,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
     if (threadIdx.x == 0) atomic_add_counter(p.occupancy, 1ull);
 
     u32x4 a[VEC], b[VEC];
-    load_v4<BLOCK, VEC>(a, p, tile, wave, lane);
+    load_v4<BLOCK, VEC>(a, p, tile);
     while (true) {
         u32x4 wave_prefix, tile_total;
         scan_v4<BLOCK, VEC, INCL>(a, s_wave, wave, lane, wave_prefix, tile_total);
@@ -263,7 +235,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             s_ticket[2] = take_ticket(p.ticket, total_tickets).tile;
         }
         __syncthreads();
-        const uint32_t next = s_ticket[2];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
         const bool has_next = next < p.num_tiles;
 
         LookbackV4 lb;
@@ -271,7 +243,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             lb.start(tile);
             lb.issue(p.status, epoch);
         }
-        if (has_next) load_v4<BLOCK, VEC>(b, p, next, wave, lane);
+        if (has_next) load_v4<BLOCK, VEC>(b, p, next);
         if (wave == 0) {
             u32x4 prefix = {0u, 0u, 0u, 0u};
             if (tile != 0) {
@@ -284,8 +256,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             }
         }
         __syncthreads();
-        store_v4<BLOCK, VEC>(p, a, (u32x4){s_prefix[0], s_prefix[1], s_prefix[2], s_prefix[3]} + wave_prefix,
-                             tile, wave, lane);
+        store_v4<BLOCK, VEC>(p, a, (u32x4){s_prefix[0], s_prefix[1], s_prefix[2], s_prefix[3]} + wave_prefix, tile);
         if (!has_next) break;
         for (int k = 0; k < VEC; ++k) a[k] = b[k];  // the prefetched tile becomes the current one
         tile = next;

@@ -31,7 +31,6 @@ struct SegParams {
     uint64_t num_segments;
     uint64_t n;
     uint32_t num_tiles;
-    uint32_t vec_ok;
     uint64_t* status;
     uint64_t* ticket;
     uint32_t* err;
@@ -133,18 +132,13 @@ __global__ __launch_bounds__(BLOCK) void segscan_u32(SegParams p) {
     }
     for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[i] = 0u;
     __syncthreads();
-    const uint32_t tile = s_ticket[0], epoch = s_ticket[1];
+    const uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]), epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     const uint64_t a = (uint64_t)tile * C::kTile;
     const uint64_t b = a + C::kTile < p.n ? a + C::kTile : p.n;
 
     // Data loads first; the head search overlaps their latency.
-    const uint64_t base = thread_base<BLOCK, VEC>(tile);
     u32x4 d[VEC];
-    const bool vec_path = p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n);
-    if (vec_path)
-        load_vec<VEC>(d, p.in + base);
-    else
-        load_guarded<VEC>(d, p.in, base, p.n);
+    load_tile<VEC>(d, p.in, a, p.n, C::kTile);
 
     if (wave == 0) {
         const uint64_t s0 = find_first_segment(p.offsets, p.num_segments, a);
@@ -183,10 +177,7 @@ __global__ __launch_bounds__(BLOCK) void segscan_u32(SegParams p) {
     }
     __syncthreads();
     seg_add_carry<VEC>(d, first_head, pre_f ? pre_v : s_prefix + pre_v);
-    if (vec_path)
-        store_vec<VEC>(p.out + base, d, 0u);
-    else
-        store_guarded<VEC>(p.out, d, 0u, base, p.n);
+    store_tile<VEC>(p.out, d, 0u, a, p.n, C::kTile);
 }
 
 // ---------------------------------------------------------------------------
@@ -223,18 +214,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     }
     for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[0][i] = 0u;
     __syncthreads();
-    uint32_t tile = s_ticket[0];
-    const uint32_t epoch = s_ticket[1];
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     if (tile >= p.num_tiles) return;
 
     u32x4 a[VEC], b[VEC];
-    {
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n))
-            load_vec<VEC>(a, p.in + base);
-        else
-            load_guarded<VEC>(a, p.in, base, p.n);
-    }
+    load_tile<VEC>(a, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
     {
         const uint64_t lo = (uint64_t)tile * C::kTile;
         const uint64_t hi = lo + C::kTile < p.n ? lo + C::kTile : p.n;
@@ -268,7 +253,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         // the other head buffer was last read by the previous tile's scan
         for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[cur ^ 1u][i] = 0u;
         __syncthreads();
-        const uint32_t next = s_ticket[2];
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_ticket[2]);
         const bool has_next = next < p.num_tiles;
 
         Lookback lb;
@@ -283,11 +268,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             mark_heads_by(s_heads[cur ^ 1u], p.offsets, p.num_segments, s0, lo, hi, next == 0, lane, kWave);
         }
         if (has_next) {
-            const uint64_t next_base = thread_base<BLOCK, VEC>(next);
-            if (p.vec_ok && tile_is_full<BLOCK, VEC>(next, p.n))
-                load_vec<VEC>(b, p.in + next_base);
-            else
-                load_guarded<VEC>(b, p.in, next_base, p.n);
+            load_tile<VEC>(b, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         }
         if (wave == 0) {
             uint32_t prefix = 0;
@@ -300,13 +281,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         }
         __syncthreads();  // also completes the next tile's head bitmap
         seg_add_carry<VEC>(a, first_head, pre_f ? pre_v : s_prefix + pre_v);
-        const uint64_t base = thread_base<BLOCK, VEC>(tile);
-        if (p.vec_ok && tile_is_full<BLOCK, VEC>(tile, p.n))
-            store_vec<VEC>(p.out + base, a, 0u);
-        else
-            store_guarded<VEC>(p.out, a, 0u, base, p.n);
+        store_tile<VEC>(p.out, a, 0u, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
-#pragma unroll
         for (int k = 0; k < VEC; ++k) a[k] = b[k];
         tile = next;
         cur ^= 1u;
@@ -384,7 +360,7 @@ hipError_t prepare_segscan_u32(TileShape s, bool inclusive, bool persistent) {
 }
 
 hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, const uint32_t* in, uint32_t* out,
-                              const uint64_t* offsets, uint64_t num_segments, uint64_t n, uint32_t vec_ok,
+                              const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                               uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream) {
     SegParams p{};
     p.in = in;
@@ -393,7 +369,6 @@ hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, cons
     p.num_segments = num_segments;
     p.n = n;
     p.num_tiles = (uint32_t)((n + s.tile() - 1) / s.tile());
-    p.vec_ok = vec_ok;
     p.status = status;
     p.ticket = ticket;
     p.err = err;

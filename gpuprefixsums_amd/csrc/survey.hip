@@ -197,20 +197,13 @@ __global__ __launch_bounds__(kBlock) void survey_kernel(const uint32_t* in, uint
         using C = TileCfg<kBlock, 4>;
         __shared__ uint32_t s_wave[C::kWaves];
         u32x4 d[4];
-        const uint64_t base = thread_base<kBlock, 4>(blockIdx.x);
-        if (wg_base + C::kTile <= n)
-            load_vec<4>(d, in + base);
-        else
-            load_guarded<4>(d, in, base, n);
+        load_tile<4>(d, in, wg_base, n, C::kTile);
         const uint32_t run = wave_scan_run<4, INCL>(d);
         if (lane == 0) s_wave[wave_index()] = run;
         __syncthreads();
         uint32_t wave_prefix, total;
         combine_waves<C::kWaves>(s_wave, wave_index(), wave_prefix, total);
-        if (wg_base + C::kTile <= n)
-            store_vec<4>(out + base, d, wave_prefix);
-        else
-            store_guarded<4>(out, d, wave_prefix, base, n);
+        store_tile<4>(out, d, wave_prefix, wg_base, n, C::kTile);
     } else {
         const uint64_t i = wg_base + tid;
         const uint32_t x = load_or_zero(in, i, n);

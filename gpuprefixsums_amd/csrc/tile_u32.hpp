@@ -26,52 +26,88 @@ struct TileCfg {
     static constexpr uint32_t kWaveElems = 64 * kItems;
 };
 
-// Element offset of this thread's first vector inside the buffer.
-template <int BLOCK, int VEC>
-__device__ __forceinline__ uint64_t thread_base(uint32_t tile) {
-    using C = TileCfg<BLOCK, VEC>;
-    return (uint64_t)tile * C::kTile + (threadIdx.x / kWave) * C::kWaveElems + lane_id() * 4u;
+// Element offset of this thread's first vector inside its tile.
+template <int VEC>
+__device__ __forceinline__ uint32_t thread_offset() {
+    return (threadIdx.x / kWave) * (256u * VEC) + lane_id() * 4u;
 }
 
-// Full tile, 16-byte aligned: one dwordx4 per vector, nontemporal (streamed once).
-template <int VEC>
-__device__ __forceinline__ void load_vec(u32x4 (&d)[VEC], const uint32_t* p) {
-    const u32x4* v = reinterpret_cast<const u32x4*>(p);
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) d[k] = __builtin_nontemporal_load(v + k * 64);
+// Tile input and output. Buffers are only element-aligned (a slice x[1:] is an
+// ordinary input) and n is any number, so:
+//   - vectors are moved as dwordx4 from any 4-byte address, which gfx950 does
+//     at full rate (a wave's 1 KiB then spans nine 128-byte lines, not eight);
+//   - a partial tile is a raw buffer that ends at n: its loads return zero and
+//     its stores do nothing for each dword past the end. Stores go through the
+//     buffer always, so they need no second path; full tiles load through
+//     plain addresses (buffer loads took 341.5 us for the 2^28 scan, plain
+//     ones 340.0).
+// Four guarded 4-byte accesses per vector, each a quarter of a line's bytes,
+// took twice as long where a whole scan ran on them, and one partial tile of
+// them at the end held up aligned scans too: 12,345,677 elements one element
+// into a buffer 45.7 -> 21.0 us, the same aligned 26.3 -> 20.3 us; 2^28
+// elements off by one 653 -> 343 us.
+typedef u32x4 u32x4_any __attribute__((aligned(4)));
+
+// base and bytes are the same in every lane (the resource is scalar).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* base, uint32_t bytes) {
+    const uint64_t p = reinterpret_cast<uint64_t>(base);
+    // The builtin returns int: the casts keep a low word of 2^31 or more from
+    // extending its sign over the high one.
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)p);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
+    const uint64_t u = (uint64_t)hi << 32 | lo;
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(u), 0, __builtin_amdgcn_readfirstlane(bytes),
+                                             0x00020000);
+}
+constexpr int kNontemporal = 2;  // buffer cache policy: nt
+
+// Valid elements of the tile that starts at `start` (uniform).
+__device__ __forceinline__ uint32_t tile_valid(uint64_t start, uint64_t n, uint32_t tile_elems) {
+    const uint64_t left = n - start;
+    return left < tile_elems ? (uint32_t)left : tile_elems;
 }
 
-// Partial tile or unaligned buffer: element-wise, zero beyond n.
-template <int VEC>
-__device__ __forceinline__ void load_guarded(u32x4 (&d)[VEC], const uint32_t* in, uint64_t base, uint64_t n) {
+// Inputs up to a quarter of the 256 MiB Infinity Cache are loaded with the
+// ordinary policy, so that what is there is used and stays; larger ones stream
+// past it. Nontemporal / ordinary loads, one input again and again: 2^20
+// elements 6.1 / 5.3 us, 2^24 25.2 / 22.7, 2^25 48.4 / 40.5, 2^28 340 / 348;
+// three inputs in turn: 2^24 25.4 / 22.8, 2^25 48.8 / 48.7, 2^26 89.8 / 91.0.
+// So from 2^25 on it pays only for a caller that scans the same large input
+// again, and costs 1-5% otherwise. (Ordinary stores are slower at every size:
+// the output pushes the input out.)
+constexpr uint64_t kCachedBytes = 64ull << 20;
+
+// LEAN: no address registers for the streaming path (buffer loads there too).
+template <int VEC, bool LEAN = false>
+__device__ __forceinline__ void load_tile(u32x4 (&d)[VEC], const uint32_t* in, uint64_t start, uint64_t n,
+                                          uint32_t tile_elems) {
+    const uint32_t valid = tile_valid(start, n, tile_elems), at = thread_offset<VEC>();
+    const bool stream = 4u * n > kCachedBytes;
+    if (LEAN && stream) {
+        const __amdgpu_buffer_rsrc_t r = raw_buffer(in + start, 4u * valid);
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) {
+        for (int k = 0; k < VEC; ++k)
+            d[k] = __builtin_amdgcn_raw_buffer_load_b128(r, 4u * at + k * 1024u, 0, kNontemporal);
+    } else if (stream && valid == tile_elems) {
+        const u32x4_any* v = reinterpret_cast<const u32x4_any*>(in + start + at);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-            d[k][c] = i < n ? in[i] : 0u;
-        }
+        for (int k = 0; k < VEC; ++k) d[k] = __builtin_nontemporal_load(v + k * 64);
+    } else {
+        const __amdgpu_buffer_rsrc_t r = raw_buffer(in + start, 4u * valid);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) d[k] = __builtin_amdgcn_raw_buffer_load_b128(r, 4u * at + k * 1024u, 0, 0);
     }
 }
 
-template <int VEC>
-__device__ __forceinline__ void store_vec(uint32_t* p, const u32x4 (&d)[VEC], uint32_t add) {
-    u32x4* v = reinterpret_cast<u32x4*>(p);
+// `add`: a uint32, or a u32x4 for the struct scan.
+template <int VEC, class Add>
+__device__ __forceinline__ void store_tile(uint32_t* out, const u32x4 (&d)[VEC], Add add, uint64_t start, uint64_t n,
+                                           uint32_t tile_elems) {
+    const uint32_t valid = tile_valid(start, n, tile_elems), at = 4u * thread_offset<VEC>();
+    const __amdgpu_buffer_rsrc_t r = raw_buffer(out + start, 4u * valid);
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) __builtin_nontemporal_store(d[k] + add, v + k * 64);
-}
-
-template <int VEC>
-__device__ __forceinline__ void store_guarded(uint32_t* out, const u32x4 (&d)[VEC], uint32_t add, uint64_t base,
-                                              uint64_t n) {
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint64_t i = base + (uint64_t)k * 256u + (uint64_t)c;
-            if (i < n) out[i] = d[k][c] + add;
-        }
-    }
+    for (int k = 0; k < VEC; ++k)
+        __builtin_amdgcn_raw_buffer_store_b128(d[k] + add, r, at + k * 1024u, 0, kNontemporal);
 }
 
 // Scans the wave's run in registers. On return d holds, per element, the
@@ -107,12 +143,6 @@ __device__ __forceinline__ uint32_t thread_sum(const u32x4 (&d)[VEC]) {
 #pragma unroll
     for (int k = 0; k < VEC; ++k) s += d[k].x + d[k].y + d[k].z + d[k].w;
     return s;
-}
-
-// True when the whole tile lies inside [0, n).
-template <int BLOCK, int VEC>
-__device__ __forceinline__ bool tile_is_full(uint32_t tile, uint64_t n) {
-    return (uint64_t)(tile + 1u) * TileCfg<BLOCK, VEC>::kTile <= n;
 }
 
 // Exclusive prefix of this wave inside the tile, and the tile total, from the
