@@ -114,7 +114,7 @@ inline void size_adaptive_config(uint64_t n, TileShape& shape, uint32_t& schedul
     }
 }
 
-// Each launcher enqueues exactly one kernel (RTS: three) on `stream` and
+// Each launcher enqueues exactly one kernel (RTS: two or three) on `stream` and
 // returns the HIP launch status.
 hipError_t launch_csdl_u32(TileShape s, bool inclusive, const ScanParams& p, hipStream_t stream);
 // Persistent pipelined CSDL: grid = resident workgroups (<= num_tiles).

@@ -852,19 +852,40 @@ csdldf_pp_u32(ScanParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Reduce-then-scan. Three launches: per-tile sums, an exclusive scan of the
-// sums by one workgroup, and a rescan of every tile with its carry-in. Reads
-// the input twice (12 B/elem of traffic against 8 B algorithmic).
+// Reduce-then-scan: per-tile sums, then a rescan of every tile with its
+// carry-in. Reads the input twice (12 B/elem of traffic against 8 B
+// algorithmic), which is what bounds it: 7.1 TB/s over those 12 B at 2^26. Up
+// to kRtsDirect tiles the rescan adds up the sums before its tile by itself (a
+// load per thread and 512 tiles, from L2, beside the tile's own loads);
+// beyond, one workgroup scans them in between. The reduce loads with the
+// ordinary cache policy, so that the rescan finds part of the input in the
+// Infinity Cache, and the rescan streams past it. Against a spine of 4096
+// sums per round at every size and nontemporal loads (three inputs in turn):
+// 2^20 6.6 -> 5.0 us, 2^22 11.4 -> 8.6, 2^24 36.5 -> 28.5, 2^26 131 -> 118,
+// 2^28 522 -> 489; with a spine from 1025 tiles on, 2^24 31.1, 2^25 59.4
+// against 58.0. (Sums per group of tiles instead of the spine, from atomics
+// or the group's last workgroup, cost the reduce 8-14 us at 2^26.)
 // The reference's partial-tile reduce predicate is inverted
 // (ReduceThenScan.cuh:36-37); here the last tile is reduced over [.., n).
 // ---------------------------------------------------------------------------
+constexpr uint32_t kRtsDirect = 16384;
+
+template <int VEC, int POLICY>
+__device__ __forceinline__ void load_tile_policy(u32x4 (&d)[VEC], const uint32_t* in, uint64_t start, uint64_t n,
+                                                 uint32_t tile_elems) {
+    const __amdgpu_buffer_rsrc_t r = raw_buffer(in + start, 4u * tile_valid(start, n, tile_elems));
+    const uint32_t at = 4u * thread_offset<VEC>();
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) d[k] = __builtin_amdgcn_raw_buffer_load_b128(r, at + k * 1024u, 0, POLICY);
+}
+
 template <int BLOCK, int VEC>
 __global__ __launch_bounds__(BLOCK) void rts_reduce_u32(const uint32_t* in, uint64_t n, uint32_t* tile_sums) {
     using C = TileCfg<BLOCK, VEC>;
     __shared__ uint32_t s_red[C::kWaves];
     const uint32_t tile = blockIdx.x;
     u32x4 d[VEC];
-    load_tile<VEC>(d, in, (uint64_t)tile * C::kTile, n, C::kTile);
+    load_tile_policy<VEC, 0>(d, in, (uint64_t)tile * C::kTile, n, C::kTile);
     const uint32_t ws = wave_sum(thread_sum<VEC>(d));
     if (lane_id() == 0) s_red[threadIdx.x / kWave] = ws;
     __syncthreads();
@@ -876,44 +897,59 @@ __global__ __launch_bounds__(BLOCK) void rts_reduce_u32(const uint32_t* in, uint
     }
 }
 
-// One workgroup of 1024 threads; exclusive scan of tile_sums in place, 4096
-// values per round with a uniform carry between rounds.
+// One workgroup of 1024 threads; exclusive scan of tile_sums in place, 32768
+// values per round with a uniform carry between rounds; the next round's
+// loads are in flight during this one's scan.
 constexpr int kSpineBlock = 1024;
+constexpr int kSpineVec = 8;
 __global__ __launch_bounds__(kSpineBlock) void rts_spine_u32(uint32_t* tile_sums, uint32_t num_tiles) {
-    using C = TileCfg<kSpineBlock, 1>;
+    using C = TileCfg<kSpineBlock, kSpineVec>;
     __shared__ uint32_t s_wave[C::kWaves];
-    const uint32_t wave = threadIdx.x / kWave;
+    const uint32_t wave = wave_index();
     uint32_t carry = 0;
-    for (uint32_t round = 0; round * C::kTile < num_tiles; ++round) {
-        u32x4 d[1];
-        load_tile<1>(d, tile_sums, (uint64_t)round * C::kTile, num_tiles, C::kTile);
-        const uint32_t run = wave_scan_run<1, false>(d);
+    u32x4 d[kSpineVec], next[kSpineVec];
+    load_tile_policy<kSpineVec, 0>(d, tile_sums, 0, num_tiles, C::kTile);
+    for (uint64_t start = 0; start < num_tiles; start += C::kTile) {
+        if (start + C::kTile < num_tiles)
+            load_tile_policy<kSpineVec, 0>(next, tile_sums, start + C::kTile, num_tiles, C::kTile);
+        const uint32_t run = wave_scan_run<kSpineVec, false>(d);
         if (lane_id() == 0) s_wave[wave] = run;
         __syncthreads();
         uint32_t wave_prefix, total;
         combine_waves<C::kWaves>(s_wave, wave, wave_prefix, total);
-        store_tile<1>(tile_sums, d, carry + wave_prefix, (uint64_t)round * C::kTile, num_tiles, C::kTile);
+        store_tile<kSpineVec>(tile_sums, d, carry + wave_prefix, start, num_tiles, C::kTile);
         carry += total;
+        for (int k = 0; k < kSpineVec; ++k) d[k] = next[k];
         __syncthreads();
     }
 }
 
-template <int BLOCK, int VEC, bool INCL>
+// DIRECT: tile_sums holds sums, not their scan.
+template <int BLOCK, int VEC, bool INCL, bool DIRECT>
 __global__ __launch_bounds__(BLOCK) void rts_downsweep_u32(const uint32_t* in, uint32_t* out, uint64_t n,
-                                                           const uint32_t* tile_prefix) {
+                                                           const uint32_t* tile_sums) {
     using C = TileCfg<BLOCK, VEC>;
-    __shared__ uint32_t s_wave[C::kWaves];
+    __shared__ uint32_t s_wave[C::kWaves], s_before[C::kWaves];
     const uint32_t tile = blockIdx.x;
-    const uint32_t wave = threadIdx.x / kWave;
+    const uint32_t wave = wave_index();
+    uint32_t before = 0;
+    if (DIRECT)
+        for (uint32_t j = threadIdx.x; j < tile; j += BLOCK) before += tile_sums[j];
+    else
+        before = tile_sums[tile];
     u32x4 d[VEC];
-    load_tile<VEC>(d, in, (uint64_t)tile * C::kTile, n, C::kTile);
+    load_tile_policy<VEC, kNontemporal>(d, in, (uint64_t)tile * C::kTile, n, C::kTile);
     const uint32_t run = wave_scan_run<VEC, INCL>(d);
     if (lane_id() == 0) s_wave[wave] = run;
+    if (DIRECT) {
+        const uint32_t sum = wave_sum(before);
+        if (lane_id() == 0) s_before[wave] = sum;
+    }
     __syncthreads();
     uint32_t wave_prefix, total;
+    if (DIRECT) combine_waves<C::kWaves>(s_before, wave, wave_prefix, before);
     combine_waves<C::kWaves>(s_wave, wave, wave_prefix, total);
-    const uint32_t add = tile_prefix[tile] + wave_prefix;
-    store_tile<VEC>(out, d, add, (uint64_t)tile * C::kTile, n, C::kTile);
+    store_tile<VEC>(out, d, before + wave_prefix, (uint64_t)tile * C::kTile, n, C::kTile);
 }
 
 // ---------------------------------------------------------------------------
@@ -1173,21 +1209,27 @@ hipError_t launch_csdldf_pp_u32(TileShape s, bool inclusive, const ScanParams& p
     return hipErrorInvalidValue;
 }
 
+template <int B, int V, bool I>
+static hipError_t launch_rts(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t num_tiles, uint32_t* tile_sums,
+                             hipStream_t stream) {
+    hipLaunchKernelGGL((rts_reduce_u32<B, V>), dim3(num_tiles), dim3(B), 0, stream, in, n, tile_sums);
+    if (num_tiles <= kRtsDirect) {
+        hipLaunchKernelGGL((rts_downsweep_u32<B, V, I, true>), dim3(num_tiles), dim3(B), 0, stream, in, out, n,
+                           (const uint32_t*)tile_sums);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(rts_spine_u32, dim3(1), dim3(kSpineBlock), 0, stream, tile_sums, num_tiles);
+    hipLaunchKernelGGL((rts_downsweep_u32<B, V, I, false>), dim3(num_tiles), dim3(B), 0, stream, in, out, n,
+                       (const uint32_t*)tile_sums);
+    return hipGetLastError();
+}
+
 hipError_t launch_rts_u32(TileShape s, bool inclusive, const uint32_t* in, uint32_t* out, uint64_t n,
                           uint32_t num_tiles, uint32_t* tile_sums, hipStream_t stream) {
-#define X(B, V)                                                                                           \
-    if (s.block == B && s.vec == V) {                                                                     \
-        hipLaunchKernelGGL((rts_reduce_u32<B, V>), dim3(num_tiles), dim3(B), 0, stream, in, n,    \
-                           tile_sums);                                                                    \
-        hipLaunchKernelGGL(rts_spine_u32, dim3(1), dim3(kSpineBlock), 0, stream, tile_sums, num_tiles);  \
-        if (inclusive)                                                                                    \
-            hipLaunchKernelGGL((rts_downsweep_u32<B, V, true>), dim3(num_tiles), dim3(B), 0, stream, in,  \
-                               out, n, (const uint32_t*)tile_sums);                               \
-        else                                                                                              \
-            hipLaunchKernelGGL((rts_downsweep_u32<B, V, false>), dim3(num_tiles), dim3(B), 0, stream, in, \
-                               out, n, (const uint32_t*)tile_sums);                               \
-        return hipGetLastError();                                                                         \
-    }
+#define X(B, V)                                                                             \
+    if (s.block == B && s.vec == V)                                                         \
+        return inclusive ? launch_rts<B, V, true>(in, out, n, num_tiles, tile_sums, stream) \
+                         : launch_rts<B, V, false>(in, out, n, num_tiles, tile_sums, stream);
     GPS_SHAPES(X)
 #undef X
     return hipErrorInvalidValue;

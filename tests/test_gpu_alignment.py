@@ -113,3 +113,21 @@ def test_segmented_u32_at_every_offset(schedule, inclusive):
                     assert np.array_equal(got, want), (n, shift_in, shift_out, first_mismatch(got, want))
                     check_guards(buf, n, shift_out)
         assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("inclusive", [False, True], ids=["excl", "incl"])
+@pytest.mark.parametrize("block,vec", [(256, 2), (512, 2), (1024, 8)])
+def test_rts_with_and_without_the_spine(block, vec, inclusive):
+    """Tile counts around the last one whose rescan adds up the tile sums by
+    itself (16384), and around the spine's rounds of 32768 sums."""
+    tile = block * vec * 4
+    counts = [1, 2, 511, 513, 16384, 16385] + ([32768, 32769] if tile <= 4096 else [])
+    n_max = max(counts) * tile
+    x = torch.empty(n_max + 1, dtype=torch.int32, device="cuda")
+    gps.fill_random_u32(x, n_max + 1, seed=9)
+    out = torch.empty(n_max, dtype=torch.int32, device="cuda")
+    with gps.ScanHandle(gps.ALGO_RTS, n_max, block_threads=block, vec_per_thread=vec) as h:
+        for c in counts:
+            for n in (c * tile - 3, c * tile):
+                h.scan(x[1:], out, n, inclusive)
+                assert gps.validate_scan_u32(x[1:], out, n, inclusive) == 0, (c, n)
