@@ -143,7 +143,7 @@ int scan_u32(gps_handle* h, const uint32_t* in, uint32_t* out, uint64_t n, bool 
     p.status = h->status;
     p.ticket = h->ticket;
     p.err = h->err;
-    p.spin_limit = h->spin_limit;
+    p.spin_limit = h->algo == GPS_ALGO_CSDL ? h->round_patience : h->spin_limit;
     p.stall_period = h->stall_period;
     p.counters = h->counters;
     p.carry_in = carry_in;
@@ -221,6 +221,7 @@ int gps_create(int algo, uint64_t max_n, const gps_tuning* tuning, gps_handle** 
     h->max_n = max_n;
     h->shape = shape;
     h->spin_limit = spin_limit;
+    if (tuning && tuning->spin_limit) h->round_patience = tuning->spin_limit;
     h->stall_period = stall_period;
     h->schedule = schedule;
     h->size_adaptive = size_adaptive;

@@ -30,14 +30,20 @@ gps::TileShape seg_shape(const gps_handle* h, uint64_t n) {
 
 // FP kernels likewise: the handle's shape when it is an FP shape, else
 // 1024 x 4. A default handle picks from n (sweep timings and back-to-back
-// launches on MI355X): one FP scan uses 256 x 4 up to 2^18 elements (2^16:
-// 4.8 against 9.0 us for 1024 x 4 ... 1024 x 8), 1024 x 4 up to 2^22 and
-// 1024 x 8 above; the segmented FP kernel uses 256 x 4 below 2^20 and
-// 1024 x 4 above (1.00 against 1.03-1.08 for 1024 x 8).
+// launches on MI355X): one FP scan uses 256 x 4 up to 2^19 elements (2^18 + 1
+// pairs: 5.2 against 5.9 us for 1024 x 4; 2^20: 7.7 against 6.8), 1024 x 4 up
+// to 2^22 and 1024 x 8 above. The segmented FP kernel uses 256 x 4 below 2^20,
+// 512 x 4 up to 9 * 2^18 and 1024 x 4 above: its runs are walked through LDS
+// twice, and until the chip is full smaller workgroups start and end that
+// earlier (FP32 pairs, 100 / 100000 segments: 700,000 elements 6.4 / 7.6 us at
+// 256 x 4, 6.7 / 7.8 at 512 x 4; 2,000,000 7.6 / 8.6 at 512 x 4, 8.8 / 10.1 at
+// 1024 x 4; 2,500,000 9.0 / 10.2 at 512 x 4, 8.6 / 10.4 at 1024 x 4).
 gps::TileShape fp_shape(const gps_handle* h, uint64_t n, bool segmented) {
     if (h->size_adaptive) {
-        if (segmented) return n < (1ull << 20) ? gps::TileShape{256, 4} : gps::TileShape{1024, 4};
-        return n <= (1ull << 18) ? gps::TileShape{256, 4} : n <= (1ull << 22) ? gps::TileShape{1024, 4}
+        if (segmented)
+            return n < (1ull << 20) ? gps::TileShape{256, 4} : n <= (9ull << 18) ? gps::kSegFpMid
+                                                                                 : gps::TileShape{1024, 4};
+        return n <= (1ull << 19) ? gps::TileShape{256, 4} : n <= (1ull << 22) ? gps::TileShape{1024, 4}
                                                                                : gps::TileShape{1024, 8};
     }
     return gps::fp_shape_supported(h->shape) ? h->shape : gps::TileShape{1024, 4};
@@ -72,11 +78,14 @@ int enqueue_segmented(gps_handle* h, const uint32_t* in, uint32_t* out, const ui
 namespace {
 
 // One FP scan with pair or plain carries runs the persistent kernel on a
-// handle with the persistent schedule (the CSDL default); a default handle
-// picks it above 2^24 elements (2^25 FP32 pairs: 4398 against 4319 GB/s for
-// one workgroup per tile; 2^23: 3663 against 3778).
+// handle with the persistent schedule (the CSDL default). A default handle
+// picks it above 2^23 elements, against one workgroup per tile, both at
+// 1024 x 8: FP32 pairs 2^23 15.4 against 13.0 us, 9,000,000 16.6 against
+// 20.3; BF16 pairs 14.1 against 12.8 and 14.8 against 19.7; FP32 plain 14.3
+// against 11.7 and 15.0 against 16.7. (Between 5 and 7 million FP32 pairs it
+// is up to 8% faster, BF16 pairs slower, plain carries either.)
 bool fp_persistent(const gps_handle* h, uint64_t n) {
-    if (h->size_adaptive) return n > (1ull << 24);
+    if (h->size_adaptive) return n > (1ull << 23);
     return h->schedule == GPS_SCHEDULE_PERSISTENT;
 }
 
@@ -96,8 +105,8 @@ int scan_fp(gps_handle* h, const void* in, float* out, uint64_t n, bool bf16, in
     const gps::TileShape s = fp_shape(h, n, false);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
-    HIP_TRY(gps::launch_scan_fp(s, bf16, compensated, fp_persistent(h, n), in, out, n, h->status, h->ticket, h->err,
-                                st));
+    HIP_TRY(gps::launch_scan_fp(s, bf16, compensated, fp_persistent(h, n), h->round_patience, in, out, n,
+                                h->status, h->ticket, h->err, st));
     return GPS_OK;
 }
 
@@ -131,8 +140,8 @@ int segscan_fp(gps_handle* h, const void* in, float* out, const uint64_t* offset
     const gps::TileShape s = persistent && h->size_adaptive ? gps::TileShape{1024, 8} : fp_shape(h, n, true);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
-    HIP_TRY(gps::launch_segscan_fp(s, bf16, compensated != 0, persistent, in, out, offsets, num_segments, n,
-                                   h->status, h->ticket, h->err, st));
+    HIP_TRY(gps::launch_segscan_fp(s, bf16, compensated != 0, persistent, h->round_patience, in, out, offsets,
+                                   num_segments, n, h->status, h->ticket, h->err, st));
     return GPS_OK;
 }
 

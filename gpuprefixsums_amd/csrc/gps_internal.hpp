@@ -18,6 +18,11 @@ constexpr uint64_t kSlotWords = 16;
 constexpr uint64_t kCounterWords = 8;
 constexpr uint64_t kCounterOccupancy = 4;
 
+// Polls of a status window before a wave of a one-round scan computes a
+// missing tile's aggregate itself: tens of microseconds, far beyond what a
+// workgroup that has started needs.
+constexpr uint32_t kRoundPatience = 64;
+
 // Launch parameters shared by the single-pass uint32 kernels (CSDL, CSDLDF).
 struct ScanParams {
     const uint32_t* in;
@@ -27,8 +32,8 @@ struct ScanParams {
     uint64_t* status;  // one word per tile
     uint64_t* ticket;  // (epoch << 32) | tickets taken
     uint32_t* err;     // device error bits (watchdogs)
+    uint32_t spin_limit;  // decoupled fallback, and the one-round scan's patience
     // decoupled fallback only
-    uint32_t spin_limit;
     uint32_t stall_period;              // 0: no emulated stalls
     unsigned long long* counters;       // [polls, fallbacks, insertions, stall timeouts] or null
     // persistent CSDL only: +1 per workgroup that takes a tile, or null
@@ -94,12 +99,11 @@ bool shape_supported(TileShape s);
 // Shape and schedule of a default CSDL handle for an n-element scan (the
 // schedule constants of gps.h: 1 = one workgroup per tile, 2 = persistent),
 // measured on MI355X (back-to-back launches): below 2^24 elements one
-// workgroup per tile beats the persistent grid, which has too few tiles per
-// workgroup to pay for its ramp; below 2^22 smaller tiles also shorten the
-// lookback chain. 2^16: 3.6 against 5.5 us; 2^20: 6.1 against 7.4 us; 2^23:
-// 14.4 against 15.4 us; from 2^24 up the persistent 1024 x 8 kernel wins
-// (26.7 against 28.9 us at 2^24). Leaves shape and schedule unchanged from
-// 2^24 up (the persistent 1024 x 8 default).
+// workgroup per tile, all started together (the one-round scan), beats the
+// persistent grid, which has too few tiles per workgroup to pay for its ramp;
+// up to 2^21 smaller tiles also occupy more of the chip. 2^20: 5.1 us; 2^23:
+// 11.4 against 14.5; 12,345,677: 17.9 against 18.2; just below 2^24 24.1
+// against 23.0. Leaves shape and schedule unchanged there.
 inline void size_adaptive_config(uint64_t n, TileShape& shape, uint32_t& schedule) {
     constexpr uint32_t kTile = 1;  // GPS_SCHEDULE_TILE
     if (n <= (1ull << 18)) {
@@ -153,13 +157,15 @@ bool fp_shape_supported(TileShape s);
 enum FpCarry : int { kFpPlain = 0, kFpPair = 1 };
 // persistent: resident workgroups loop over ticketed tiles, loading tile i+1
 // while tile i's lookback resolves (otherwise one workgroup per tile).
-hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, const void* in, float* out,
-                          uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
+hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, uint32_t patience, const void* in,
+                          float* out, uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
                           hipStream_t stream);
 // Batched segmented FP inclusive scan (one launch; same shapes as launch_scan_fp;
-// persistent as there).
-hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, const void* in, float* out,
-                             const uint64_t* offsets, uint64_t num_segments, uint64_t n,
+// persistent as there), and one workgroup per tile of shape kSegFpMid for 2 to
+// 513 tiles.
+constexpr TileShape kSegFpMid{512, 4};
+hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, uint32_t patience,
+                             const void* in, float* out, const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                              uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream);
 
 // Member-wise scan of n 4-member uint32 structs (4 status words per tile).

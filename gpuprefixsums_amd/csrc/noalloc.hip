@@ -99,6 +99,7 @@ extern "C" int gps_scan_u32_noalloc(const uint32_t* d_in, uint32_t* d_out, uint6
     p.out = d_out;
     p.n = n;
     p.num_tiles = (uint32_t)tiles;
+    p.spin_limit = gps::kRoundPatience;
     p.status = w;
     p.ticket = w + kTicketWord;
     p.err = reinterpret_cast<uint32_t*>(w + kErrWord);

@@ -52,23 +52,29 @@ __device__ __forceinline__ ff ff_add1(ff x, float v) {
 #define GPS_DPP_F(x, CTRL, RM, BC) \
     __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (x)), CTRL, RM, 0xf, BC))
 
-// Inclusive wave scan of pairs (same DPP schedule as the integer scan).
-template <bool COMP>
-__device__ __forceinline__ ff wave_incl_scan_ff(ff x) {
-#define GPS_FF_STEP(CTRL, RM, BC)                                                 \
-    {                                                                             \
-        const ff y = {GPS_DPP_F(x.s, CTRL, RM, BC), COMP ? GPS_DPP_F(x.c, CTRL, RM, BC) : 0.f}; \
-        x = ff_add<COMP>(y, x);                                                   \
+// Inclusive scans of pairs over each row of 16 lanes, and over the wave (same
+// DPP schedule as the integer scan).
+#define GPS_FF_STEP(CTRL, RM, BC)                                                                   \
+    {                                                                                               \
+        const ff y = {GPS_DPP_F(x.s, CTRL, RM, BC), COMP ? GPS_DPP_F(x.c, CTRL, RM, BC) : 0.f};     \
+        x = ff_add<COMP>(y, x);                                                                     \
     }
+template <bool COMP>
+__device__ __forceinline__ ff row_incl_scan_ff(ff x) {
     GPS_FF_STEP(0x111, 0xf, true)
     GPS_FF_STEP(0x112, 0xf, true)
     GPS_FF_STEP(0x114, 0xf, true)
     GPS_FF_STEP(0x118, 0xf, true)
-    GPS_FF_STEP(0x142, 0xa, false)
-    GPS_FF_STEP(0x143, 0xc, false)
-#undef GPS_FF_STEP
     return x;
 }
+template <bool COMP>
+__device__ __forceinline__ ff wave_incl_scan_ff(ff x) {
+    x = row_incl_scan_ff<COMP>(x);
+    GPS_FF_STEP(0x142, 0xa, false)
+    GPS_FF_STEP(0x143, 0xc, false)
+    return x;
+}
+#undef GPS_FF_STEP
 
 __device__ __forceinline__ float readlane_f(float x, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
@@ -157,11 +163,28 @@ __device__ __forceinline__ ff lookback_ff(const uint64_t* status, uint32_t tile,
     }
 }
 
+// Wave totals in LDS (after a barrier): lane q takes wave q's total (at most
+// 16) and one pair row scan gives this wave's exclusive prefix and the tile total (a
+// serial loop over the totals held 32 more registers: 102 against 79 VGPRs at
+// 1024 x 8).
+template <int WAVES, bool COMP>
+__device__ __forceinline__ void combine_waves_ff(const float* s_s, const float* s_c, uint32_t wave, ff& wave_pre,
+                                                 ff& total) {
+    const uint32_t lane = lane_id();
+    const uint32_t q = lane < (uint32_t)WAVES ? lane : 0u;
+    const ff v = {lane < (uint32_t)WAVES ? s_s[q] : 0.f, lane < (uint32_t)WAVES ? s_c[q] : 0.f};
+    const ff sc = row_incl_scan_ff<COMP>(v);
+    const ff ex = {GPS_DPP_F(sc.s, 0x138, 0xf, true), COMP ? GPS_DPP_F(sc.c, 0x138, 0xf, true) : 0.f};
+    wave_pre = {readlane_f(ex.s, (int)wave), COMP ? readlane_f(ex.c, (int)wave) : 0.f};
+    total = {readlane_f(sc.s, WAVES - 1), COMP ? readlane_f(sc.c, WAVES - 1) : 0.f};
+}
+
 struct FpParams {
     const void* in;  // float or bf16 bits
     float* out;
     uint64_t n;
     uint32_t num_tiles;
+    uint32_t patience;  // one-round scans: polls before a wave helps
     uint64_t* status;  // 2 words per tile
     uint64_t* ticket;
     uint32_t* err;
@@ -227,6 +250,120 @@ __device__ __forceinline__ void store_fp(float* out, const f32x4 (&x)[VEC], uint
     store_tile<VEC>(reinterpret_cast<uint32_t*>(out), d, 0u, start, n, tile_elems);
 }
 
+// A wave's slice of LDS for the lane-blocked layout (see scan_fp_bl).
+template <int VEC>
+struct BlockedSlice {
+    static constexpr uint32_t kRow = 4u * VEC + 4u;  // floats per padded row
+    static constexpr uint32_t kFloats = 64u * kRow;
+};
+
+// Striped (lane l, vector k) <-> blocked (lane l, vector q) through the
+// wave's LDS slice. Striped element of (k, l, c): 256k + 4l + c; blocked
+// element of (l, q, c): 4*VEC*l + 4q + c.
+template <int VEC>
+__device__ __forceinline__ void striped_to_blocked(f32x4 (&x)[VEC], float* slice) {
+    using S = BlockedSlice<VEC>;
+    const uint32_t l = lane_id();
+    constexpr uint32_t kRowsPerVec = 256u / (4u * VEC);  // rows covered by one striped vector
+    constexpr uint32_t kLanesPerRow = VEC;                // striped lanes that share a row
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+        const uint32_t row = k * kRowsPerVec + l / kLanesPerRow;
+        *reinterpret_cast<f32x4*>(slice + row * S::kRow + 4u * (l % kLanesPerRow)) = x[k];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) x[q] = *reinterpret_cast<const f32x4*>(slice + l * S::kRow + 4u * q);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int VEC>
+__device__ __forceinline__ void blocked_to_striped(f32x4 (&x)[VEC], float* slice) {
+    using S = BlockedSlice<VEC>;
+    const uint32_t l = lane_id();
+    constexpr uint32_t kRowsPerVec = 256u / (4u * VEC);
+    constexpr uint32_t kLanesPerRow = VEC;
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) *reinterpret_cast<f32x4*>(slice + l * S::kRow + 4u * q) = x[q];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+        const uint32_t row = k * kRowsPerVec + l / kLanesPerRow;
+        x[k] = *reinterpret_cast<const f32x4*>(slice + row * S::kRow + 4u * (l % kLanesPerRow));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The tile in registers. Plain carries stay striped: per vector the lane's
+// total and a wave scan give the lane's carry inside the wave's run. Pair
+// carries are lane-blocked: the run is transposed through the wave's LDS slice
+// so that a lane holds 4 * VEC consecutive elements and one pair wave scan
+// serves the run instead of VEC. The wave totals meet in LDS (s_ws, s_wc; a
+// barrier between scan_run and combine); each output is recomputed from its
+// input and its carry.
+template <int BLOCK, int VEC, bool COMP>
+struct FpTile {
+    using C = TileCfg<BLOCK, VEC>;
+    static constexpr uint32_t kSliceFloats = COMP ? C::kWaves * BlockedSlice<VEC>::kFloats : 1u;
+    f32x4 x[VEC];
+    ff lane_carry[COMP ? 1 : VEC];
+    ff wave_pre, total;
+
+    __device__ __forceinline__ static ff shr1(ff s) {  // exclusive = inclusive of the lane below (lane 0: zero)
+        return {GPS_DPP_F(s.s, 0x138, 0xf, true), COMP ? GPS_DPP_F(s.c, 0x138, 0xf, true) : 0.f};
+    }
+    __device__ __forceinline__ void scan_run(float* slice, float* s_ws, float* s_wc, uint32_t wave) {
+        ff run = {0.f, 0.f};
+        if constexpr (COMP) {
+            striped_to_blocked<VEC>(x, slice);
+            ff t = {x[0].x, 0.f};
+#pragma unroll
+            for (int e = 1; e < 4 * VEC; ++e) t = ff_add1<COMP>(t, x[e / 4][e % 4]);
+            const ff s = wave_incl_scan_ff<COMP>(t);
+            lane_carry[0] = shr1(s);
+            run = {readlane_f(s.s, 63), readlane_f(s.c, 63)};
+        } else {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                ff t = {x[k].x, 0.f};
+                t = ff_add1<COMP>(t, x[k].y);
+                t = ff_add1<COMP>(t, x[k].z);
+                t = ff_add1<COMP>(t, x[k].w);
+                const ff s = wave_incl_scan_ff<COMP>(t);
+                lane_carry[k] = ff_add<COMP>(run, shr1(s));
+                run = ff_add<COMP>(run, {readlane_f(s.s, 63), 0.f});
+            }
+        }
+        if (lane_id() == 0) {
+            s_ws[wave] = run.s;
+            s_wc[wave] = run.c;
+        }
+    }
+    __device__ __forceinline__ void combine(const float* s_ws, const float* s_wc, uint32_t wave) {
+        combine_waves_ff<C::kWaves, COMP>(s_ws, s_wc, wave, wave_pre, total);
+    }
+    __device__ __forceinline__ void outputs(ff prefix, float* slice) {
+        const ff base = ff_add<COMP>(prefix, wave_pre);
+        ff acc = ff_add<COMP>(base, lane_carry[0]);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            if (!COMP && k) acc = ff_add<COMP>(base, lane_carry[k]);
+            f32x4 y;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                acc = ff_add1<COMP>(acc, x[k][c]);
+                y[c] = acc.s + acc.c;
+            }
+            x[k] = y;
+        }
+        if constexpr (COMP) blocked_to_striped<VEC>(x, slice);
+    }
+};
+
 template <int BLOCK, int VEC, bool BF16, bool COMP>
 __global__ __launch_bounds__(BLOCK) void scan_fp(FpParams p) {
     using C = TileCfg<BLOCK, VEC>;
@@ -241,53 +378,24 @@ __global__ __launch_bounds__(BLOCK) void scan_fp(FpParams p) {
         s_ticket[1] = t.epoch;
     }
     __syncthreads();
-    const uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]), epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
-    f32x4 x[VEC];
-    load_fp<BF16, VEC>(x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
-
-    // Per vector: lane total (pair), wave exclusive scan -> lane carry L_k.
-    ff lane_carry[VEC];
-    ff run = {0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-        ff t = {x[k].x, 0.f};
-        t = ff_add1<COMP>(t, x[k].y);
-        t = ff_add1<COMP>(t, x[k].z);
-        t = ff_add1<COMP>(t, x[k].w);
-        const ff s = wave_incl_scan_ff<COMP>(t);
-        // exclusive = inclusive of the lane below (lane 0: zero)
-        ff e;
-        e.s = GPS_DPP_F(s.s, 0x138, 0xf, true);  // wave_shr:1
-        e.c = COMP ? GPS_DPP_F(s.c, 0x138, 0xf, true) : 0.f;
-        lane_carry[k] = ff_add<COMP>(run, e);
-        const ff tot = {readlane_f(s.s, 63), COMP ? readlane_f(s.c, 63) : 0.f};
-        run = ff_add<COMP>(run, tot);
-    }
-    if (lane == 0) {
-        s_ws[wave] = run.s;
-        s_wc[wave] = run.c;
-    }
+    const uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]),
+                   epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
+    using F = FpTile<BLOCK, VEC, COMP>;
+    __shared__ __align__(16) float s_slices[F::kSliceFloats];
+    float* const slice = s_slices + wave * (F::kSliceFloats / C::kWaves);
+    F f;
+    load_fp<BF16, VEC>(f.x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
+    f.scan_run(slice, s_ws, s_wc, wave);
     __syncthreads();
-    // Wave totals: lane q takes wave q's total and one pair wave scan gives
-    // every wave its exclusive prefix and the tile total (a serial loop over
-    // the totals held 32 more registers: 102 against 79 VGPRs at 1024 x 8).
-    ff wave_pre, tile_tot;
-    {
-        const uint32_t q = lane < C::kWaves ? lane : 0u;
-        const ff v = {lane < C::kWaves ? s_ws[q] : 0.f, lane < C::kWaves ? s_wc[q] : 0.f};
-        const ff sc = wave_incl_scan_ff<COMP>(v);
-        const ff ex = {GPS_DPP_F(sc.s, 0x138, 0xf, true), COMP ? GPS_DPP_F(sc.c, 0x138, 0xf, true) : 0.f};
-        wave_pre = {readlane_f(ex.s, (int)wave), COMP ? readlane_f(ex.c, (int)wave) : 0.f};
-        tile_tot = {readlane_f(sc.s, C::kWaves - 1), COMP ? readlane_f(sc.c, C::kWaves - 1) : 0.f};
-    }
+    f.combine(s_ws, s_wc, wave);
     if (wave == 0) {
         ff prefix = {0.f, 0.f};
         if (tile == 0) {
-            if (lane == 0) publish_ff<COMP>(p.status, 0, tile_tot, kFlagIncl, epoch);
+            if (lane == 0) publish_ff<COMP>(p.status, 0, f.total, kFlagIncl, epoch);
         } else {
-            if (lane == 0) publish_ff<COMP>(p.status, tile, tile_tot, kFlagAgg, epoch);
+            if (lane == 0) publish_ff<COMP>(p.status, tile, f.total, kFlagAgg, epoch);
             prefix = lookback_ff<COMP>(p.status, tile, epoch, p.err);
-            if (lane == 0) publish_ff<COMP>(p.status, tile, ff_add<COMP>(prefix, tile_tot), kFlagIncl, epoch);
+            if (lane == 0) publish_ff<COMP>(p.status, tile, ff_add<COMP>(prefix, f.total), kFlagIncl, epoch);
         }
         if (lane == 0) {
             s_ps = prefix.s;
@@ -295,19 +403,118 @@ __global__ __launch_bounds__(BLOCK) void scan_fp(FpParams p) {
         }
     }
     __syncthreads();
-    const ff base_carry = ff_add<COMP>({s_ps, s_pc}, wave_pre);
+    f.outputs({s_ps, s_pc}, slice);
+    store_fp<VEC>(p.out, f.x, (uint64_t)tile * C::kTile, p.n, C::kTile);
+}
+
+// ---------------------------------------------------------------------------
+// One-round FP scan (device_common.hpp): the tile schedule up to kRoundTiles
+// tiles; a single tile takes no ticket and publishes nothing. Back to back,
+// FP32 pairs, against tickets and a chained lookback over lane-striped tiles:
+// 1000 elements 2.6 us (4.1), 2^16 4.6 (4.6), 2^20 6.7 (8.1), 2^22 9.0 (11.5),
+// 2^23 13.0 (15.5 in scan_fp_bl); 3,000,017 BF16 7.8 (9.9).
+// ---------------------------------------------------------------------------
+// Four elements at element i (a whole vector inside the input).
+template <bool BF16>
+__device__ __forceinline__ f32x4 load_fp4(const void* in, uint64_t i) {
+    if (BF16) return widen(*reinterpret_cast<const u16x4_any*>(static_cast<const uint16_t*>(in) + i));
+    return *reinterpret_cast<const f32x4_any*>(static_cast<const float*>(in) + i);
+}
+
+// Sum of the elements [from, to) by one wave, in pairs.
+template <bool BF16, bool COMP>
+__device__ __forceinline__ ff help_sum_ff(const void* in, uint64_t from, uint64_t to) {
+    ff t = {0.f, 0.f};
+    for (uint64_t i = from + 4u * lane_id(); i < to; i += 256u) {
+        if (i + 4u <= to) {
+            const f32x4 x = load_fp4<BF16>(in, i);
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-        ff acc = ff_add<COMP>(base_carry, lane_carry[k]);
-        f32x4 y;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            acc = ff_add1<COMP>(acc, x[k][c]);
-            y[c] = acc.s + acc.c;
+            for (int c = 0; c < 4; ++c) t = ff_add1<COMP>(t, x[c]);
+        } else {
+            for (uint64_t j = i; j < to; ++j)
+                t = ff_add1<COMP>(t, BF16 ? __builtin_bit_cast(float, (uint32_t)static_cast<const uint16_t*>(in)[j] << 16)
+                                          : static_cast<const float*>(in)[j]);
         }
-        x[k] = y;
     }
-    store_fp<VEC>(p.out, x, (uint64_t)tile * C::kTile, p.n, C::kTile);
+    const ff s = wave_incl_scan_ff<COMP>(t);
+    return {readlane_f(s.s, 63), COMP ? readlane_f(s.c, 63) : 0.f};
+}
+
+// Sum of the aggregates of the tiles top, top - 1, ..., at most 64 (one wave).
+template <uint32_t TILE, bool BF16, bool COMP>
+__device__ __forceinline__ ff round_window_ff(const FpParams& p, int64_t top, uint32_t epoch) {
+    const uint32_t lane = lane_id();
+    const int64_t idx = top - (int64_t)lane;
+    const uint64_t* const slot = p.status + kSlotWords * (uint64_t)(idx >= 0 ? idx : 0);
+    bool helped = idx < 0;
+    ff value = {0.f, 0.f};
+    uint32_t polls = 0;
+    while (true) {
+        uint64_t ws, wc;
+        load_pair_words(slot, ws, wc);
+        const uint32_t fs = status_flag(ws, epoch);
+        const bool ready = fs != 0u && fs == status_flag(wc, epoch);
+        if (ready && !helped) value = {__builtin_bit_cast(float, (uint32_t)ws), __builtin_bit_cast(float, (uint32_t)wc)};
+        const uint64_t missing = ballot(!ready && !helped);
+        if (!missing) {
+            const ff s = wave_incl_scan_ff<COMP>(value);
+            return {readlane_f(s.s, 63), COMP ? readlane_f(s.c, 63) : 0.f};
+        }
+        if (++polls < p.patience) {
+            __builtin_amdgcn_s_sleep(1);
+            continue;
+        }
+        const uint32_t l = (uint32_t)__builtin_ctzll(missing);
+        const uint32_t j = (uint32_t)(top - (int64_t)l);
+        ff sum = help_sum_ff<BF16, COMP>(p.in, (uint64_t)j * TILE, (uint64_t)(j + 1u) * TILE);
+        wait_performed();
+        load_pair_words(p.status + kSlotWords * (uint64_t)j, ws, wc);
+        if (status_flag(ws, epoch) != 0u && status_flag(ws, epoch) == status_flag(wc, epoch))
+            sum = {__builtin_bit_cast(float, (uint32_t)ws), __builtin_bit_cast(float, (uint32_t)wc)};
+        if (lane == l) {
+            value = sum;
+            helped = true;
+        }
+    }
+}
+
+template <int BLOCK, int VEC, bool BF16, bool COMP, bool SINGLE>
+__global__ __launch_bounds__(BLOCK) void scan_fp_round(FpParams p) {
+    using C = TileCfg<BLOCK, VEC>;
+    __shared__ float s_ws[C::kWaves], s_wc[C::kWaves];
+    __shared__ float s_bs[C::kWaves], s_bc[C::kWaves];
+    __shared__ uint32_t s_epoch;
+    const uint32_t tile = SINGLE ? 0u : blockIdx.x, wave = wave_index(), lane = lane_id();
+    uint64_t entered = 0;
+    if (!SINGLE && threadIdx.x == 0) entered = round_enter(p.ticket, p.num_tiles);
+    using F = FpTile<BLOCK, VEC, COMP>;
+    __shared__ __align__(16) float s_slices[F::kSliceFloats];
+    float* const slice = s_slices + wave * (F::kSliceFloats / C::kWaves);
+    F f;
+    load_fp<BF16, VEC>(f.x, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
+    f.scan_run(slice, s_ws, s_wc, wave);
+    if (!SINGLE && threadIdx.x == 0) s_epoch = round_epoch(p.ticket, entered, p.num_tiles);
+    __syncthreads();
+    f.combine(s_ws, s_wc, wave);
+    ff prefix = {0.f, 0.f};
+    if (!SINGLE) {
+        const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
+        if (threadIdx.x == 0) publish_ff<COMP>(p.status, tile, f.total, kFlagAgg, epoch);
+        ff before = {0.f, 0.f};
+        for (int64_t top = (int64_t)tile - 1 - 64 * (int64_t)wave; top >= 0; top -= 64 * (int64_t)C::kWaves)
+            before = ff_add<COMP>(before, round_window_ff<C::kTile, BF16, COMP>(p, top, epoch));
+        if (lane == 0) {
+            s_bs[wave] = before.s;
+            s_bc[wave] = before.c;
+        }
+        if (wave == 0) wait_performed();  // the words above, before any wave's output stores
+        if (threadIdx.x == BLOCK - kWave) round_leave(p.ticket, p.status, tile, p.num_tiles);
+        __syncthreads();
+        ff unused;
+        combine_waves_ff<C::kWaves, COMP>(s_bs, s_bc, wave, unused, prefix);
+    }
+    f.outputs(prefix, slice);
+    store_fp<VEC>(p.out, f.x, (uint64_t)tile * C::kTile, p.n, C::kTile);
 }
 
 // ---------------------------------------------------------------------------
@@ -536,6 +743,7 @@ struct SegFpParams {
     uint64_t num_segments;
     uint64_t n;
     uint32_t num_tiles;
+    uint32_t patience;  // one-round scans: polls before a wave helps
     uint64_t* status;  // 2 words per tile
     uint64_t* ticket;
     uint32_t* err;
@@ -844,53 +1052,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
 // instructions of one wave complete in order, and a wavefront-scope fence
 // keeps the compiler from reordering the cross-lane write/read pairs.
 // ---------------------------------------------------------------------------
-template <int VEC>
-struct BlockedSlice {
-    static constexpr uint32_t kRow = 4u * VEC + 4u;  // floats per padded row
-    static constexpr uint32_t kFloats = 64u * kRow;
-};
-
-// Striped (lane l, vector k) <-> blocked (lane l, vector q) through the
-// wave's LDS slice. Striped element of (k, l, c): 256k + 4l + c; blocked
-// element of (l, q, c): 4*VEC*l + 4q + c.
-template <int VEC>
-__device__ __forceinline__ void striped_to_blocked(f32x4 (&x)[VEC], float* slice) {
-    using S = BlockedSlice<VEC>;
-    const uint32_t l = lane_id();
-    constexpr uint32_t kRowsPerVec = 256u / (4u * VEC);  // rows covered by one striped vector
-    constexpr uint32_t kLanesPerRow = VEC;                // striped lanes that share a row
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-        const uint32_t row = k * kRowsPerVec + l / kLanesPerRow;
-        *reinterpret_cast<f32x4*>(slice + row * S::kRow + 4u * (l % kLanesPerRow)) = x[k];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int q = 0; q < VEC; ++q) x[q] = *reinterpret_cast<const f32x4*>(slice + l * S::kRow + 4u * q);
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-template <int VEC>
-__device__ __forceinline__ void blocked_to_striped(f32x4 (&x)[VEC], float* slice) {
-    using S = BlockedSlice<VEC>;
-    const uint32_t l = lane_id();
-    constexpr uint32_t kRowsPerVec = 256u / (4u * VEC);
-    constexpr uint32_t kLanesPerRow = VEC;
-#pragma unroll
-    for (int q = 0; q < VEC; ++q) *reinterpret_cast<f32x4*>(slice + l * S::kRow + 4u * q) = x[q];
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-        const uint32_t row = k * kRowsPerVec + l / kLanesPerRow;
-        x[k] = *reinterpret_cast<const f32x4*>(slice + row * S::kRow + 4u * (l % kLanesPerRow));
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 template <int BLOCK, int VEC, bool BF16, class Ops>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void scan_fp_bl(FpParams p) {
     using C = TileCfg<BLOCK, VEC>;
@@ -1172,6 +1333,167 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     }
 }
 
+// ---------------------------------------------------------------------------
+// One-round segmented FP scan (device_common.hpp): one workgroup per tile
+// while a workgroup's waves cover the tiles before it in one window each; a
+// single tile takes no ticket and publishes nothing. Lane-blocked runs as
+// segscan_fp_bl. The search for the tile's heads starts with its loads.
+// Back to back, FP32 pairs, against segscan_fp (tickets, window lookback,
+// striped): 1000 elements 3.5 us (5.6), 2^16 in 1000 segments 5.7 (6.4), 2^20
+// in 16384 segments 8.2 (11.1), 2^21 + 17 in 16384 segments 8.9 (12.0).
+// ---------------------------------------------------------------------------
+// The carry that the tiles top, top - 1, ... (at most 64; one wave) pass on:
+// the sum back to the nearest tile that holds a head; `closed` if there is one.
+template <uint32_t TILE, bool BF16, bool COMP>
+__device__ __forceinline__ ff round_window_seg_ff(const SegFpParams& p, int64_t top, uint32_t epoch, bool& closed) {
+    const uint32_t lane = lane_id();
+    const int64_t idx = top - (int64_t)lane;
+    const uint64_t* const slot = p.status + kSlotWords * (uint64_t)(idx >= 0 ? idx : 0);
+    bool helped = idx < 0;
+    uint32_t flag = (uint32_t)kFlagIncl;
+    ff value = {0.f, 0.f};
+    uint32_t polls = 0;
+    while (true) {
+        uint64_t ws, wc;
+        load_pair_words(slot, ws, wc);
+        const uint32_t f0 = status_flag(ws, epoch), f1 = status_flag(wc, epoch);
+        if (!helped) {
+            flag = f0 == f1 ? f0 : 0u;
+            value = {__builtin_bit_cast(float, (uint32_t)ws), __builtin_bit_cast(float, (uint32_t)wc)};
+        }
+        const uint64_t ready = ballot(flag != 0u), incl = ballot(flag == (uint32_t)kFlagIncl);
+        const uint32_t run = (~ready) ? (uint32_t)__builtin_ctzll(~ready) : 64u;
+        const uint32_t first_incl = incl ? (uint32_t)__builtin_ctzll(incl) : 64u;
+        closed = first_incl < run;
+        if (closed || run == 64u) {
+            const uint32_t take = closed ? first_incl + 1u : 64u;
+            const ff s = wave_incl_scan_ff<COMP>(lane < take ? value : ff{0.f, 0.f});
+            return {readlane_f(s.s, 63), COMP ? readlane_f(s.c, 63) : 0.f};
+        }
+        if (++polls < p.patience) {
+            __builtin_amdgcn_s_sleep(1);
+            continue;
+        }
+        const uint32_t j = (uint32_t)(top - (int64_t)run);
+        const uint64_t end = (uint64_t)(j + 1u) * TILE;
+        const TailOfTile tail = find_tail(p.offsets, p.num_segments, end - TILE, end);
+        ff sum = help_sum_ff<BF16, COMP>(p.in, tail.from, end);
+        uint32_t f = tail.has_head ? (uint32_t)kFlagIncl : (uint32_t)kFlagAgg;
+        wait_performed();
+        load_pair_words(p.status + kSlotWords * (uint64_t)j, ws, wc);
+        const uint32_t g0 = status_flag(ws, epoch), g1 = status_flag(wc, epoch);
+        if (g0 != 0u && g0 == g1) {
+            f = g0;
+            sum = {__builtin_bit_cast(float, (uint32_t)ws), __builtin_bit_cast(float, (uint32_t)wc)};
+        }
+        if (lane == run) {
+            flag = f;
+            value = sum;
+            helped = true;
+        }
+    }
+}
+
+template <int BLOCK, int VEC, bool BF16, bool COMP, bool SINGLE>
+__global__ __launch_bounds__(BLOCK) void segscan_fp_round(SegFpParams p) {
+    using C = TileCfg<BLOCK, VEC>;
+    using Ops = PairCarry<COMP>;
+    constexpr uint32_t kWords = C::kTile / 32;
+    __shared__ __align__(16) float s_slices[C::kWaves * BlockedSlice<VEC>::kFloats];
+    __shared__ uint32_t s_heads[kWords], s_bracket[C::kWaves];
+    __shared__ float s_ws[C::kWaves], s_wc[C::kWaves], s_bs[C::kWaves], s_bc[C::kWaves];
+    __shared__ uint32_t s_wf[C::kWaves], s_closed[C::kWaves];
+    __shared__ uint32_t s_epoch;
+    const uint32_t tile = SINGLE ? 0u : blockIdx.x, wave = wave_index(), lane = lane_id();
+    float* const slice = s_slices + wave * BlockedSlice<VEC>::kFloats;
+    const uint64_t lo = (uint64_t)tile * C::kTile;
+    const uint64_t hi = lo + C::kTile < p.n ? lo + C::kTile : p.n;
+    uint64_t entered = 0;
+    if (!SINGLE && threadIdx.x == 0) entered = round_enter(p.ticket, p.num_tiles);
+    f32x4 x[VEC];
+    load_fp<BF16, VEC>(x, p.in, lo, p.n, C::kTile);
+    for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[i] = 0u;
+    __syncthreads();
+    find_and_mark_heads<BLOCK>(s_heads, s_bracket, p.offsets, p.num_segments, lo, hi, tile == 0);
+    __syncthreads();
+
+    // As segscan_fp_bl: the run's segmented total, from its last head on.
+    striped_to_blocked<VEC>(x, slice);
+    const uint32_t heads = lane_run_heads<VEC>(s_heads, wave * C::kWaveElems, lane);
+    ff t = {0.f, 0.f};
+    {
+        const uint32_t last = heads ? 31u - (uint32_t)__builtin_clz(heads) : 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4u * VEC; ++i) t = Ops::add1(t, i >= last ? x[i / 4][i % 4] : 0.f);
+    }
+    uint32_t sf = heads != 0u;
+    ff sv = t;
+    wave_seg_scan_ff<COMP>(sf, sv);
+    const uint32_t ef = GPS_DPP_I(sf, 0x138, 0xf, true);  // wave_shr:1, lane 0 gets 0
+    const ff ev = Ops::shr1(sv);
+    if (lane == 0) {
+        s_ws[wave] = readlane_f(sv.s, 63);
+        s_wc[wave] = COMP ? readlane_f(sv.c, 63) : 0.f;
+        s_wf[wave] = readlane(sf, 63);
+    }
+    if (!SINGLE && threadIdx.x == 0) s_epoch = round_epoch(p.ticket, entered, p.num_tiles);
+    __syncthreads();
+    uint32_t pre_f, tile_f;
+    ff pre, tile_tot;
+    const uint32_t q = lane < C::kWaves ? lane : 0u;
+    {
+        uint32_t f = lane < C::kWaves ? s_wf[q] : 0u;
+        ff v = {lane < C::kWaves ? s_ws[q] : 0.f, lane < C::kWaves ? s_wc[q] : 0.f};
+        wave_seg_scan_ff<COMP>(f, v);
+        const uint32_t wef = GPS_DPP_I(f, 0x138, 0xf, true);
+        pre_f = readlane(wef, (int)wave);
+        pre = Ops::lane(Ops::shr1(v), (int)wave);
+        tile_f = readlane(f, C::kWaves - 1);
+        tile_tot = Ops::lane(v, C::kWaves - 1);
+    }
+    ff prefix = {0.f, 0.f};
+    if (!SINGLE) {
+        const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
+        if (threadIdx.x == 0)
+            publish_ff<COMP>(p.status, tile, tile_tot, (tile_f || tile == 0) ? kFlagIncl : kFlagAgg, epoch);
+        // A tile that starts with a head takes nothing from the ones before.
+        ff before = {0.f, 0.f};
+        bool closed = true;
+        const int64_t top = (int64_t)tile - 1 - 64 * (int64_t)wave;
+        if (top >= 0 && (s_heads[0] & 1u) == 0u)
+            before = round_window_seg_ff<C::kTile, BF16, COMP>(p, top, epoch, closed);
+        if (lane == 0) {
+            s_bs[wave] = before.s;
+            s_bc[wave] = before.c;
+            s_closed[wave] = closed;
+        }
+        if (wave == 0) wait_performed();  // the words above, before any wave's output stores
+        if (threadIdx.x == BLOCK - kWave) round_leave(p.ticket, p.status, tile, p.num_tiles);
+        __syncthreads();
+        // Windows up to the nearest one that is closed.
+        const uint64_t stop = ballot(lane < C::kWaves && s_closed[q] != 0u);
+        const uint32_t take = stop ? (uint32_t)__builtin_ctzll(stop) + 1u : C::kWaves;
+        const ff v = {lane < take ? s_bs[q] : 0.f, lane < take ? s_bc[q] : 0.f};
+        const ff sum = row_incl_scan_ff<COMP>(v);
+        prefix = {readlane_f(sum.s, C::kWaves - 1), COMP ? readlane_f(sum.c, C::kWaves - 1) : 0.f};
+    }
+    const ff run_in = pre_f ? pre : ff_add<COMP>(prefix, pre);
+    ff acc = ef ? ev : ff_add<COMP>(run_in, ev);
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+        f32x4 o;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if ((heads >> (4 * k + c)) & 1u) acc = {0.f, 0.f};
+            acc = Ops::add1(acc, x[k][c]);
+            o[c] = Ops::round(acc);
+        }
+        x[k] = o;
+    }
+    blocked_to_striped<VEC>(x, slice);
+    store_fp<VEC>(p.out, x, lo, p.n, C::kTile);
+}
+
 #define GPS_FP_SHAPES(X) \
     X(256, 4)            \
     X(512, 8)            \
@@ -1212,8 +1534,19 @@ static hipError_t launch_fp_pp_carry(int carry, const FpParams& p, hipStream_t s
     return launch_fp_pp<B, V, BF16, PairCarry<false>>(p, stream);
 }
 
-hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, const void* in, float* out,
-                          uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
+// One workgroup per tile.
+template <int B, int V, bool BF16, bool COMP>
+static void launch_fp_tile(const FpParams& p, hipStream_t stream) {
+    if (p.num_tiles == 1)
+        hipLaunchKernelGGL((scan_fp_round<B, V, BF16, COMP, true>), dim3(1), dim3(B), 0, stream, p);
+    else if (p.num_tiles <= kRoundTiles)
+        hipLaunchKernelGGL((scan_fp_round<B, V, BF16, COMP, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+    else
+        hipLaunchKernelGGL((scan_fp<B, V, BF16, COMP>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+}
+
+hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, uint32_t patience, const void* in,
+                          float* out, uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
                           hipStream_t stream) {
     const bool compensated = carry == kFpPair;
     FpParams p{};
@@ -1223,6 +1556,7 @@ hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, co
     p.num_tiles = (uint32_t)((n + s.tile() - 1) / s.tile());
     p.status = status;
     p.ticket = ticket;
+    p.patience = patience;
     p.err = err;
 #define X(B, V)                                                                                                 \
     if (s.block == B && s.vec == V) {                                                                           \
@@ -1230,13 +1564,13 @@ hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, co
             return bf16 ? launch_fp_pp_carry<B, V, true>(carry, p, stream)                                      \
                         : launch_fp_pp_carry<B, V, false>(carry, p, stream);                                    \
         if (bf16 && compensated)                                                                                \
-            hipLaunchKernelGGL((scan_fp<B, V, true, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);       \
+            launch_fp_tile<B, V, true, true>(p, stream);                                                        \
         else if (bf16)                                                                                          \
-            hipLaunchKernelGGL((scan_fp<B, V, true, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);      \
+            launch_fp_tile<B, V, true, false>(p, stream);                                                       \
         else if (compensated)                                                                                   \
-            hipLaunchKernelGGL((scan_fp<B, V, false, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);      \
+            launch_fp_tile<B, V, false, true>(p, stream);                                                       \
         else                                                                                                    \
-            hipLaunchKernelGGL((scan_fp<B, V, false, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);     \
+            launch_fp_tile<B, V, false, false>(p, stream);                                                      \
         return hipGetLastError();                                                                               \
     }
     GPS_FP_SHAPES(X)
@@ -1261,8 +1595,26 @@ static hipError_t launch_segfp_pp(const SegFpParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, const void* in, float* out,
-                             const uint64_t* offsets, uint64_t num_segments, uint64_t n,
+// One workgroup per tile.
+template <int B, int V, bool BF16, bool COMP>
+static void launch_segfp_tile(const SegFpParams& p, hipStream_t stream) {
+    if (p.num_tiles == 1)
+        hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, COMP, true>), dim3(1), dim3(B), 0, stream, p);
+    else if (p.num_tiles <= (uint32_t)B + 1u)  // B / 64 waves x 64 tiles
+        hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, COMP, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+    else
+        hipLaunchKernelGGL((segscan_fp<B, V, BF16, COMP>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+}
+
+// kSegFpMid: 2 to 513 tiles.
+template <bool BF16, bool COMP>
+static void launch_segfp_round(const SegFpParams& p, hipStream_t stream) {
+    hipLaunchKernelGGL((segscan_fp_round<kSegFpMid.block, kSegFpMid.vec, BF16, COMP, false>), dim3(p.num_tiles),
+                       dim3(kSegFpMid.block), 0, stream, p);
+}
+
+hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, uint32_t patience,
+                             const void* in, float* out, const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                              uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream) {
     SegFpParams p{};
     p.in = in;
@@ -1273,7 +1625,20 @@ hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool pers
     p.num_tiles = (uint32_t)((n + s.tile() - 1) / s.tile());
     p.status = status;
     p.ticket = ticket;
+    p.patience = patience;
     p.err = err;
+    if (s.block == kSegFpMid.block && s.vec == kSegFpMid.vec) {
+        if (persistent || p.num_tiles < 2 || p.num_tiles > (uint32_t)kSegFpMid.block + 1u) return hipErrorInvalidValue;
+        if (bf16 && compensated)
+            launch_segfp_round<true, true>(p, stream);
+        else if (bf16)
+            launch_segfp_round<true, false>(p, stream);
+        else if (compensated)
+            launch_segfp_round<false, true>(p, stream);
+        else
+            launch_segfp_round<false, false>(p, stream);
+        return hipGetLastError();
+    }
 #define X(B, V)                                                                                                  \
     if (s.block == B && s.vec == V) {                                                                            \
         if (persistent)                                                                                          \
@@ -1282,13 +1647,13 @@ hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool pers
                         : (compensated ? launch_segfp_pp<B, V, false, true>(p, stream)                           \
                                        : launch_segfp_pp<B, V, false, false>(p, stream));                        \
         if (bf16 && compensated)                                                                                 \
-            hipLaunchKernelGGL((segscan_fp<B, V, true, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);     \
+            launch_segfp_tile<B, V, true, true>(p, stream);                                                      \
         else if (bf16)                                                                                           \
-            hipLaunchKernelGGL((segscan_fp<B, V, true, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);    \
+            launch_segfp_tile<B, V, true, false>(p, stream);                                                     \
         else if (compensated)                                                                                    \
-            hipLaunchKernelGGL((segscan_fp<B, V, false, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);    \
+            launch_segfp_tile<B, V, false, true>(p, stream);                                                     \
         else                                                                                                     \
-            hipLaunchKernelGGL((segscan_fp<B, V, false, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);   \
+            launch_segfp_tile<B, V, false, false>(p, stream);                                                    \
         return hipGetLastError();                                                                                \
     }
     GPS_FP_SHAPES(X)

@@ -102,6 +102,109 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(GPS_WAVES
 }
 
 // ---------------------------------------------------------------------------
+// One-round CSDL (device_common.hpp): the tile schedule up to kRoundTiles
+// tiles. Back to back, against csdl_u32: 2^16 elements 3.7 us (3.9), 2^20 5.1
+// (5.4), 2^22 8.1 (8.6), 2^23 11.4 (14.2; 14.7 in csdl_pp_u32).
+// ---------------------------------------------------------------------------
+// Sum of tile j (a full one) by one wave, with the carry-in tile 0 starts from.
+template <uint32_t TILE>
+__device__ __forceinline__ uint32_t help_tile_u32(const ScanParams& p, uint32_t j) {
+    const u32x4_any* v = reinterpret_cast<const u32x4_any*>(p.in + (uint64_t)j * TILE) + lane_id();
+    uint32_t sum = 0;
+#pragma unroll 4
+    for (uint32_t k = 0; k < TILE / 256u; ++k) {
+        const u32x4 x = v[k * 64u];
+        sum += x.x + x.y + x.z + x.w;
+    }
+    return wave_sum(sum) + (j == 0 && p.carry_in ? *p.carry_in : 0u);
+}
+
+// Sum of the aggregates of the tiles top, top - 1, ..., at most 64 (one wave).
+template <uint32_t TILE>
+__device__ __forceinline__ uint32_t round_window_u32(const ScanParams& p, int64_t top, uint32_t epoch) {
+    const uint32_t lane = lane_id();
+    const int64_t idx = top - (int64_t)lane;
+    uint64_t* const word = p.status + kSlotWords * (uint64_t)(idx >= 0 ? idx : 0);
+    bool helped = idx < 0;  // this lane's value is final without its word
+    uint32_t value = 0, polls = 0;
+    while (true) {
+        const uint64_t w = atomic_load_agent(word);
+        const bool ready = status_flag(w, epoch) != 0u;
+        value = helped || !ready ? value : (uint32_t)w;
+        const uint64_t missing = ballot(!ready && !helped);
+        if (!missing) return wave_sum(value);
+        if (++polls < p.spin_limit) {
+            __builtin_amdgcn_s_sleep(GPS_POLL_SLEEP);
+            continue;
+        }
+        const uint32_t l = (uint32_t)__builtin_ctzll(missing);
+        const uint32_t j = (uint32_t)(top - (int64_t)l);
+        const uint32_t own = help_tile_u32<TILE>(p, j);
+        wait_performed();
+        const uint64_t again = atomic_load_agent(p.status + kSlotWords * (uint64_t)j);
+        const uint32_t sum = status_flag(again, epoch) != 0u ? (uint32_t)again : own;
+        value = lane == l ? sum : value;
+        helped = helped || lane == l;
+    }
+}
+
+template <int BLOCK, int VEC, bool INCL>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(GPS_WAVES_PER_EU))) void csdl_round_u32(
+    ScanParams p) {
+    using C = TileCfg<BLOCK, VEC>;
+    __shared__ uint32_t s_wave[C::kWaves], s_before[C::kWaves];
+    __shared__ uint32_t s_epoch;
+    const uint32_t tile = blockIdx.x, wave = wave_index(), lane = lane_id();
+    uint64_t entered = 0;
+    if (threadIdx.x == 0) entered = round_enter(p.ticket, p.num_tiles);
+    u32x4 d[VEC];
+    load_tile<VEC>(d, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
+    const uint32_t run = wave_scan_run<VEC, INCL>(d);
+    if (lane == 0) s_wave[wave] = run;
+    if (threadIdx.x == 0) s_epoch = round_epoch(p.ticket, entered, p.num_tiles);
+    __syncthreads();
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
+    uint32_t wave_prefix, tile_total;
+    combine_waves<C::kWaves>(s_wave, wave, wave_prefix, tile_total);
+    const uint32_t carry = tile == 0 && p.carry_in ? *p.carry_in : 0u;
+    if (threadIdx.x == 0)
+        atomic_store_agent(p.status + kSlotWords * tile, make_status(carry + tile_total, kFlagAgg, epoch));
+    uint32_t before = 0;
+    for (int64_t top = (int64_t)tile - 1 - 64 * (int64_t)wave; top >= 0; top -= 64 * (int64_t)C::kWaves)
+        before += round_window_u32<C::kTile>(p, top, epoch);
+    if (lane == 0) s_before[wave] = before;
+    if (wave == 0) wait_performed();  // the word above, before any wave's output stores
+    if (threadIdx.x == BLOCK - kWave) round_leave(p.ticket, p.status, tile, p.num_tiles);
+    __syncthreads();
+    uint32_t unused, prefix;
+    combine_waves<C::kWaves>(s_before, wave, unused, prefix);
+    prefix += carry;
+    if (p.carry_out && tile == p.num_tiles - 1 && threadIdx.x == 0) *p.carry_out = prefix + tile_total;
+    store_tile<VEC>(p.out, d, prefix + wave_prefix, (uint64_t)tile * C::kTile, p.n, C::kTile);
+}
+
+// A scan of one tile: no ticket and no status word.
+template <int BLOCK, int VEC, bool INCL>
+__global__ __launch_bounds__(BLOCK) void scan_single_u32(const uint32_t* in, uint32_t* out, uint32_t n,
+                                                         const uint32_t* carry_in, uint32_t* carry_out) {
+    using C = TileCfg<BLOCK, VEC>;
+    __shared__ uint32_t s_wave[C::kWaves];
+    const uint32_t wave = wave_index();
+    u32x4 d[VEC];
+    load_tile<VEC>(d, in, 0, n, C::kTile);
+    const uint32_t carry = carry_in ? *carry_in : 0u;
+    const uint32_t run = wave_scan_run<VEC, INCL>(d);
+    uint32_t wave_prefix = 0, total = run;
+    if (C::kWaves > 1) {
+        if (lane_id() == 0) s_wave[wave] = run;
+        __syncthreads();
+        combine_waves<C::kWaves>(s_wave, wave, wave_prefix, total);
+    }
+    store_tile<VEC>(out, d, carry + wave_prefix, 0, n, C::kTile);
+    if (carry_out && threadIdx.x == 0) *carry_out = carry + total;
+}
+
+// ---------------------------------------------------------------------------
 // Persistent, software-pipelined CSDL (the MI355X default schedule).
 //
 // A chained scan's workgroup must wait for its tile's exclusive prefix before
@@ -1067,9 +1170,36 @@ bool shape_supported(TileShape s) {
     return false;
 }
 
+template <int B, int V>
+static hipError_t launch_single(bool inclusive, const ScanParams& p, hipStream_t stream) {
+    if (inclusive)
+        hipLaunchKernelGGL((scan_single_u32<B, V, true>), dim3(1), dim3(B), 0, stream, p.in, p.out, (uint32_t)p.n,
+                           p.carry_in, p.carry_out);
+    else
+        hipLaunchKernelGGL((scan_single_u32<B, V, false>), dim3(1), dim3(B), 0, stream, p.in, p.out, (uint32_t)p.n,
+                           p.carry_in, p.carry_out);
+    return hipGetLastError();
+}
+
 hipError_t launch_csdl_u32(TileShape s, bool inclusive, const ScanParams& p, hipStream_t stream) {
+    // One workgroup up to 16384 elements: 2.6 us there against 3.4 for two
+    // tiles of 8192 (2^15: 3.5 against 3.4 for four); 1021 elements 1.9 us,
+    // 2.9 with a ticket and a status word.
+    if (p.num_tiles == 1 || (s.block == 1024 && p.n <= 16384)) {
+#define S(B, V) \
+    if (p.n <= TileCfg<B, V>::kTile) return launch_single<B, V>(inclusive, p, stream);
+        S(64, 2) S(256, 2) S(512, 2) S(1024, 2) S(1024, 4) S(1024, 8)
+#undef S
+    }
 #define X(B, V)                                                                          \
     if (s.block == B && s.vec == V) {                                                    \
+        if (p.num_tiles <= kRoundTiles) {                                                \
+            if (inclusive)                                                               \
+                hipLaunchKernelGGL((csdl_round_u32<B, V, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);  \
+            else                                                                         \
+                hipLaunchKernelGGL((csdl_round_u32<B, V, false>), dim3(p.num_tiles), dim3(B), 0, stream, p); \
+            return hipGetLastError();                                                    \
+        }                                                                                \
         if (inclusive)                                                                   \
             hipLaunchKernelGGL((csdl_u32<B, V, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);  \
         else                                                                             \

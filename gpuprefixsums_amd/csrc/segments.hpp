@@ -66,6 +66,72 @@ __device__ __forceinline__ void mark_heads_by(uint32_t* s_heads, const uint64_t*
     }
 }
 
+// Marks the heads of the tile [a, b) with the whole workgroup, finding them as
+// it goes: up to 4 * BLOCK offsets are simply all read (one load latency);
+// beyond, each round samples BLOCK evenly spaced ones and keeps the bracket
+// around a, and the marking starts at its low end, past which only offsets
+// below a are passed over. Against one wave's 64-ary search before the marking
+// this saves two dependent loads at 16384 segments. s_heads zeroed and visible;
+// a barrier must follow. s_bracket: BLOCK / 64 words.
+template <int BLOCK>
+__device__ __forceinline__ void find_and_mark_heads(uint32_t* s_heads, uint32_t* s_bracket, const uint64_t* offsets,
+                                                    uint64_t S, uint64_t a, uint64_t b, bool first_tile) {
+    constexpr uint32_t kWaves = BLOCK / kWave;
+    const uint32_t lane = lane_id(), wave = wave_index();
+    uint64_t lo = 0, hi = S;  // the first offset >= a has an index in [lo, hi]
+    while (hi - lo > 4u * BLOCK) {
+        const uint64_t step = (hi - lo + BLOCK - 1) / BLOCK;
+        const uint64_t pos = lo + (uint64_t)(threadIdx.x + 1u) * step - 1u;
+        const uint64_t hit = ballot(offsets[pos < hi ? pos : hi - 1u] >= a);
+        if (lane == 0) s_bracket[wave] = hit ? wave * kWave + (uint32_t)__builtin_ctzll(hit) : BLOCK;
+        __syncthreads();
+        uint32_t f = BLOCK;  // first sample at or past a
+        for (uint32_t w = 0; w < kWaves; ++w) f = s_bracket[w] < f ? s_bracket[w] : f;
+        f = (uint32_t)__builtin_amdgcn_readfirstlane(f);
+        __syncthreads();
+        const uint64_t low = lo + (uint64_t)f * step;  // past sample f - 1
+        if (f == BLOCK || low >= hi) {
+            lo = hi;
+            break;
+        }
+        const uint64_t high = lo + (uint64_t)(f + 1u) * step - 1u;
+        hi = high < hi ? high : hi;
+        lo = low;
+    }
+    if (first_tile && threadIdx.x == 0) atomicOr(&s_heads[0], 1u);
+    for (uint64_t s = lo + threadIdx.x; s < S; s += 4ull * BLOCK) {
+        uint64_t o[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint64_t su = s + (uint64_t)u * BLOCK;
+            o[u] = su < S ? offsets[su] : b;
+        }
+        bool past = false;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (o[u] >= a && o[u] < b) {
+                const uint32_t rel = (uint32_t)(o[u] - a);
+                atomicOr(&s_heads[rel >> 5], 1u << (rel & 31u));
+            }
+            past = past || o[u] >= b;
+        }
+        if (past) break;
+    }
+}
+
+// Start of the part of tile [a, b) that its carry-out sums (its last segment
+// head, else a) and whether it holds a head; one wave.
+struct TailOfTile {
+    uint64_t from;
+    bool has_head;
+};
+__device__ __forceinline__ TailOfTile find_tail(const uint64_t* offsets, uint64_t S, uint64_t a, uint64_t b) {
+    const uint64_t s = find_first_segment(offsets, S, b);
+    const uint64_t last = s ? offsets[s - 1u] : 0u;
+    const bool in_tile = s != 0u && last >= a;
+    return {in_tile ? last : a, in_tile || a == 0u};
+}
+
 // mark_heads_by with the whole workgroup.
 template <int BLOCK>
 __device__ __forceinline__ void mark_heads(uint32_t* s_heads, const uint64_t* offsets, uint64_t S, uint64_t s0,

@@ -106,14 +106,16 @@ def candidates(dtype: str, stall_period: int = 0) -> List[Config]:
 
 def default_config(dtype: str, segments: int, n: int = 1 << 30, stall_period: int = 0) -> Config:
     """What the library does without the tuner: a default handle's choice for
-    n elements (the same rules as libgps's size-adaptive defaults). Under
+    n elements (the same rules as libgps's size-adaptive defaults, but for two
+    things: FP scans run persistent from 2^23 elements on, and the segmented FP
+    kernel has 512 x 4 tiles, no candidate, between 2^20 and 9 * 2^18). Under
     emulated deadlock it is the default decoupled-fallback handle (1024 x 8,
     spin limit 4)."""
     if stall_period:
         return Config("loop_csdldf", 1024, 8, 4)
     if dtype != "u32":
         if segments == 1:
-            b, v = (256, 4) if n <= 1 << 18 else (1024, 4) if n <= 1 << 22 else (1024, 8)
+            b, v = (256, 4) if n <= 1 << 19 else (1024, 4) if n <= 1 << 22 else (1024, 8)
             return Config("loop_fp", b, v, persistent=n > 1 << 24)
         if n > 1 << 22:
             return Config("batched_fp", 1024, 8, persistent=True)

@@ -53,7 +53,9 @@ typedef struct gps_tuning {
     uint32_t vec_per_thread; /* uint4 vectors per thread: 2, 4 or 8 (items = 4x) */
     uint32_t spin_limit;     /* CSDLDF: polls without progress before a fallback (default 4), for the
                                 blocking tile's nearest successor; a waiter k tiles farther waits
-                                (1 + min(k, 7)) x spin_limit polls; at most 65536 */
+                                (1 + min(k, 7)) x spin_limit polls; at most 65536. CSDL, one workgroup
+                                per tile, up to 1024 tiles: polls before a workgroup sums a tile that
+                                it waits for by itself (default 64) */
     uint32_t stall_period;   /* CSDLDF: stall tiles with index % period == 0 (0 = no emulation, >= 2);
                                 with GPS_SCHEDULE_SPLIT, defer them to a second launch instead */
     uint32_t schedule;       /* CSDL, CSDLDF: GPS_SCHEDULE_* (0 = default) */
@@ -216,7 +218,7 @@ int gps_survey_scan_u32(int alg, const uint32_t* d_in, uint32_t* d_out, uint64_t
  *                     rounded once.
  * Other values return GPS_ERR_INVALID. No FP64 arithmetic is used. One
  * kernel launch; needs a GPS_ALGO_CSDL handle. Runs the persistent kernel on
- * a handle with the persistent schedule (a default handle: above 2^24
+ * a handle with the persistent schedule (a default handle: above 2^23
  * elements), else one workgroup per tile. */
 #define GPS_FP_PLAIN 0
 #define GPS_FP_PAIR 1
