@@ -41,6 +41,21 @@ def _ptr(x) -> int:
     raise TypeError(f"expected a device pointer or tensor, got {type(x)!r}")
 
 
+_raw_stream = None  # torch's current stream of a device index, as an address
+
+
+def _current_stream(b) -> int:
+    """torch's current stream of a device tensor. The raw query takes 0.1 us,
+    torch.cuda.current_stream 1.9 us of the 7 us that a small scan's call took."""
+    global _raw_stream
+    import torch
+    if _raw_stream is None:
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", False)
+    if _raw_stream and isinstance(b, torch.Tensor):
+        return _raw_stream(b.get_device())
+    return int(torch.cuda.current_stream(b.device).cuda_stream)
+
+
 def _stream(s, *bufs) -> Optional[int]:
     """The stream to launch on: `s` if given, else torch's current stream of
     the first device tensor among `bufs` (so tensor callers get stream-ordered
@@ -48,8 +63,7 @@ def _stream(s, *bufs) -> Optional[int]:
     if s is None:
         for b in bufs:
             if getattr(b, "is_cuda", False):
-                import torch
-                return int(torch.cuda.current_stream(b.device).cuda_stream)
+                return _current_stream(b)
         return None
     if isinstance(s, int):
         return s
@@ -70,10 +84,13 @@ def _need(what: str, nbytes: int, *bufs) -> None:
     explicit n can never make a kernel run past a buffer. Raw addresses are
     the caller's responsibility."""
     for b in bufs:
-        if b is not None and hasattr(b, "numel") and hasattr(b, "element_size"):
-            have = int(b.numel()) * int(b.element_size())
-            if have < nbytes:
-                raise ValueError(f"{what}: a buffer holds {have} bytes but the call needs {nbytes}")
+        try:
+            numel, size = b.numel, b.element_size
+        except AttributeError:
+            continue
+        have = int(numel()) * int(size())
+        if have < nbytes:
+            raise ValueError(f"{what}: a buffer holds {have} bytes but the call needs {nbytes}")
 
 
 class ScanHandle:

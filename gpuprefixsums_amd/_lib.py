@@ -105,6 +105,8 @@ SIGNATURES = {
 }
 
 _lib = None
+# Handles that libgps_torch.so may launch on: open until the process ends.
+kept_open: list = []
 
 
 def load() -> ctypes.CDLL:

@@ -5,7 +5,8 @@ gpuprefixsums_amd/libgps.so (the product library), the vendor comparator
 gpuprefixsums_amd/libgps_vendor.so (rocPRIM's scan, for tests and benchmarks
 only; it links libgps.so), the memory-ceiling probes
 gpuprefixsums_amd/libgps_ceiling.so (benchmark only; it links libgps.so), the
-reference-style test program gpuprefixsums_amd/gps_main, and the oracle (oracle/liboracle.so, test
+PyTorch operators' device kernels gpuprefixsums_amd/libgps_torch.so (they link
+libgps.so and the installed PyTorch), the reference-style test program gpuprefixsums_amd/gps_main, and the oracle (oracle/liboracle.so, test
 infrastructure) with make.
 
     python -m gpuprefixsums_amd.build          # build everything
@@ -27,6 +28,7 @@ BUILD = PKG / "_build"
 LIB = PKG / "libgps.so"
 VENDOR_LIB = PKG / "libgps_vendor.so"
 CEILING_LIB = PKG / "libgps_ceiling.so"
+TORCH_LIB = PKG / "libgps_torch.so"
 MAIN = PKG / "gps_main"
 ARCH = "gfx950"
 
@@ -56,6 +58,9 @@ VENDOR_SOURCES = [
 CEILING_SOURCES = [
     "ceiling.hip",
 ]
+
+# The PyTorch operators' device kernels (host code against PyTorch's headers).
+TORCH_SOURCE = "torch_ops.cpp"
 
 COMMON_FLAGS = [
     f"--offload-arch={ARCH}",
@@ -117,6 +122,21 @@ def build_lib(jobs: int = 8) -> Path:
     return LIB
 
 
+def build_torch() -> Path:
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    obj = BUILD / (TORCH_SOURCE + ".o")
+    cmd = [hipcc(), "-O2", "-std=c++17", "-fPIC", "-Wall", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+           *(f"-isystem{p}" for p in include_paths()), "-c", str(CSRC / TORCH_SOURCE), "-o", str(obj)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"hipcc failed for {TORCH_SOURCE}:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    libs = Path(torch.__file__).parent / "lib"
+    return _link([obj], TORCH_LIB, [f"-L{PKG}", "-lgps", "-Wl,-rpath,$ORIGIN", f"-L{libs}", "-ltorch", "-ltorch_cpu",
+                                    "-lc10", "-lc10_hip"])
+
+
 def build_main() -> Path:
     src = CSRC / "gps_main.cpp"
     if not src.exists():
@@ -138,6 +158,7 @@ def build_oracle() -> Path:
 
 def build_all() -> None:
     build_lib()
+    build_torch()
     build_main()
     build_oracle()
 

@@ -18,15 +18,20 @@ of the needed size exists for the (device, stream) pair, so they can be
 captured after one eager call at that size on the capturing stream; a call
 that would need a new or larger handle during capture raises. Replaced
 handles are kept open, so earlier captures stay valid.
+
+An ordinary call on the device (contiguous, on the current device, no gradient
+asked for, the stream's handle in place) runs in csrc/torch_ops.cpp, which
+falls back to the implementations here for all others.
 """
 from __future__ import annotations
 
+import ctypes
 import threading
 from typing import Dict, List, Tuple
 
 import torch
 
-from . import ALGO_CSDL, ScanHandle
+from . import ALGO_CSDL, ScanHandle, _lib
 
 _INT = (torch.int32, torch.uint32)
 _FLOAT = (torch.float32, torch.bfloat16)
@@ -36,6 +41,17 @@ _handles: Dict[Tuple[int, int], ScanHandle] = {}
 # their status and ticket addresses and may be replayed at any time.
 _retired: List[ScanHandle] = []
 _lock = threading.Lock()
+
+
+def _load_kernels() -> ctypes.CDLL:
+    """Loads libgps_torch.so, which registers the operators' device kernels."""
+    path = _lib.LIB_PATH.with_name("libgps_torch.so")
+    if not path.exists():
+        raise ImportError(f"{path} is not built; run `python -m gpuprefixsums_amd.build`")
+    lib = ctypes.CDLL(str(path))
+    lib.gps_torch_set_handle.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint64]
+    lib.gps_torch_set_handle.restype = None
+    return lib
 
 
 def _handle(x: torch.Tensor, n: int) -> ScanHandle:
@@ -59,6 +75,8 @@ def _handle(x: torch.Tensor, n: int) -> ScanHandle:
             with torch.cuda.device(x.device):
                 h = ScanHandle(ALGO_CSDL, max(n, 1 << 20))
             _handles[key] = h
+            _lib.kept_open.append(h)
+            _kernels.gps_torch_set_handle(*key, h.handle, h.max_n)
         return h
 
 
@@ -136,5 +154,7 @@ def segmented_cumsum(x: torch.Tensor, offsets: torch.Tensor, inclusive: bool = T
 def _(x, offsets, inclusive=True, compensated=True):
     return torch.empty_like(x) if x.dtype in _INT else x.new_empty(x.shape, dtype=torch.float32)
 
+
+_kernels = _load_kernels()
 
 __all__ = ["cumsum", "segmented_cumsum"]
