@@ -33,16 +33,17 @@ gps::TileShape seg_shape(const gps_handle* h, uint64_t n) {
 // launches on MI355X): one FP scan uses 256 x 4 up to 2^19 elements (2^18 + 1
 // pairs: 5.2 against 5.9 us for 1024 x 4; 2^20: 7.7 against 6.8), 1024 x 4 up
 // to 2^22 and 1024 x 8 above. The segmented FP kernel uses 256 x 4 below 2^20,
-// 512 x 4 up to 9 * 2^18 and 1024 x 4 above: its runs are walked through LDS
-// twice, and until the chip is full smaller workgroups start and end that
+// for pairs 512 x 4 up to 9 * 2^18, and 1024 x 4 above: the pair kernel's runs
+// are walked through LDS twice, and until the chip is full smaller workgroups start and end that
 // earlier (FP32 pairs, 100 / 100000 segments: 700,000 elements 6.4 / 7.6 us at
 // 256 x 4, 6.7 / 7.8 at 512 x 4; 2,000,000 7.6 / 8.6 at 512 x 4, 8.8 / 10.1 at
 // 1024 x 4; 2,500,000 9.0 / 10.2 at 512 x 4, 8.6 / 10.4 at 1024 x 4).
-gps::TileShape fp_shape(const gps_handle* h, uint64_t n, bool segmented) {
+gps::TileShape fp_shape(const gps_handle* h, uint64_t n, bool segmented, int compensated) {
     if (h->size_adaptive) {
         if (segmented)
-            return n < (1ull << 20) ? gps::TileShape{256, 4} : n <= (9ull << 18) ? gps::kSegFpMid
-                                                                                 : gps::TileShape{1024, 4};
+            return n < (1ull << 20) ? gps::TileShape{256, 4}
+                   : n <= (9ull << 18) && compensated == gps::kFpPair ? gps::kSegFpMid
+                                                                      : gps::TileShape{1024, 4};
         return n <= (1ull << 19) ? gps::TileShape{256, 4} : n <= (1ull << 22) ? gps::TileShape{1024, 4}
                                                                                : gps::TileShape{1024, 8};
     }
@@ -102,7 +103,7 @@ int scan_fp(gps_handle* h, const void* in, float* out, uint64_t n, bool bf16, in
     const uintptr_t ia = reinterpret_cast<uintptr_t>(in), oa = reinterpret_cast<uintptr_t>(out);
     if ((ia & (bf16 ? 1u : 3u)) || (oa & 3u)) return fail(GPS_ERR_INVALID, "misaligned buffer");
     if (n == 0) return GPS_OK;
-    const gps::TileShape s = fp_shape(h, n, false);
+    const gps::TileShape s = fp_shape(h, n, false, compensated);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
     HIP_TRY(gps::launch_scan_fp(s, bf16, compensated, fp_persistent(h, n), h->round_patience, in, out, n,
@@ -137,7 +138,7 @@ int segscan_fp(gps_handle* h, const void* in, float* out, const uint64_t* offset
         return fail(GPS_ERR_INVALID, "compensated must be 0 (plain) or 1 (two-float pairs)");
     if (n == 0) return GPS_OK;
     const bool persistent = segfp_persistent(h, n);
-    const gps::TileShape s = persistent && h->size_adaptive ? gps::TileShape{1024, 8} : fp_shape(h, n, true);
+    const gps::TileShape s = persistent && h->size_adaptive ? gps::TileShape{1024, 8} : fp_shape(h, n, true, compensated);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
     HIP_TRY(gps::launch_segscan_fp(s, bf16, compensated != 0, persistent, h->round_patience, in, out, offsets,

@@ -161,8 +161,8 @@ hipError_t launch_scan_fp(TileShape s, bool bf16, int carry, bool persistent, ui
                           float* out, uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
                           hipStream_t stream);
 // Batched segmented FP inclusive scan (one launch; same shapes as launch_scan_fp;
-// persistent as there), and one workgroup per tile of shape kSegFpMid for 2 to
-// 513 tiles.
+// persistent as there), and, with pair carries, one workgroup per tile of shape
+// kSegFpMid for 2 to 513 tiles.
 constexpr TileShape kSegFpMid{512, 4};
 hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, uint32_t patience,
                              const void* in, float* out, const uint64_t* offsets, uint64_t num_segments, uint64_t n,

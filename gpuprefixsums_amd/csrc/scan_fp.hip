@@ -1337,14 +1337,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
 // One-round segmented FP scan (device_common.hpp): one workgroup per tile
 // while a workgroup's waves cover the tiles before it in one window each; a
 // single tile takes no ticket and publishes nothing. Lane-blocked runs as
-// segscan_fp_bl. The search for the tile's heads starts with its loads.
+// segscan_fp_bl. The search for the tile's heads starts with its loads. Pair
+// carries only: over runs of 16 elements plain FP32 sums are 1.3 times as far
+// from the exact ones (relative 1.16e-7 against 8.7e-8, normal floats in
+// segments of 128) as over segscan_fp's striped vectors.
 // Back to back, FP32 pairs, against segscan_fp (tickets, window lookback,
 // striped): 1000 elements 3.5 us (5.6), 2^16 in 1000 segments 5.7 (6.4), 2^20
 // in 16384 segments 8.2 (11.1), 2^21 + 17 in 16384 segments 8.9 (12.0).
 // ---------------------------------------------------------------------------
 // The carry that the tiles top, top - 1, ... (at most 64; one wave) pass on:
 // the sum back to the nearest tile that holds a head; `closed` if there is one.
-template <uint32_t TILE, bool BF16, bool COMP>
+template <uint32_t TILE, bool BF16>
 __device__ __forceinline__ ff round_window_seg_ff(const SegFpParams& p, int64_t top, uint32_t epoch, bool& closed) {
     const uint32_t lane = lane_id();
     const int64_t idx = top - (int64_t)lane;
@@ -1367,8 +1370,8 @@ __device__ __forceinline__ ff round_window_seg_ff(const SegFpParams& p, int64_t 
         closed = first_incl < run;
         if (closed || run == 64u) {
             const uint32_t take = closed ? first_incl + 1u : 64u;
-            const ff s = wave_incl_scan_ff<COMP>(lane < take ? value : ff{0.f, 0.f});
-            return {readlane_f(s.s, 63), COMP ? readlane_f(s.c, 63) : 0.f};
+            const ff s = wave_incl_scan_ff<true>(lane < take ? value : ff{0.f, 0.f});
+            return {readlane_f(s.s, 63), readlane_f(s.c, 63)};
         }
         if (++polls < p.patience) {
             __builtin_amdgcn_s_sleep(1);
@@ -1377,7 +1380,7 @@ __device__ __forceinline__ ff round_window_seg_ff(const SegFpParams& p, int64_t 
         const uint32_t j = (uint32_t)(top - (int64_t)run);
         const uint64_t end = (uint64_t)(j + 1u) * TILE;
         const TailOfTile tail = find_tail(p.offsets, p.num_segments, end - TILE, end);
-        ff sum = help_sum_ff<BF16, COMP>(p.in, tail.from, end);
+        ff sum = help_sum_ff<BF16, true>(p.in, tail.from, end);
         uint32_t f = tail.has_head ? (uint32_t)kFlagIncl : (uint32_t)kFlagAgg;
         wait_performed();
         load_pair_words(p.status + kSlotWords * (uint64_t)j, ws, wc);
@@ -1394,10 +1397,10 @@ __device__ __forceinline__ ff round_window_seg_ff(const SegFpParams& p, int64_t 
     }
 }
 
-template <int BLOCK, int VEC, bool BF16, bool COMP, bool SINGLE>
+template <int BLOCK, int VEC, bool BF16, bool SINGLE>
 __global__ __launch_bounds__(BLOCK) void segscan_fp_round(SegFpParams p) {
     using C = TileCfg<BLOCK, VEC>;
-    using Ops = PairCarry<COMP>;
+    using Ops = PairCarry<true>;
     constexpr uint32_t kWords = C::kTile / 32;
     __shared__ __align__(16) float s_slices[C::kWaves * BlockedSlice<VEC>::kFloats];
     __shared__ uint32_t s_heads[kWords], s_bracket[C::kWaves];
@@ -1428,12 +1431,12 @@ __global__ __launch_bounds__(BLOCK) void segscan_fp_round(SegFpParams p) {
     }
     uint32_t sf = heads != 0u;
     ff sv = t;
-    wave_seg_scan_ff<COMP>(sf, sv);
+    wave_seg_scan_ff<true>(sf, sv);
     const uint32_t ef = GPS_DPP_I(sf, 0x138, 0xf, true);  // wave_shr:1, lane 0 gets 0
     const ff ev = Ops::shr1(sv);
     if (lane == 0) {
         s_ws[wave] = readlane_f(sv.s, 63);
-        s_wc[wave] = COMP ? readlane_f(sv.c, 63) : 0.f;
+        s_wc[wave] = readlane_f(sv.c, 63);
         s_wf[wave] = readlane(sf, 63);
     }
     if (!SINGLE && threadIdx.x == 0) s_epoch = round_epoch(p.ticket, entered, p.num_tiles);
@@ -1444,7 +1447,7 @@ __global__ __launch_bounds__(BLOCK) void segscan_fp_round(SegFpParams p) {
     {
         uint32_t f = lane < C::kWaves ? s_wf[q] : 0u;
         ff v = {lane < C::kWaves ? s_ws[q] : 0.f, lane < C::kWaves ? s_wc[q] : 0.f};
-        wave_seg_scan_ff<COMP>(f, v);
+        wave_seg_scan_ff<true>(f, v);
         const uint32_t wef = GPS_DPP_I(f, 0x138, 0xf, true);
         pre_f = readlane(wef, (int)wave);
         pre = Ops::lane(Ops::shr1(v), (int)wave);
@@ -1455,13 +1458,13 @@ __global__ __launch_bounds__(BLOCK) void segscan_fp_round(SegFpParams p) {
     if (!SINGLE) {
         const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
         if (threadIdx.x == 0)
-            publish_ff<COMP>(p.status, tile, tile_tot, (tile_f || tile == 0) ? kFlagIncl : kFlagAgg, epoch);
+            publish_ff<true>(p.status, tile, tile_tot, (tile_f || tile == 0) ? kFlagIncl : kFlagAgg, epoch);
         // A tile that starts with a head takes nothing from the ones before.
         ff before = {0.f, 0.f};
         bool closed = true;
         const int64_t top = (int64_t)tile - 1 - 64 * (int64_t)wave;
         if (top >= 0 && (s_heads[0] & 1u) == 0u)
-            before = round_window_seg_ff<C::kTile, BF16, COMP>(p, top, epoch, closed);
+            before = round_window_seg_ff<C::kTile, BF16>(p, top, epoch, closed);
         if (lane == 0) {
             s_bs[wave] = before.s;
             s_bc[wave] = before.c;
@@ -1474,11 +1477,11 @@ __global__ __launch_bounds__(BLOCK) void segscan_fp_round(SegFpParams p) {
         const uint64_t stop = ballot(lane < C::kWaves && s_closed[q] != 0u);
         const uint32_t take = stop ? (uint32_t)__builtin_ctzll(stop) + 1u : C::kWaves;
         const ff v = {lane < take ? s_bs[q] : 0.f, lane < take ? s_bc[q] : 0.f};
-        const ff sum = row_incl_scan_ff<COMP>(v);
-        prefix = {readlane_f(sum.s, C::kWaves - 1), COMP ? readlane_f(sum.c, C::kWaves - 1) : 0.f};
+        const ff sum = row_incl_scan_ff<true>(v);
+        prefix = {readlane_f(sum.s, C::kWaves - 1), readlane_f(sum.c, C::kWaves - 1)};
     }
-    const ff run_in = pre_f ? pre : ff_add<COMP>(prefix, pre);
-    ff acc = ef ? ev : ff_add<COMP>(run_in, ev);
+    const ff run_in = pre_f ? pre : ff_add<true>(prefix, pre);
+    ff acc = ef ? ev : ff_add<true>(run_in, ev);
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
         f32x4 o;
@@ -1598,19 +1601,12 @@ static hipError_t launch_segfp_pp(const SegFpParams& p, hipStream_t stream) {
 // One workgroup per tile.
 template <int B, int V, bool BF16, bool COMP>
 static void launch_segfp_tile(const SegFpParams& p, hipStream_t stream) {
-    if (p.num_tiles == 1)
-        hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, COMP, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (p.num_tiles <= (uint32_t)B + 1u)  // B / 64 waves x 64 tiles
-        hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, COMP, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+    if (COMP && p.num_tiles == 1)
+        hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, true>), dim3(1), dim3(B), 0, stream, p);
+    else if (COMP && p.num_tiles <= (uint32_t)B + 1u)  // B / 64 waves x 64 tiles
+        hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((segscan_fp<B, V, BF16, COMP>), dim3(p.num_tiles), dim3(B), 0, stream, p);
-}
-
-// kSegFpMid: 2 to 513 tiles.
-template <bool BF16, bool COMP>
-static void launch_segfp_round(const SegFpParams& p, hipStream_t stream) {
-    hipLaunchKernelGGL((segscan_fp_round<kSegFpMid.block, kSegFpMid.vec, BF16, COMP, false>), dim3(p.num_tiles),
-                       dim3(kSegFpMid.block), 0, stream, p);
 }
 
 hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool persistent, uint32_t patience,
@@ -1628,15 +1624,12 @@ hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool pers
     p.patience = patience;
     p.err = err;
     if (s.block == kSegFpMid.block && s.vec == kSegFpMid.vec) {
-        if (persistent || p.num_tiles < 2 || p.num_tiles > (uint32_t)kSegFpMid.block + 1u) return hipErrorInvalidValue;
-        if (bf16 && compensated)
-            launch_segfp_round<true, true>(p, stream);
-        else if (bf16)
-            launch_segfp_round<true, false>(p, stream);
-        else if (compensated)
-            launch_segfp_round<false, true>(p, stream);
+        constexpr uint32_t kB = kSegFpMid.block;
+        if (persistent || !compensated || p.num_tiles < 2 || p.num_tiles > kB + 1u) return hipErrorInvalidValue;
+        if (bf16)
+            hipLaunchKernelGGL((segscan_fp_round<kB, kSegFpMid.vec, true, false>), dim3(p.num_tiles), dim3(kB), 0, stream, p);
         else
-            launch_segfp_round<false, false>(p, stream);
+            hipLaunchKernelGGL((segscan_fp_round<kB, kSegFpMid.vec, false, false>), dim3(p.num_tiles), dim3(kB), 0, stream, p);
         return hipGetLastError();
     }
 #define X(B, V)                                                                                                  \
