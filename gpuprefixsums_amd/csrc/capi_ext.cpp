@@ -80,13 +80,14 @@ namespace {
 
 // One FP scan with pair or plain carries runs the persistent kernel on a
 // handle with the persistent schedule (the CSDL default). A default handle
-// picks it above 2^23 elements, against one workgroup per tile, both at
-// 1024 x 8: FP32 pairs 2^23 15.4 against 13.0 us, 9,000,000 16.6 against
-// 20.3; BF16 pairs 14.1 against 12.8 and 14.8 against 19.7; FP32 plain 14.3
-// against 11.7 and 15.0 against 16.7. (Between 5 and 7 million FP32 pairs it
-// is up to 8% faster, BF16 pairs slower, plain carries either.)
-bool fp_persistent(const gps_handle* h, uint64_t n) {
-    if (h->size_adaptive) return n > (1ull << 23);
+// picks it for pairs above 2^23 elements, against one workgroup per tile, both
+// at 1024 x 8: FP32 2^23 15.4 against 13.0 us, 9,000,000 16.6 against 20.3;
+// BF16 14.1 against 12.8 and 14.8 against 19.7. (Between 5 and 7 million FP32
+// it is up to 8% faster, BF16 slower.) For plain carries above 2^24: at
+// 10,000,000 it is 6% faster, but one workgroup per tile adds the aggregates
+// before a tile in fewer roundings (relative error 2.3e-7 against 2.5e-7).
+bool fp_persistent(const gps_handle* h, uint64_t n, int compensated) {
+    if (h->size_adaptive) return n > (compensated == gps::kFpPair ? 1ull << 23 : 1ull << 24);
     return h->schedule == GPS_SCHEDULE_PERSISTENT;
 }
 
@@ -106,7 +107,7 @@ int scan_fp(gps_handle* h, const void* in, float* out, uint64_t n, bool bf16, in
     const gps::TileShape s = fp_shape(h, n, false, compensated);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
-    HIP_TRY(gps::launch_scan_fp(s, bf16, compensated, fp_persistent(h, n), h->round_patience, in, out, n,
+    HIP_TRY(gps::launch_scan_fp(s, bf16, compensated, fp_persistent(h, n, compensated), h->round_patience, in, out, n,
                                 h->status, h->ticket, h->err, st));
     return GPS_OK;
 }
@@ -161,9 +162,10 @@ int scan_u32x4(gps_handle* h, const uint32_t* in, uint32_t* out, uint64_t n, boo
     bool persistent = h->schedule != GPS_SCHEDULE_TILE;
     if (h->size_adaptive) {
         // As for the plain scan, measured on MI355X: one workgroup per tile
-        // below 2^22 structs, 1024 x 4 up to 2^19 (2^16 structs: 5.4 against
-        // 6.7 us for the persistent 1024 x 8 kernel).
-        if (n <= (1ull << 19)) {
+        // below 2^22 structs (3,000,000: 21.4 against 21.3 us for the persistent
+        // kernel, 2,000,000 12.4 against 14.8), 1024 x 4 up to 2^20 (1,000,003:
+        // 8.5 against 9.3 us for 1024 x 8; 2,000,000 15.9 against 12.4).
+        if (n <= (1ull << 20)) {
             s = {1024, 4};
             persistent = false;
         } else if (n < (1ull << 22)) {
@@ -175,7 +177,8 @@ int scan_u32x4(gps_handle* h, const uint32_t* in, uint32_t* out, uint64_t n, boo
     if ((n + tile - 1) / tile > h->max_tiles) return fail(GPS_ERR_TOO_LARGE, "not enough status slots");
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(gps::before_epoch_launch(h, st));
-    HIP_TRY(gps::launch_csdl_u32x4(s, inclusive, persistent, in, out, n, h->status, h->ticket, h->err, st));
+    HIP_TRY(gps::launch_csdl_u32x4(s, inclusive, persistent, h->round_patience, in, out, n, h->status, h->ticket,
+                                   h->err, st));
     return GPS_OK;
 }
 
@@ -315,7 +318,8 @@ int gps_estimate_occupancy(gps_handle* h, const uint32_t* d_in, uint32_t* d_out,
     if (struct_scan) {
         const gps::TileShape s = gps::v4_shape_supported(h->shape) ? h->shape : gps::TileShape{1024, 8};
         *resident = gps::v4_resident_workgroups(s, true);
-        HIP_TRY(gps::launch_csdl_u32x4(s, true, true, d_in, d_out, n, h->status, h->ticket, h->err, st, count, true));
+        HIP_TRY(gps::launch_csdl_u32x4(s, true, true, h->round_patience, d_in, d_out, n, h->status, h->ticket, h->err,
+                                       st, count, true));
     } else {
         gps::ScanParams p{};
         const uint64_t tile = h->shape.tile();

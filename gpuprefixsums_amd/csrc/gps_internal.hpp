@@ -172,9 +172,9 @@ hipError_t launch_segscan_fp(TileShape s, bool bf16, bool compensated, bool pers
 bool v4_shape_supported(TileShape s);
 // persistent: resident workgroups with the pipelined ticket loop; otherwise
 // one workgroup per tile.
-hipError_t launch_csdl_u32x4(TileShape s, bool inclusive, bool persistent, const uint32_t* in, uint32_t* out,
-                             uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream,
-                             unsigned long long* occupancy = nullptr, bool grid_all_tiles = false);
+hipError_t launch_csdl_u32x4(TileShape s, bool inclusive, bool persistent, uint32_t patience, const uint32_t* in,
+                             uint32_t* out, uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
+                             hipStream_t stream, unsigned long long* occupancy = nullptr, bool grid_all_tiles = false);
 uint32_t v4_resident_workgroups(TileShape s, bool inclusive);
 
 // Survey of wave and block scan networks over fixed-length segments

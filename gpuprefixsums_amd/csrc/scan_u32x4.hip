@@ -13,7 +13,8 @@
 //   - a tile publishes four status words (one per member, the integer word
 //     layout); a reader takes a tile only when all four carry the same flag
 //     and epoch, so a half-updated publication reads as not ready;
-//   - persistent (default) or one workgroup per tile, as the plain scan.
+//   - persistent, or one workgroup per tile (one round up to 1024 tiles), as
+//     the plain scan.
 #include "gps_internal.hpp"
 #include "tile_u32.hpp"
 
@@ -27,6 +28,7 @@ struct V4Params {
     uint64_t* status;  // 4 words per tile
     uint64_t* ticket;
     uint32_t* err;
+    uint32_t patience;              // one-round scan: polls of a window before summing a missing tile
     unsigned long long* occupancy;  // persistent kernel: +1 per workgroup that takes a tile, or null
 };
 
@@ -196,6 +198,90 @@ __global__ __launch_bounds__(BLOCK) void csdl_u32x4(V4Params p) {
     store_v4<BLOCK, VEC>(p, d, (u32x4){s_prefix[0], s_prefix[1], s_prefix[2], s_prefix[3]} + wave_prefix, tile);
 }
 
+// ---------------------------------------------------------------------------
+// One-round struct scan (device_common.hpp): the tile schedule up to
+// kRoundTiles tiles; a single tile takes no ticket and publishes nothing.
+// Back to back, against tickets and csdl_u32x4's lookback over 16-tile windows:
+// 1000 structs 3.1 us (4.0), 2^16 5.2 (5.6), 2^18 5.9 (7.3), 1,000,003 8.5
+// (10.8), 2,000,000 12.4 (13.9). Up to some 2^16 structs the 24 DPP steps and
+// 12 adds of every vector, 1 us of each CU, weigh as much as the memory;
+// runs of whole structs per lane would trade them for as many LDS cycles.
+// ---------------------------------------------------------------------------
+// Member sums of tile j (a full one of TILE structs) by one wave; lane l
+// returns member l % 4.
+template <uint32_t TILE>
+__device__ __forceinline__ uint32_t help_tile_v4(const V4Params& p, uint32_t j) {
+    const u32x4_any* v = reinterpret_cast<const u32x4_any*>(p.in + 4ull * TILE * j) + lane_id();
+    u32x4 sum = {0u, 0u, 0u, 0u};
+#pragma unroll 4
+    for (uint32_t k = 0; k < TILE / 64u; ++k) sum += v[k * 64u];
+    const uint32_t m = lane_id() & 3u;
+    const uint32_t s0 = wave_sum(sum.x), s1 = wave_sum(sum.y), s2 = wave_sum(sum.z), s3 = wave_sum(sum.w);
+    return m == 0u ? s0 : m == 1u ? s1 : m == 2u ? s2 : s3;
+}
+
+// Lane l's aggregate: member l % 4 of tile top - l / 4 (0 below tile 0).
+template <uint32_t TILE>
+__device__ __forceinline__ uint32_t round_window_v4(const V4Params& p, int64_t top, uint32_t epoch) {
+    const uint32_t lane = lane_id();
+    const int64_t idx = top - (int64_t)(lane >> 2);
+    const uint64_t* const word = p.status + kSlotWords * (uint64_t)(idx >= 0 ? idx : 0) + (lane & 3u);
+    bool helped = idx < 0;  // this lane's value is final without its word
+    uint32_t value = 0, polls = 0;
+    while (true) {
+        const uint64_t w = atomic_load_agent(word);
+        const bool ready = status_flag(w, epoch) != 0u;
+        value = helped || !ready ? value : (uint32_t)w;
+        const uint64_t missing = ballot(!ready && !helped);
+        if (!missing) return value;
+        if (++polls < p.patience) {
+            __builtin_amdgcn_s_sleep(GPS_POLL_SLEEP);
+            continue;
+        }
+        const uint32_t t = (uint32_t)__builtin_ctzll(missing) >> 2;
+        const uint32_t own = help_tile_v4<TILE>(p, (uint32_t)(top - (int64_t)t));
+        wait_performed();
+        const uint64_t again = atomic_load_agent(p.status + kSlotWords * (uint64_t)(top - (int64_t)t) + (lane & 3u));
+        const uint32_t sum = status_flag(again, epoch) != 0u ? (uint32_t)again : own;
+        value = (lane >> 2) == t ? sum : value;
+        helped = helped || (lane >> 2) == t;
+    }
+}
+
+template <int BLOCK, int VEC, bool INCL, bool SINGLE>
+__global__ __launch_bounds__(BLOCK) void csdl_round_u32x4(V4Params p) {
+    constexpr uint32_t kWaves = BLOCK / kWave, kTile = BLOCK * VEC;
+    __shared__ uint32_t s_wave[4][kWaves];
+    __shared__ u32x4 s_before[4 * kWaves];  // per row of 16 lanes: four tiles' sums, by member
+    __shared__ uint32_t s_epoch;
+    const uint32_t tile = SINGLE ? 0u : blockIdx.x, wave = wave_index(), lane = lane_id();
+    uint64_t entered = 0;
+    if (!SINGLE && threadIdx.x == 0) entered = round_enter(p.ticket, p.num_tiles);
+    u32x4 d[VEC];
+    load_v4<BLOCK, VEC>(d, p, tile);
+    if (!SINGLE && threadIdx.x == 0) s_epoch = round_epoch(p.ticket, entered, p.num_tiles);
+    u32x4 wave_prefix, tile_total;
+    scan_v4<BLOCK, VEC, INCL>(d, s_wave, wave, lane, wave_prefix, tile_total);
+    u32x4 prefix = {0u, 0u, 0u, 0u};
+    if (!SINGLE) {
+        const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
+        if (threadIdx.x == 0) publish_v4(p.status, tile, tile_total, kFlagAgg, epoch);
+        uint32_t before = 0;
+        for (int64_t top = (int64_t)tile - 1 - 16 * (int64_t)wave; top >= 0; top -= 16 * (int64_t)kWaves)
+            before += round_window_v4<kTile>(p, top, epoch);
+        before += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)before, 0x114, 0xf, 0xf, true);  // row_shr:4
+        before += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)before, 0x118, 0xf, 0xf, true);  // row_shr:8
+        if ((lane & 15u) >= 12u) s_before[4u * wave + (lane >> 4)][lane & 3u] = before;
+        if (wave == 0) wait_performed();  // the words above, before any wave's output stores
+        if (threadIdx.x == BLOCK - kWave) round_leave(p.ticket, p.status, tile, p.num_tiles);
+        __syncthreads();
+        const u32x4 b = lane < 4u * kWaves ? s_before[lane < 4u * kWaves ? lane : 0u] : prefix;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) prefix[m] = wave_sum(b[m]);
+    }
+    store_v4<BLOCK, VEC>(p, d, prefix + wave_prefix, tile);
+}
+
 // Persistent, software-pipelined form (the schedule of the plain CSDL scan's
 // default): resident workgroups own streams of tickets; with tile i scanned
 // and its aggregates published, a workgroup takes the next ticket, issues
@@ -314,9 +400,21 @@ uint32_t v4_resident_workgroups(TileShape s, bool inclusive) {
     return 0;
 }
 
-hipError_t launch_csdl_u32x4(TileShape s, bool inclusive, bool persistent, const uint32_t* in, uint32_t* out,
-                             uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream,
-                             unsigned long long* occupancy, bool grid_all_tiles) {
+// One workgroup per tile.
+template <int B, int V, bool I>
+static hipError_t launch_tile_v4(const V4Params& p, hipStream_t stream) {
+    if (p.num_tiles == 1)
+        hipLaunchKernelGGL((csdl_round_u32x4<B, V, I, true>), dim3(1), dim3(B), 0, stream, p);
+    else if (p.num_tiles <= kRoundTiles)
+        hipLaunchKernelGGL((csdl_round_u32x4<B, V, I, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+    else
+        hipLaunchKernelGGL((csdl_u32x4<B, V, I>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_csdl_u32x4(TileShape s, bool inclusive, bool persistent, uint32_t patience, const uint32_t* in,
+                             uint32_t* out, uint64_t n, uint64_t* status, uint64_t* ticket, uint32_t* err,
+                             hipStream_t stream, unsigned long long* occupancy, bool grid_all_tiles) {
     V4Params p{};
     p.in = in;
     p.out = out;
@@ -325,17 +423,14 @@ hipError_t launch_csdl_u32x4(TileShape s, bool inclusive, bool persistent, const
     p.status = status;
     p.ticket = ticket;
     p.err = err;
+    p.patience = patience;
     p.occupancy = occupancy;
 #define X(B, V)                                                                                            \
     if (s.block == B && s.vec == V) {                                                                      \
         if (persistent)                                                                                    \
             return inclusive ? launch_pp_v4<B, V, true>(p, stream, grid_all_tiles)                         \
                              : launch_pp_v4<B, V, false>(p, stream, grid_all_tiles);                       \
-        if (inclusive)                                                                                     \
-            hipLaunchKernelGGL((csdl_u32x4<B, V, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);     \
-        else                                                                                               \
-            hipLaunchKernelGGL((csdl_u32x4<B, V, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);    \
-        return hipGetLastError();                                                                          \
+        return inclusive ? launch_tile_v4<B, V, true>(p, stream) : launch_tile_v4<B, V, false>(p, stream); \
     }
     GPS_V4_SHAPES(X)
 #undef X

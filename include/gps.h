@@ -219,7 +219,7 @@ int gps_survey_scan_u32(int alg, const uint32_t* d_in, uint32_t* d_out, uint64_t
  * Other values return GPS_ERR_INVALID. No FP64 arithmetic is used. One
  * kernel launch; needs a GPS_ALGO_CSDL handle. Runs the persistent kernel on
  * a handle with the persistent schedule (a default handle: above 2^23
- * elements), else one workgroup per tile. */
+ * elements with pair carries, 2^24 with plain ones), else one workgroup per tile. */
 #define GPS_FP_PLAIN 0
 #define GPS_FP_PAIR 1
 int gps_inclusive_scan_f32(gps_handle* h, const float* d_in, float* d_out, uint64_t n, int compensated,

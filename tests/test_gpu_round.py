@@ -37,6 +37,19 @@ def check_u32(h, n, seed, inclusive, in_place):
     assert np.array_equal(got, want), (n, first_mismatch(got, want))
 
 
+def check_struct(h, n, seed, inclusive, in_place):
+    x = oracle.gen_u32(seed, 4 * n, 32)
+    d_in = to_dev(x)
+    out = d_in if in_place else torch.full_like(d_in, -7)
+    h.scan_u32x4(d_in, out, n, inclusive)
+    torch.cuda.synchronize()
+    got, x = out.cpu().numpy().view(np.uint32).reshape(n, 4), x.reshape(n, 4)
+    want = np.cumsum(x, axis=0, dtype=np.uint32)
+    if not inclusive:
+        want -= x
+    assert np.array_equal(got, want), (n, np.flatnonzero((got != want).any(axis=1))[0])
+
+
 def check_fp(h, n, seed, bf16, comp, segments, in_place):
     rng = np.random.default_rng(seed)
     x = torch.from_numpy(rng.integers(-1, 2, n)).to(torch.bfloat16 if bf16 else torch.float32).cuda()
@@ -82,6 +95,18 @@ def test_fp_tile_counts(spin, comp, bf16, segments):
         assert h.device_error() == 0
 
 
+@pytest.mark.parametrize("in_place", [False, True], ids=["apart", "in_place"])
+@pytest.mark.parametrize("spin", SPINS)
+@pytest.mark.parametrize("shape", [(512, 8), (1024, 4)])
+def test_struct_tile_counts(spin, in_place, shape):
+    with gps.ScanHandle(gps.ALGO_CSDL, 1025 * TILE, block_threads=shape[0], vec_per_thread=shape[1],
+                        schedule=gps.SCHEDULE_TILE, spin_limit=SPINS[spin]) as h:
+        for k, tiles in enumerate([1, 2, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257, 1024, 1025]):
+            for n in (tiles * TILE, tiles * TILE - 5):
+                check_struct(h, n, k, k % 2 == 0, in_place)
+        assert h.device_error() == 0
+
+
 def test_default_handle_on_both_sides_of_each_size_rule():
     with gps.ScanHandle(gps.ALGO_CSDL, (1 << 23) + 1) as h:
         for k, edge in enumerate(RULES):
@@ -91,6 +116,8 @@ def test_default_handle_on_both_sides_of_each_size_rule():
                     check_fp(h, n, k, bf16, gps.FP_PAIR, 0, False)
                     check_fp(h, n, k, bf16, gps.FP_PLAIN, 2000, False)
                 check_fp(h, n, k, False, gps.FP_PAIR, 7, True)
+                if n <= (1 << 22) + 1:
+                    check_struct(h, n, k, k % 2 == 0, False)
         assert h.device_error() == 0
 
 
