@@ -21,7 +21,7 @@ namespace gps {
 // combine the wave runs. Leaves d scanned (without the tile prefix) and sets
 // wave_prefix / tile_total.
 // ---------------------------------------------------------------------------
-template <int BLOCK, int VEC, bool INCL>
+template <int BLOCK, int VEC, bool INCL, bool LEAN = false>
 struct TileFront {
     using C = TileCfg<BLOCK, VEC>;
     u32x4 d[VEC];
@@ -43,7 +43,7 @@ struct TileFront {
         __syncthreads();
         tile = __builtin_amdgcn_readfirstlane(s_ticket[0]);
         epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
-        load_tile<VEC>(d, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
+        load_tile<VEC, LEAN>(d, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
         const uint32_t run_total = wave_scan_run<VEC, INCL>(d);
         if (lane_id() == 0) s_wave[wave] = run_total;
         __syncthreads();
@@ -500,17 +500,30 @@ __device__ __forceinline__ bool claim_for_fallback(uint64_t* status, int64_t top
     return true;
 }
 
-template <int BLOCK, int VEC, bool INCL>
-__global__ __launch_bounds__(BLOCK) void csdldf_u32(ScanParams p) {
+// STASH: the last STASH vectors of the tile wait in LDS for their prefix. In
+// registers a tile of 1024 x 8 and the lookback take 110 VGPRs, one workgroup
+// per CU; so they fit in 64, two per CU. Under emulated deadlock every tile
+// waits for its stalled predecessor to be claimed, re-read and inserted, so
+// what is resident sets the pace: 2^28 elements, period 7, 445 us so, 507
+// without. Without stalls the second workgroup gains nothing at 2^28 (368
+// against 365 us) and loses below (2^25 61 against 52).
+template <int BLOCK, int VEC, bool INCL, int STASH>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(STASH ? GPS_WAVES_PER_EU : BLOCK / 256))) void
+csdldf_u32(ScanParams p) {
     using C = TileCfg<BLOCK, VEC>;
     __shared__ uint32_t s_wave[C::kWaves];
     __shared__ uint32_t s_red[C::kWaves];
     __shared__ uint32_t s_ticket[2];
     __shared__ uint32_t s_prefix;
     __shared__ uint32_t s_poll_done, s_cas_done, s_fb_tile;
+    __shared__ uint32_t s_count[3];  // polls, fallbacks, insertions (STASH)
+    __shared__ u32x4 s_stash[STASH ? STASH * BLOCK : 1];
 
-    TileFront<BLOCK, VEC, INCL> f;
+    if (STASH && threadIdx.x == 0) s_count[0] = s_count[1] = s_count[2] = 0u;
+    TileFront<BLOCK, VEC, INCL, STASH != 0> f;
     f.run(p, s_wave, s_ticket);
+#pragma unroll
+    for (int k = 0; k < STASH; ++k) s_stash[k * BLOCK + threadIdx.x] = f.d[VEC - STASH + k];
     const uint32_t tile = f.tile, epoch = f.epoch;
     const uint32_t wave = wave_index();
     const uint32_t lane = lane_id();
@@ -539,6 +552,12 @@ __global__ __launch_bounds__(BLOCK) void csdldf_u32(ScanParams p) {
         int64_t top = (int64_t)tile - 1;
         uint64_t stale = 0;
         unsigned long long c_polls = 0, c_fallbacks = 0, c_inserts = 0;
+        const auto count = [&](int c, unsigned long long& own) {
+            if (!STASH)
+                ++own;
+            else if (lane == 0)
+                ++s_count[c];
+        };
 
         while (true) {
             if (wave == 0) {
@@ -553,7 +572,7 @@ __global__ __launch_bounds__(BLOCK) void csdldf_u32(ScanParams p) {
                     const uint64_t incl = ballot(fl == (uint32_t)kFlagIncl);
                     const uint32_t run = (~ready) ? (uint32_t)__builtin_ctzll(~ready) : 64u;
                     const uint32_t first_incl = incl ? (uint32_t)__builtin_ctzll(incl) : 64u;
-                    ++c_polls;
+                    count(0, c_polls);
                     if (first_incl < run) {
                         prefix += wave_sum(lane <= first_incl ? (uint32_t)w : 0u);
                         done = 1;
@@ -583,30 +602,41 @@ __global__ __launch_bounds__(BLOCK) void csdldf_u32(ScanParams p) {
                 }
             }
             __syncthreads();
-            if (s_poll_done) break;
+            if (STASH ? __builtin_amdgcn_readfirstlane(s_poll_done) : s_poll_done) break;
 
             // Workgroup-wide redundant reduction of tile j (always a full tile:
             // only the last tile is partial and it is nobody's predecessor).
             const uint32_t j = __builtin_amdgcn_readfirstlane(s_fb_tile);
             {
-                u32x4 fd[VEC];
-                load_tile<VEC>(fd, p.in, (uint64_t)j * C::kTile, p.n, C::kTile);
-                const uint32_t ws = wave_sum(thread_sum<VEC>(fd));
+                constexpr int kPart = STASH ? VEC - STASH : VEC;
+                constexpr uint32_t kPartElems = C::kTile / VEC * kPart;
+                uint32_t ts = 0;
+#pragma unroll 1
+                for (uint32_t at = 0; at < C::kTile; at += kPartElems) {
+                    u32x4 fd[kPart];
+                    load_tile<kPart, STASH != 0>(fd, p.in, (uint64_t)j * C::kTile + at, p.n, kPartElems);
+                    ts += thread_sum<kPart>(fd);
+                }
+                const uint32_t ws = wave_sum(ts);
                 if (lane == 0) s_red[wave] = ws;
             }
             __syncthreads();
             if (wave == 0) {
                 uint32_t fsum = 0;
+                if (STASH) {
+                    fsum = wave_sum(lane < C::kWaves ? s_red[lane < C::kWaves ? lane : 0u] : 0u);
+                } else {
 #pragma unroll
-                for (uint32_t q = 0; q < C::kWaves; ++q) fsum += s_red[q];
+                    for (uint32_t q = 0; q < C::kWaves; ++q) fsum += s_red[q];
+                }
                 const uint64_t mine = make_status(fsum, j ? kFlagAgg : kFlagIncl, epoch);
                 uint64_t found = mine;
                 if (lane == 0) found = atomic_cas_agent(p.status + kSlotWords * j, stale, mine);
                 found = ((uint64_t)readlane((uint32_t)(found >> 32), 0) << 32) | readlane((uint32_t)found, 0);
-                ++c_fallbacks;
+                count(1, c_fallbacks);
                 uint32_t fl;
                 if (found == stale) {  // inserted ours
-                    ++c_inserts;
+                    count(2, c_inserts);
                     fl = j ? (uint32_t)kFlagAgg : (uint32_t)kFlagIncl;
                     found = mine;
                 } else {
@@ -636,15 +666,17 @@ __global__ __launch_bounds__(BLOCK) void csdldf_u32(ScanParams p) {
                 }
             }
             __syncthreads();
-            if (s_cas_done) break;
+            if (STASH ? __builtin_amdgcn_readfirstlane(s_cas_done) : s_cas_done) break;
         }
         if (threadIdx.x == 0 && p.counters) {
-            atomic_add_counter(p.counters + 0, c_polls);
-            atomic_add_counter(p.counters + 1, c_fallbacks);
-            atomic_add_counter(p.counters + 2, c_inserts);
+            atomic_add_counter(p.counters + 0, STASH ? s_count[0] : c_polls);
+            atomic_add_counter(p.counters + 1, STASH ? s_count[1] : c_fallbacks);
+            atomic_add_counter(p.counters + 2, STASH ? s_count[2] : c_inserts);
         }
     }
     __syncthreads();
+#pragma unroll
+    for (int k = 0; k < STASH; ++k) f.d[VEC - STASH + k] = s_stash[k * BLOCK + threadIdx.x];
     f.store(p, s_prefix + f.wave_prefix);
 }
 
@@ -1287,16 +1319,24 @@ hipError_t launch_csdl_cw_u32(TileShape s, bool inclusive, const ScanParams& p, 
     return hipErrorInvalidValue;
 }
 
+// Tiles that stall in place, above 3 * 2^25 elements: half of a 1024 x 8 tile
+// waits in LDS (periods 7 / 2: 2^25 73.5 / 77.5 us so, 72.5 / 76.4 without; 2^26 129 /
+// 146 so, 135 / 141 without; 2^27 235 / 264 so, 259 / 276 without).
+template <int B, int V, bool I>
+static hipError_t launch_df(const ScanParams& p, uint32_t grid, hipStream_t stream) {
+    constexpr int kStash = B == 1024 && V == 8 ? 4 : 0;
+    if (kStash && p.stall_period && !p.split_pass && p.n > (3ull << 25))
+        hipLaunchKernelGGL((csdldf_u32<B, V, I, kStash>), dim3(grid), dim3(B), 0, stream, p);
+    else
+        hipLaunchKernelGGL((csdldf_u32<B, V, I, 0>), dim3(grid), dim3(B), 0, stream, p);
+    return hipGetLastError();
+}
+
 static hipError_t launch_csdldf_grid(TileShape s, bool inclusive, const ScanParams& p, uint32_t grid,
                                      hipStream_t stream) {
-#define X(B, V)                                                                            \
-    if (s.block == B && s.vec == V) {                                                      \
-        if (inclusive)                                                                     \
-            hipLaunchKernelGGL((csdldf_u32<B, V, true>), dim3(grid), dim3(B), 0, stream, p);  \
-        else                                                                               \
-            hipLaunchKernelGGL((csdldf_u32<B, V, false>), dim3(grid), dim3(B), 0, stream, p); \
-        return hipGetLastError();                                                          \
-    }
+#define X(B, V)                    \
+    if (s.block == B && s.vec == V) \
+        return inclusive ? launch_df<B, V, true>(p, grid, stream) : launch_df<B, V, false>(p, grid, stream);
     GPS_SHAPES(X)
 #undef X
     return hipErrorInvalidValue;
