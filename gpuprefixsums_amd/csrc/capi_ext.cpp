@@ -12,20 +12,26 @@ using gps::hip_fail;
 namespace {
 
 // The persistent segmented kernel unless the handle asks for one workgroup
-// per tile.
-bool seg_persistent(const gps_handle* h) { return h->schedule != GPS_SCHEDULE_TILE; }
+// per tile. A default handle runs it above 2^23 elements (100 / 16000 segments,
+// against one workgroup per tile at 1024 x 8: 9,000,000 17.8 / 19.7 against
+// 21.6 / 24.0 us, 2^23 16.9 / 17.8 against 13.9 / 15.7, 5,000,000 12.5 / 13.2
+// against 10.9 / 12.4; with three inputs in turn 2^23 17.5 / 18.4 against 16.3 / 17.8).
+bool seg_persistent(const gps_handle* h, uint64_t n) {
+    if (h->size_adaptive) return n > (1ull << 23);
+    return h->schedule != GPS_SCHEDULE_TILE;
+}
 
 // Segmented kernels use the handle's tile shape when it is one of theirs,
 // otherwise 1024 threads x 8 uint4 (32768-element tiles). A default handle
-// picks the shape from n, from the exhaustive sweep's timings on MI355X
-// (mean time over the best shape, batched u32 workloads): 1024 x 2 below
-// 2^20 elements (1.00-1.14 against 1.4-1.8 for 1024 x 8), 1024 x 4 below
-// 2^22, 1024 x 8 from there (1.00 against 1.08-1.19 for 1024 x 4).
+// picks the shape from n: 1024 x 2 up to 9 * 2^18 elements (100 / 16000
+// segments: 1,500,000 6.3 / 8.0 us against 7.1 / 8.7 for 1024 x 4, 3,000,000 8.6 /
+// 10.9 against 7.5 / 9.6), 1024 x 4 up to 2^22 (there 9.1 / 11.2 against
+// 10.7 / 12.7 for 1024 x 8; 6,000,000 1024 x 8), 1024 x 8 above.
 gps::TileShape seg_shape(const gps_handle* h, uint64_t n) {
     if (h->size_adaptive)
-        return n < (1ull << 20) ? gps::TileShape{1024, 2} : n < (1ull << 22) ? gps::TileShape{1024, 4}
-                                                                            : gps::TileShape{1024, 8};
-    return gps::seg_shape_supported(h->shape, seg_persistent(h)) ? h->shape : gps::TileShape{1024, 8};
+        return n <= (9ull << 18) ? gps::TileShape{1024, 2} : n <= (1ull << 22) ? gps::TileShape{1024, 4}
+                                                                              : gps::TileShape{1024, 8};
+    return gps::seg_shape_supported(h->shape, seg_persistent(h, n)) ? h->shape : gps::TileShape{1024, 8};
 }
 
 // FP kernels likewise: the handle's shape when it is an FP shape, else
@@ -69,8 +75,8 @@ int enqueue_segmented(gps_handle* h, const uint32_t* in, uint32_t* out, const ui
                       uint64_t num_segments, uint64_t n, bool inclusive, hipStream_t s) {
     if (n == 0) return GPS_OK;
     HIP_TRY(gps::before_epoch_launch(h, s));
-    HIP_TRY(gps::launch_segscan_u32(seg_shape(h, n), inclusive, seg_persistent(h), in, out, offsets, num_segments, n,
-                                    h->status, h->ticket, h->err, s));
+    HIP_TRY(gps::launch_segscan_u32(seg_shape(h, n), inclusive, seg_persistent(h, n), h->round_patience, in, out, offsets,
+                                    num_segments, n, h->status, h->ticket, h->err, s));
     return GPS_OK;
 }
 
@@ -222,7 +228,7 @@ int gps_segmented_graph_create(gps_handle* h, const uint32_t* d_in, uint32_t* d_
     *out = nullptr;
     int rc = check_seg(h, d_in, d_out, d_offsets, n);
     if (rc) return rc;
-    HIP_TRY(gps::prepare_segscan_u32(seg_shape(h, n), inclusive != 0, seg_persistent(h)));
+    HIP_TRY(gps::prepare_segscan_u32(seg_shape(h, n), inclusive != 0, seg_persistent(h, n)));
     hipStream_t s = nullptr;
     HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     gps_graph* g = new (std::nothrow) gps_graph();
@@ -234,8 +240,9 @@ int gps_segmented_graph_create(gps_handle* h, const uint32_t* d_in, uint32_t* d_
     if (e == hipSuccess) {
         // No re-arm check inside a capture: a graph node must not depend on
         // the host-side launch count (gps_reset re-arms explicitly).
-        rc = n ? (gps::launch_segscan_u32(seg_shape(h, n), inclusive != 0, seg_persistent(h), d_in, d_out, d_offsets,
-                                          num_segments, n, h->status, h->ticket, h->err, s) == hipSuccess
+        rc = n ? (gps::launch_segscan_u32(seg_shape(h, n), inclusive != 0, seg_persistent(h, n), h->round_patience, d_in,
+                                          d_out, d_offsets, num_segments, n, h->status, h->ticket, h->err,
+                                          s) == hipSuccess
                       ? GPS_OK
                       : GPS_ERR_HIP)
                : GPS_OK;

@@ -147,8 +147,8 @@ bool seg_shape_supported(TileShape s, bool persistent);
 // Runs the persistent kernel's one-time occupancy query (call before a
 // stream capture, so the capture holds only the launch).
 hipError_t prepare_segscan_u32(TileShape s, bool inclusive, bool persistent);
-hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, const uint32_t* in, uint32_t* out,
-                              const uint64_t* offsets, uint64_t num_segments, uint64_t n,
+hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, uint32_t patience, const uint32_t* in,
+                              uint32_t* out, const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                               uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream);
 
 // FP32 / BF16-input inclusive scans with FP32 output (2 status words per tile).

@@ -34,6 +34,7 @@ struct SegParams {
     uint64_t* status;
     uint64_t* ticket;
     uint32_t* err;
+    uint32_t patience;  // one-round scan: polls of a window before summing a missing tile
 };
 
 // Segmented scan of one wave's run (256 * VEC elements starting at tile
@@ -178,6 +179,125 @@ __global__ __launch_bounds__(BLOCK) void segscan_u32(SegParams p) {
     __syncthreads();
     seg_add_carry<VEC>(d, first_head, pre_f ? pre_v : s_prefix + pre_v);
     store_tile<VEC>(p.out, d, 0u, a, p.n, C::kTile);
+}
+
+// ---------------------------------------------------------------------------
+// One-round segmented scan (device_common.hpp): one workgroup per tile while a
+// workgroup's waves cover the tiles before it in one window each; a single
+// tile takes no ticket and publishes nothing. The search for the tile's heads
+// starts with its loads.
+// Back to back, us, against segscan_pp_u32, which served these sizes: 4096
+// elements in 100 segments 3.3 (4.7), 2^18 in 100 5.1 (6.0), 1,000,000 in 16000 7.7
+// (8.0), 2^21 + 17 in 100 / 16000 6.8 / 8.5 (8.8 / 9.4), 2^22 9.1 / 11.2 (11.6 / 12.3).
+// ---------------------------------------------------------------------------
+// Sum of the elements [from, to) by one wave.
+__device__ __forceinline__ uint32_t help_sum_u32(const uint32_t* in, uint64_t from, uint64_t to) {
+    uint32_t sum = 0;
+    for (uint64_t i = from + 4u * lane_id(); i < to; i += 256u) {
+        if (i + 4u <= to) {
+            const u32x4 x = *reinterpret_cast<const u32x4_any*>(in + i);
+            sum += (x.x + x.y) + (x.z + x.w);
+        } else {
+            for (uint64_t j = i; j < to; ++j) sum += in[j];
+        }
+    }
+    return wave_sum(sum);
+}
+
+// The carry that the tiles top, top - 1, ... (at most 64; one wave) pass on:
+// the sum back to the nearest tile that holds a head; `closed` if there is one.
+template <uint32_t TILE>
+__device__ __forceinline__ uint32_t round_window_seg_u32(const SegParams& p, int64_t top, uint32_t epoch,
+                                                         bool& closed) {
+    const uint32_t lane = lane_id();
+    const int64_t idx = top - (int64_t)lane;
+    const uint64_t* const word = p.status + kSlotWords * (uint64_t)(idx >= 0 ? idx : 0);
+    bool helped = idx < 0;
+    uint32_t flag = (uint32_t)kFlagIncl, value = 0, polls = 0;
+    while (true) {
+        const uint64_t w = atomic_load_agent(word);
+        flag = helped ? flag : status_flag(w, epoch);
+        value = helped ? value : (uint32_t)w;
+        const uint64_t ready = ballot(flag != 0u), incl = ballot(flag == (uint32_t)kFlagIncl);
+        const uint32_t run = (~ready) ? (uint32_t)__builtin_ctzll(~ready) : 64u;
+        const uint32_t first_incl = incl ? (uint32_t)__builtin_ctzll(incl) : 64u;
+        closed = first_incl < run;
+        if (closed || run == 64u) return wave_sum(lane < (closed ? first_incl + 1u : 64u) ? value : 0u);
+        if (++polls < p.patience) {
+            __builtin_amdgcn_s_sleep(GPS_POLL_SLEEP);
+            continue;
+        }
+        const uint32_t j = (uint32_t)(top - (int64_t)run);
+        const uint64_t end = (uint64_t)(j + 1u) * TILE;
+        const TailOfTile tail = find_tail(p.offsets, p.num_segments, end - TILE, end);
+        const uint32_t own = help_sum_u32(p.in, tail.from, end);
+        const uint32_t own_flag = tail.has_head || j == 0u ? (uint32_t)kFlagIncl : (uint32_t)kFlagAgg;
+        wait_performed();
+        const uint64_t again = atomic_load_agent(p.status + kSlotWords * (uint64_t)j);
+        const uint32_t f = status_flag(again, epoch);
+        if (lane == run) {
+            flag = f ? f : own_flag;
+            value = f ? (uint32_t)again : own;
+            helped = true;
+        }
+    }
+}
+
+template <int BLOCK, int VEC, bool INCL, bool SINGLE>
+__global__ __launch_bounds__(BLOCK) void segscan_round_u32(SegParams p) {
+    using C = TileCfg<BLOCK, VEC>;
+    constexpr uint32_t kWords = C::kTile / 32;
+    __shared__ uint32_t s_heads[kWords], s_bracket[C::kWaves];
+    __shared__ uint32_t s_wave_val[C::kWaves], s_wave_flag[C::kWaves], s_before[C::kWaves], s_closed[C::kWaves];
+    __shared__ uint32_t s_epoch;
+    const uint32_t tile = SINGLE ? 0u : blockIdx.x, wave = wave_index(), lane = lane_id();
+    const uint64_t lo = (uint64_t)tile * C::kTile;
+    const uint64_t hi = lo + C::kTile < p.n ? lo + C::kTile : p.n;
+    uint64_t entered = 0;
+    if (!SINGLE && threadIdx.x == 0) entered = round_enter(p.ticket, p.num_tiles);
+    u32x4 d[VEC];
+    load_tile<VEC>(d, p.in, lo, p.n, C::kTile);
+    for (uint32_t i = threadIdx.x; i < kWords; i += BLOCK) s_heads[i] = 0u;
+    __syncthreads();
+    find_and_mark_heads<BLOCK>(s_heads, s_bracket, p.offsets, p.num_segments, lo, hi, tile == 0);
+    __syncthreads();
+
+    uint32_t first_head, carry, carry_flag;
+    seg_scan_run<VEC, INCL>(d, s_heads, wave * C::kWaveElems, first_head, carry, carry_flag);
+    if (lane == 0) {
+        s_wave_val[wave] = carry;
+        s_wave_flag[wave] = carry_flag;
+    }
+    if (!SINGLE && threadIdx.x == 0) s_epoch = round_epoch(p.ticket, entered, p.num_tiles);
+    __syncthreads();
+    uint32_t pre_f, pre_v, tile_f, tile_v;
+    combine_waves_seg<C::kWaves>(s_wave_flag, s_wave_val, wave, pre_f, pre_v, tile_f, tile_v);
+    uint32_t prefix = 0;
+    if (!SINGLE) {
+        const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
+        if (threadIdx.x == 0)
+            atomic_store_agent(p.status + kSlotWords * tile,
+                               make_status(tile_v, (tile_f || tile == 0) ? kFlagIncl : kFlagAgg, epoch));
+        // A tile that starts with a head takes nothing from the ones before.
+        uint32_t before = 0;
+        bool closed = true;
+        const int64_t top = (int64_t)tile - 1 - 64 * (int64_t)wave;
+        if (top >= 0 && (s_heads[0] & 1u) == 0u) before = round_window_seg_u32<C::kTile>(p, top, epoch, closed);
+        if (lane == 0) {
+            s_before[wave] = before;
+            s_closed[wave] = closed;
+        }
+        if (wave == 0) wait_performed();  // the word above, before any wave's output stores
+        if (threadIdx.x == BLOCK - kWave) round_leave(p.ticket, p.status, tile, p.num_tiles);
+        __syncthreads();
+        // Windows up to the nearest one that is closed.
+        const uint32_t q = lane < C::kWaves ? lane : 0u;
+        const uint64_t stop = ballot(lane < C::kWaves && s_closed[q] != 0u);
+        const uint32_t take = stop ? (uint32_t)__builtin_ctzll(stop) + 1u : C::kWaves;
+        prefix = wave_sum(lane < take ? s_before[q] : 0u);
+    }
+    seg_add_carry<VEC>(d, first_head, pre_f ? pre_v : prefix + pre_v);
+    store_tile<VEC>(p.out, d, 0u, lo, p.n, C::kTile);
 }
 
 // ---------------------------------------------------------------------------
@@ -359,8 +479,20 @@ hipError_t prepare_segscan_u32(TileShape s, bool inclusive, bool persistent) {
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, const uint32_t* in, uint32_t* out,
-                              const uint64_t* offsets, uint64_t num_segments, uint64_t n,
+// One workgroup per tile.
+template <int B, int V, bool I>
+static hipError_t launch_seg_tile(const SegParams& p, hipStream_t stream) {
+    if (p.num_tiles == 1)
+        hipLaunchKernelGGL((segscan_round_u32<B, V, I, true>), dim3(1), dim3(B), 0, stream, p);
+    else if (p.num_tiles <= (uint32_t)B + 1u)  // B / 64 waves x 64 tiles
+        hipLaunchKernelGGL((segscan_round_u32<B, V, I, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+    else
+        hipLaunchKernelGGL((segscan_u32<B, V, I>), dim3(p.num_tiles), dim3(B), 0, stream, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, uint32_t patience, const uint32_t* in,
+                              uint32_t* out, const uint64_t* offsets, uint64_t num_segments, uint64_t n,
                               uint64_t* status, uint64_t* ticket, uint32_t* err, hipStream_t stream) {
     SegParams p{};
     p.in = in;
@@ -372,6 +504,7 @@ hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, cons
     p.status = status;
     p.ticket = ticket;
     p.err = err;
+    p.patience = patience;
     if (persistent) {
 #define X(B, V)                                                                                              \
     if (s.block == B && s.vec == V)                                                                          \
@@ -380,14 +513,9 @@ hipError_t launch_segscan_u32(TileShape s, bool inclusive, bool persistent, cons
 #undef X
         return hipErrorInvalidValue;
     }
-#define X(B, V)                                                                                          \
-    if (s.block == B && s.vec == V) {                                                                    \
-        if (inclusive)                                                                                   \
-            hipLaunchKernelGGL((segscan_u32<B, V, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);  \
-        else                                                                                             \
-            hipLaunchKernelGGL((segscan_u32<B, V, false>), dim3(p.num_tiles), dim3(B), 0, stream, p); \
-        return hipGetLastError();                                                                        \
-    }
+#define X(B, V)                      \
+    if (s.block == B && s.vec == V) \
+        return inclusive ? launch_seg_tile<B, V, true>(p, stream) : launch_seg_tile<B, V, false>(p, stream);
     GPS_SEG_SHAPES(X)
 #undef X
     return hipErrorInvalidValue;

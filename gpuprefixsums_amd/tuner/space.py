@@ -106,8 +106,8 @@ def candidates(dtype: str, stall_period: int = 0) -> List[Config]:
 
 def default_config(dtype: str, segments: int, n: int = 1 << 30, stall_period: int = 0) -> Config:
     """What the library does without the tuner: a default handle's choice for
-    n elements (the same rules as libgps's size-adaptive defaults, but for two
-    things: pair scans run persistent above 2^23 elements, and the segmented FP
+    n elements (the same rules as libgps's size-adaptive defaults, but for three
+    things: segmented uint32 scans run one workgroup per tile up to 2^23 elements, pair scans run persistent above 2^23 elements, and the segmented FP
     kernel has 512 x 4 tiles, no candidate, between 2^20 and 9 * 2^18). Under
     emulated deadlock it is the default decoupled-fallback handle (1024 x 8,
     spin limit 4)."""

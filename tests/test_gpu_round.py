@@ -50,6 +50,19 @@ def check_struct(h, n, seed, inclusive, in_place):
     assert np.array_equal(got, want), (n, np.flatnonzero((got != want).any(axis=1))[0])
 
 
+def check_segmented(h, n, seed, inclusive, segments, in_place):
+    rng = np.random.default_rng(seed)
+    x = oracle.gen_u32(seed, n, 32)
+    cuts = np.r_[0, np.sort(rng.integers(0, n + 1, segments - 1)), n].astype(np.uint64)  # some of them empty
+    d_in = to_dev(x)
+    out = d_in if in_place else torch.full_like(d_in, -7)
+    off = torch.from_numpy(cuts.view(np.int64)).cuda()
+    h.segmented(d_in, out, off, segments, n, inclusive)
+    torch.cuda.synchronize()
+    got, want = out.cpu().numpy().view(np.uint32), oracle.segmented_scan_u32(x, cuts, inclusive)
+    assert np.array_equal(got, want), (n, first_mismatch(got, want))
+
+
 def check_fp(h, n, seed, bf16, comp, segments, in_place):
     rng = np.random.default_rng(seed)
     x = torch.from_numpy(rng.integers(-1, 2, n)).to(torch.bfloat16 if bf16 else torch.float32).cuda()
@@ -97,6 +110,18 @@ def test_fp_tile_counts(spin, comp, bf16, segments):
 
 @pytest.mark.parametrize("in_place", [False, True], ids=["apart", "in_place"])
 @pytest.mark.parametrize("spin", SPINS)
+@pytest.mark.parametrize("segments", [1, 5, 3000])
+def test_segmented_u32_tile_counts(spin, in_place, segments):
+    with gps.ScanHandle(gps.ALGO_CSDL, 1025 * TILE, block_threads=256, vec_per_thread=4,
+                        schedule=gps.SCHEDULE_TILE, spin_limit=SPINS[spin]) as h:
+        for k, tiles in enumerate([*TILES, 1025]):
+            for n in (tiles * TILE, tiles * TILE - 5):
+                check_segmented(h, n, k, k % 2 == 0, segments, in_place)
+        assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("in_place", [False, True], ids=["apart", "in_place"])
+@pytest.mark.parametrize("spin", SPINS)
 @pytest.mark.parametrize("shape", [(512, 8), (1024, 4)])
 def test_struct_tile_counts(spin, in_place, shape):
     with gps.ScanHandle(gps.ALGO_CSDL, 1025 * TILE, block_threads=shape[0], vec_per_thread=shape[1],
@@ -112,6 +137,7 @@ def test_default_handle_on_both_sides_of_each_size_rule():
         for k, edge in enumerate(RULES):
             for n in (edge, edge + 1):
                 check_u32(h, n, k, k % 2 == 0, False)
+                check_segmented(h, n, k, k % 2 == 1, 2000, k % 2 == 0)
                 for bf16 in (False, True):
                     check_fp(h, n, k, bf16, gps.FP_PAIR, 0, False)
                     check_fp(h, n, k, bf16, gps.FP_PLAIN, 2000, False)
