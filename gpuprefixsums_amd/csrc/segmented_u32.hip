@@ -48,7 +48,8 @@ struct SegParams {
 // head lane below (the lane carry is a difference of two plain prefixes,
 // exact mod 2^32). The exclusive form needs no copy of the input: element c
 // takes 0 at a head, else the inclusive value of element c - 1.
-template <int VEC, bool INCL>
+// LONG: a run without a head, the usual one then, takes the plain scan.
+template <int VEC, bool INCL, bool LONG = false>
 __device__ __forceinline__ void seg_scan_run(u32x4 (&d)[VEC], const uint32_t* s_heads, uint32_t run_base,
                                              uint32_t& first_head, uint32_t& carry, uint32_t& carry_flag) {
     const uint32_t lane = lane_id();
@@ -56,6 +57,14 @@ __device__ __forceinline__ void seg_scan_run(u32x4 (&d)[VEC], const uint32_t* s_
     first_head = kRun;
     carry = 0;
     carry_flag = 0;
+    if (LONG) {
+        constexpr uint32_t kRunWords = kRun / 32u;  // at most one per lane
+        static_assert(kRunWords <= kWave, "a lane per bitmap word");
+        if (ballot(lane < kRunWords && s_heads[run_base / 32u + lane % kRunWords] != 0u) == 0ull) {
+            carry = wave_scan_run<VEC, INCL>(d);
+            return;
+        }
+    }
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
         const uint32_t nib = run_nibble(s_heads + run_base / 32u + lane / 8u, k, lane);
@@ -101,9 +110,14 @@ __device__ __forceinline__ void seg_scan_run(u32x4 (&d)[VEC], const uint32_t* s_
 
 // Adds the carry from earlier runs and tiles to the elements before the
 // run's first head.
-template <int VEC>
+template <int VEC, bool LONG = false>
 __device__ __forceinline__ void seg_add_carry(u32x4 (&d)[VEC], uint32_t first_head, uint32_t run_in) {
     const uint32_t lane = lane_id();
+    if (!LONG && first_head == 256u * VEC) {  // no head: the whole run (with LONG's registers this spills)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) d[k] += run_in;
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < VEC; ++k)
 #pragma unroll
@@ -310,8 +324,14 @@ __global__ __launch_bounds__(BLOCK) void segscan_round_u32(SegParams p) {
 // prefetch, so the search's dependent loads do not queue behind it). Every
 // workgroup ends on exactly one ticket past the last tile, so the ticket word
 // re-arms after num_tiles + gridDim.x tickets.
+//
+// 50.9 M elements, 407 MB: the same tiles in csdl_pp_u32 take 70.5 us. What the
+// segments cost is arithmetic, some 35 instructions a vector that four waves
+// per SIMD cannot hide: 78 us when every run took it; LONG, which gives runs
+// without a head the plain scan, 75.3 us in 4096 segments (72.0 in 10), and
+// only the carry without compares for those runs 76.4.
 // ---------------------------------------------------------------------------
-template <int BLOCK, int VEC, bool INCL>
+template <int BLOCK, int VEC, bool INCL, bool LONG>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void segscan_pp_u32(
     SegParams p) {
     using C = TileCfg<BLOCK, VEC>;
@@ -339,7 +359,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     if (tile >= p.num_tiles) return;
 
     u32x4 a[VEC], b[VEC];
-    load_tile<VEC>(a, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
+    load_tile<VEC, true>(a, p.in, (uint64_t)tile * C::kTile, p.n, C::kTile);
     {
         const uint64_t lo = (uint64_t)tile * C::kTile;
         const uint64_t hi = lo + C::kTile < p.n ? lo + C::kTile : p.n;
@@ -355,7 +375,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     uint32_t cur = 0;
     while (true) {
         uint32_t first_head, carry, carry_flag;
-        seg_scan_run<VEC, INCL>(a, s_heads[cur], wave * C::kWaveElems, first_head, carry, carry_flag);
+        seg_scan_run<VEC, INCL, LONG>(a, s_heads[cur], wave * C::kWaveElems, first_head, carry, carry_flag);
         if (lane == 0) {
             s_wave_val[wave] = carry;
             s_wave_flag[wave] = carry_flag;
@@ -388,7 +408,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             mark_heads_by(s_heads[cur ^ 1u], p.offsets, p.num_segments, s0, lo, hi, next == 0, lane, kWave);
         }
         if (has_next) {
-            load_tile<VEC>(b, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
+            load_tile<VEC, true>(b, p.in, (uint64_t)next * C::kTile, p.n, C::kTile);
         }
         if (wave == 0) {
             uint32_t prefix = 0;
@@ -400,7 +420,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             if (lane == 0) s_prefix = prefix;
         }
         __syncthreads();  // also completes the next tile's head bitmap
-        seg_add_carry<VEC>(a, first_head, pre_f ? pre_v : s_prefix + pre_v);
+        seg_add_carry<VEC, LONG>(a, first_head, pre_f ? pre_v : s_prefix + pre_v);
         store_tile<VEC>(p.out, a, 0u, (uint64_t)tile * C::kTile, p.n, C::kTile);
         if (!has_next) break;
         for (int k = 0; k < VEC; ++k) a[k] = b[k];
@@ -442,7 +462,7 @@ bool seg_shape_supported(TileShape s, bool persistent) {
 
 // Persistent grid: as many workgroups as fit on the device at once (queried
 // once per kernel instance and process), at most one per tile.
-template <int B, int V, bool I>
+template <int B, int V, bool I, bool LONG>
 static uint32_t seg_pp_residency() {
     struct Residency {
         uint32_t workgroups = 0;
@@ -450,7 +470,7 @@ static uint32_t seg_pp_residency() {
             int dev = 0, cus = 0, per_cu = 0;
             if (hipGetDevice(&dev) != hipSuccess) return;
             if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, segscan_pp_u32<B, V, I>, B, 0) != hipSuccess)
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, segscan_pp_u32<B, V, I, LONG>, B, 0) != hipSuccess)
                 return;
             workgroups = (uint32_t)(cus > 0 ? cus : 1) * (uint32_t)(per_cu > 0 ? per_cu : 1);
         }
@@ -459,21 +479,42 @@ static uint32_t seg_pp_residency() {
     return r.workgroups;
 }
 
-template <int B, int V, bool I>
+// Segments of 8192 elements and more on average, four runs of a wave at
+// 1024 x 8, are long (there 53.4 against 54.6 us at 2^25 elements; at 2930 on average
+// 23.2 against 22.6 at 12,000,000).
+template <int B, int V>
+static bool long_segments(uint64_t n, uint64_t num_segments) {
+    return V == 8 && B == 1024 && n / 8192u >= num_segments;
+}
+
+template <int B, int V, bool I, bool LONG>
 static hipError_t launch_seg_pp(const SegParams& p, hipStream_t stream) {
-    const uint32_t resident = seg_pp_residency<B, V, I>();
+    const uint32_t resident = seg_pp_residency<B, V, I, LONG>();
     if (resident == 0) return hipErrorInvalidDevice;
     const uint32_t grid = persistent_grid(p.num_tiles, resident);
-    hipLaunchKernelGGL((segscan_pp_u32<B, V, I>), dim3(grid), dim3(B), 0, stream, p);
+    hipLaunchKernelGGL((segscan_pp_u32<B, V, I, LONG>), dim3(grid), dim3(B), 0, stream, p);
     return hipGetLastError();
+}
+
+template <int B, int V, bool I>
+static hipError_t launch_seg_pp(const SegParams& p, hipStream_t stream) {
+    constexpr bool kHasLong = V == 8 && B == 1024;
+    return kHasLong && long_segments<B, V>(p.n, p.num_segments) ? launch_seg_pp<B, V, I, kHasLong>(p, stream)
+                                                                : launch_seg_pp<B, V, I, false>(p, stream);
+}
+
+template <int B, int V, bool I>
+static bool seg_pp_resident() {
+    constexpr bool kHasLong = V == 8 && B == 1024;
+    return seg_pp_residency<B, V, I, false>() && seg_pp_residency<B, V, I, kHasLong>();
 }
 
 hipError_t prepare_segscan_u32(TileShape s, bool inclusive, bool persistent) {
     if (!persistent) return hipSuccess;
 #define X(B, V)                                                                                               \
     if (s.block == B && s.vec == V)                                                                           \
-        return (inclusive ? seg_pp_residency<B, V, true>() : seg_pp_residency<B, V, false>()) ? hipSuccess \
-                                                                                               : hipErrorInvalidDevice;
+        return (inclusive ? seg_pp_resident<B, V, true>() : seg_pp_resident<B, V, false>()) ? hipSuccess       \
+                                                                                             : hipErrorInvalidDevice;
     GPS_SEG_PP_SHAPES(X)
 #undef X
     return hipErrorInvalidValue;
