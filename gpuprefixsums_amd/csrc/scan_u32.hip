@@ -543,7 +543,10 @@ csdldf_u32(ScanParams p) {
         }
         atomic_xchg_agent(p.status + kSlotWords * tile, make_status(f.tile_total, tile ? kFlagAgg : kFlagIncl, epoch));
         if (p.counters) atomic_add_counter(p.counters + 3, stall_timeouts);
-        if (tile == 0) s_prefix = 0;
+        if (tile == 0) {
+            s_prefix = 0;
+            wait_performed();  // the exchange, before the output stores; other tiles wait in their lookback
+        }
     }
 
     if (tile != 0) {
@@ -1223,9 +1226,13 @@ hipError_t launch_csdl_u32(TileShape s, bool inclusive, const ScanParams& p, hip
         S(64, 2) S(256, 2) S(512, 2) S(1024, 2) S(1024, 4) S(1024, 8)
 #undef S
     }
+    // A carry chained through one word takes tickets: a one-round scan's last
+    // tile may end, and replace the word, before tile 0 or a wave that sums
+    // tile 0 in its place has read it.
+    const bool round = p.num_tiles <= kRoundTiles && !(p.carry_in && p.carry_in == p.carry_out);
 #define X(B, V)                                                                          \
     if (s.block == B && s.vec == V) {                                                    \
-        if (p.num_tiles <= kRoundTiles) {                                                \
+        if (round) {                                                                     \
             if (inclusive)                                                               \
                 hipLaunchKernelGGL((csdl_round_u32<B, V, true>), dim3(p.num_tiles), dim3(B), 0, stream, p);  \
             else                                                                         \

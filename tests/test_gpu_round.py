@@ -17,7 +17,7 @@ from tests.gpu_util import first_mismatch, to_dev  # noqa: E402
 
 TILE = 4096  # 256 threads x 4 vectors
 TILES = [1, 2, 16, 17, 63, 64, 65, 66, 80, 81, 129, 256, 257, 258]
-RULES = [1, 2048, 4096, 8192, 16384, 1 << 18, 1 << 19, 1 << 20, 9 << 18, 1 << 21, 1 << 22, 1 << 23]
+RULES = [1, 2048, 4096, 8192, 16384, 1 << 18, 1 << 19, 1 << 20, 9 << 18, 1 << 21, 3 << 20, 1 << 22, 1 << 23]
 SPINS = {"default": 0, "help": 1}
 
 
@@ -92,6 +92,25 @@ def test_u32_tile_counts(spin, in_place):
         for k, tiles in enumerate([*TILES, 1023, 1024, 1025]):
             for n in (tiles * TILE, tiles * TILE - 5):
                 check_u32(h, n, k, k % 2 == 0, in_place)
+        assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("same_word", [False, True], ids=["two_words", "one_word"])
+@pytest.mark.parametrize("spin", SPINS)
+def test_u32_carries(spin, same_word):
+    with gps.ScanHandle(gps.ALGO_CSDL, 257 * TILE, block_threads=256, vec_per_thread=4,
+                        schedule=gps.SCHEDULE_TILE, spin_limit=SPINS[spin]) as h:
+        for k, tiles in enumerate([1, 2, 64, 65, 66, 257]):
+            n, first = tiles * TILE - 3, 0x9E3779B9
+            x = oracle.gen_u32(k, n, 32)
+            want = oracle.scan_u32(x, True) + np.uint32(first)
+            word = torch.tensor([first - (1 << 32)], dtype=torch.int32, device="cuda")
+            after = word if same_word else torch.zeros_like(word)
+            d_in = to_dev(x)
+            h.scan_carry(d_in, d_in, n, True, word, after)
+            torch.cuda.synchronize()
+            assert np.array_equal(d_in.cpu().numpy().view(np.uint32), want), tiles
+            assert int(after.item()) & 0xFFFFFFFF == int(want[-1])
         assert h.device_error() == 0
 
 
