@@ -101,7 +101,9 @@ bool shape_supported(TileShape s);
 // measured on MI355X (back-to-back launches): below 2^24 elements one
 // workgroup per tile, all started together (the one-round scan), beats the
 // persistent grid, which has too few tiles per workgroup to pay for its ramp;
-// up to 2^21 smaller tiles also occupy more of the chip. 2^20: 5.1 us; 2^23:
+// up to 3 * 2^20 smaller tiles also occupy more of the chip (2,500,000: 6.0
+// against 6.9 us for 1024 x 8; 3,500,000 6.7 against 7.2, with three inputs in
+// turn 8.1 against 7.9). 2^20: 5.1 us; 2^23:
 // 11.4 against 14.5; 12,345,677: 17.9 against 18.2; just below 2^24 24.1
 // against 23.0. Leaves shape and schedule unchanged there.
 inline void size_adaptive_config(uint64_t n, TileShape& shape, uint32_t& schedule) {
@@ -109,7 +111,7 @@ inline void size_adaptive_config(uint64_t n, TileShape& shape, uint32_t& schedul
     if (n <= (1ull << 18)) {
         shape = {1024, 2};
         schedule = kTile;
-    } else if (n <= (1ull << 21)) {
+    } else if (n <= (3ull << 20)) {
         shape = {1024, 4};
         schedule = kTile;
     } else if (n < (1ull << 24)) {

@@ -124,7 +124,7 @@ def default_config(dtype: str, segments: int, n: int = 1 << 30, stall_period: in
     if segments == 1:
         if n <= 1 << 18:
             return Config("loop_csdl", 1024, 2, tile=True)
-        if n <= 1 << 21:
+        if n <= 3 << 20:
             return Config("loop_csdl", 1024, 4, tile=True)
         if n < 1 << 24:
             return Config("loop_csdl", 1024, 8, tile=True)
