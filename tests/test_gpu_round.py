@@ -202,3 +202,26 @@ def test_replays_of_a_captured_scan(n):
             h.scan(d_in, out, n, True)
             assert torch.equal(out, want)
         assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("n", [0, 5, 1 << 16, (1 << 20) + 1, (1 << 23) + 5])
+@pytest.mark.parametrize("own_stream", [False, True], ids=["null_stream", "own_stream"])
+def test_segmented_graph_replays(n, own_stream):
+    segments = 37
+    cuts = np.linspace(0, n, segments + 1).astype(np.uint64)
+    x = oracle.gen_u32(n + 1, max(n, 1), 32)[:n]
+    want = torch.from_numpy(oracle.segmented_scan_u32(x, cuts, False).view(np.int32)).cuda() if n else None
+    d_in, out = to_dev(oracle.gen_u32(n + 1, max(n, 1), 32)), torch.empty(max(n, 1), dtype=torch.int32, device="cuda")
+    off = torch.from_numpy(cuts.view(np.int64)).cuda()
+    stream = torch.cuda.Stream() if own_stream else torch.cuda.current_stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream), gps.ScanHandle(gps.ALGO_CSDL, max(n, 1)) as h:
+        with h.segmented_graph(d_in, out, off, segments, n, False) as g:
+            for _ in range(4):
+                out.fill_(-7)
+                g.launch(stream)
+                assert n == 0 or torch.equal(out[:n], want)
+                out.fill_(-7)
+                h.segmented(d_in, out, off, segments, n, False)
+                assert n == 0 or torch.equal(out[:n], want)
+        assert h.device_error() == 0
