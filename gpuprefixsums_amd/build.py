@@ -14,6 +14,7 @@ infrastructure) with make.
 from __future__ import annotations
 
 import concurrent.futures as cf
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -158,7 +159,8 @@ def build_oracle() -> Path:
 
 def build_all() -> None:
     build_lib()
-    build_torch()
+    if importlib.util.find_spec("torch"):  # without PyTorch there are no operators to serve
+        build_torch()
     build_main()
     build_oracle()
 
