@@ -16,6 +16,7 @@
 // This file is compiled with -ffp-contract=off: a fused multiply-add would
 // break the TwoSum error terms.
 #include "gps_internal.hpp"
+#include "round_rules.hpp"
 #include "segments.hpp"
 #include "tile_u32.hpp"
 
@@ -1542,7 +1543,7 @@ template <int B, int V, bool BF16, bool COMP>
 static void launch_fp_tile(const FpParams& p, hipStream_t stream) {
     if (p.num_tiles == 1)
         hipLaunchKernelGGL((scan_fp_round<B, V, BF16, COMP, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (p.num_tiles <= kRoundTiles)
+    else if (p.num_tiles <= kRoundTiles && round_buffers(p.in, (BF16 ? 2u : 4u) * p.n, p.out, 4u * p.n))
         hipLaunchKernelGGL((scan_fp_round<B, V, BF16, COMP, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((scan_fp<B, V, BF16, COMP>), dim3(p.num_tiles), dim3(B), 0, stream, p);

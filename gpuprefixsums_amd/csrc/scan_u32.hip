@@ -12,6 +12,7 @@
 //     (the inclusive and exclusive fallback kernels)
 //   GPUPrefixSumsCUDA/ReduceThenScan.cuh:15-161 (RTS)
 #include "gps_internal.hpp"
+#include "round_rules.hpp"
 #include "tile_u32.hpp"
 
 namespace gps {
@@ -1226,10 +1227,9 @@ hipError_t launch_csdl_u32(TileShape s, bool inclusive, const ScanParams& p, hip
         S(64, 2) S(256, 2) S(512, 2) S(1024, 2) S(1024, 4) S(1024, 8)
 #undef S
     }
-    // A carry chained through one word takes tickets: a one-round scan's last
-    // tile may end, and replace the word, before tile 0 or a wave that sums
-    // tile 0 in its place has read it.
-    const bool round = p.num_tiles <= kRoundTiles && !(p.carry_in && p.carry_in == p.carry_out);
+    // Buffers that overlap and a carry chained through one word take tickets.
+    const bool round = p.num_tiles <= kRoundTiles && round_buffers(p.in, 4u * p.n, p.out, 4u * p.n) &&
+                       round_carries(p.carry_in, p.carry_out, p.in, p.out, 4u * p.n);
 #define X(B, V)                                                                          \
     if (s.block == B && s.vec == V) {                                                    \
         if (round) {                                                                     \

@@ -16,6 +16,7 @@
 //   - persistent, or one workgroup per tile (one round up to 1024 tiles), as
 //     the plain scan.
 #include "gps_internal.hpp"
+#include "round_rules.hpp"
 #include "tile_u32.hpp"
 
 namespace gps {
@@ -405,7 +406,7 @@ template <int B, int V, bool I>
 static hipError_t launch_tile_v4(const V4Params& p, hipStream_t stream) {
     if (p.num_tiles == 1)
         hipLaunchKernelGGL((csdl_round_u32x4<B, V, I, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (p.num_tiles <= kRoundTiles)
+    else if (p.num_tiles <= kRoundTiles && round_buffers(p.in, 16u * p.n, p.out, 16u * p.n))
         hipLaunchKernelGGL((csdl_round_u32x4<B, V, I, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((csdl_u32x4<B, V, I>), dim3(p.num_tiles), dim3(B), 0, stream, p);
