@@ -221,7 +221,7 @@ int gps_create(int algo, uint64_t max_n, const gps_tuning* tuning, gps_handle** 
     h->max_n = max_n;
     h->shape = shape;
     h->spin_limit = spin_limit;
-    if (tuning && tuning->spin_limit) h->round_patience = tuning->spin_limit;
+    h->round_patience = gps::round_patience(tuning && tuning->schedule == GPS_SCHEDULE_TILE, spin_limit);
     h->stall_period = stall_period;
     h->schedule = schedule;
     h->size_adaptive = size_adaptive;

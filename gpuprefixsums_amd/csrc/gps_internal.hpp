@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "round_rules.hpp"
+
 namespace gps {
 
 // Tile status words are laid out one tile per 128-byte slot of kSlotWords
@@ -18,11 +20,6 @@ constexpr uint64_t kSlotWords = 16;
 constexpr uint64_t kCounterWords = 8;
 constexpr uint64_t kCounterOccupancy = 4;
 
-// Polls of a status window before a wave of a one-round scan computes a
-// missing tile's aggregate itself: tens of microseconds, far beyond what a
-// workgroup that has started needs.
-constexpr uint32_t kRoundPatience = 64;
-
 // Launch parameters shared by the single-pass uint32 kernels (CSDL, CSDLDF).
 struct ScanParams {
     const uint32_t* in;
@@ -32,7 +29,7 @@ struct ScanParams {
     uint64_t* status;  // one word per tile
     uint64_t* ticket;  // (epoch << 32) | tickets taken
     uint32_t* err;     // device error bits (watchdogs)
-    uint32_t spin_limit;  // decoupled fallback, and the one-round scan's patience
+    uint32_t spin_limit;  // decoupled fallback; the one-round scan: its patience
     // decoupled fallback only
     uint32_t stall_period;              // 0: no emulated stalls
     unsigned long long* counters;       // [polls, fallbacks, insertions, stall timeouts] or null

@@ -41,7 +41,7 @@ struct gps_handle {
     uint64_t max_n = 0;
     gps::TileShape shape{256, 4};
     uint32_t spin_limit = 4;
-    uint32_t round_patience = gps::kRoundPatience;  // CSDL: tuning.spin_limit if given
+    uint32_t round_patience = gps::kRoundPatience;
     uint32_t stall_period = 0;
     uint32_t schedule = GPS_SCHEDULE_TILE;
     bool size_adaptive = false;  // CSDL with default shape and schedule: both picked per call from n

@@ -16,7 +16,6 @@
 // This file is compiled with -ffp-contract=off: a fused multiply-add would
 // break the TwoSum error terms.
 #include "gps_internal.hpp"
-#include "round_rules.hpp"
 #include "segments.hpp"
 #include "tile_u32.hpp"
 

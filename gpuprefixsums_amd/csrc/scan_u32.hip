@@ -12,7 +12,6 @@
 //     (the inclusive and exclusive fallback kernels)
 //   GPUPrefixSumsCUDA/ReduceThenScan.cuh:15-161 (RTS)
 #include "gps_internal.hpp"
-#include "round_rules.hpp"
 #include "tile_u32.hpp"
 
 namespace gps {

@@ -16,7 +16,6 @@
 //   - persistent, or one workgroup per tile (one round up to 1024 tiles), as
 //     the plain scan.
 #include "gps_internal.hpp"
-#include "round_rules.hpp"
 #include "tile_u32.hpp"
 
 namespace gps {

@@ -53,9 +53,10 @@ typedef struct gps_tuning {
     uint32_t vec_per_thread; /* uint4 vectors per thread: 2, 4 or 8 (items = 4x) */
     uint32_t spin_limit;     /* CSDLDF: polls without progress before a fallback (default 4), for the
                                 blocking tile's nearest successor; a waiter k tiles farther waits
-                                (1 + min(k, 7)) x spin_limit polls; at most 65536. CSDL, one workgroup
-                                per tile, up to 1024 tiles: polls before a workgroup sums a tile that
-                                it waits for by itself (default 64) */
+                                (1 + min(k, 7)) x spin_limit polls; at most 65536. CSDL
+                                handles take no notice of it, but with GPS_SCHEDULE_TILE 1, 2 or 3
+                                make a workgroup that waits for a tile sum it by itself after 1, 4 or
+                                16 polls instead of 64 (slower; for tests) */
     uint32_t stall_period;   /* CSDLDF: stall tiles with index % period == 0 (0 = no emulation, >= 2);
                                 with GPS_SCHEDULE_SPLIT, defer them to a second launch instead */
     uint32_t schedule;       /* CSDL, CSDLDF: GPS_SCHEDULE_* (0 = default) */

@@ -22,7 +22,7 @@ def holds(tmp_path, *conditions):
     src, exe = tmp_path / "rules.cpp", tmp_path / "rules"
     checks = "\n".join(f"    if (!({c})) return {k + 1};" for k, c in enumerate(conditions))
     src.write_text('#include "round_rules.hpp"\nusing namespace gps;\n'
-                   "static const uint32_t* at(uint64_t k) { return reinterpret_cast<const uint32_t*>(4096 + k); }\n"
+                   "[[maybe_unused]] static const uint32_t* at(uint64_t k) { return reinterpret_cast<const uint32_t*>(4096 + k); }\n"
                    f"int main() {{\n{checks}\n    return 0;\n}}\n")
     subprocess.run([cxx, "-std=c++17", "-Wall", "-Werror", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
     k = subprocess.run([str(exe)]).returncode
@@ -52,6 +52,16 @@ def test_carry_words(tmp_path):
           "!round_carries(at(796), at(900), at(0), at(400), 400)",
           "!round_carries(nullptr, at(0), at(0), at(400), 400)",   # written: anywhere but input and output
           "!round_carries(nullptr, at(796), at(0), at(400), 400)")
+
+
+def test_patience(tmp_path):
+    """Spin limits as they were given before the one-round scans, and as a
+    handle reports them (4 by default), leave the patience at 64 polls; only a
+    tile-schedule handle asks for less."""
+    holds(tmp_path,
+          "kRoundPatience == 64",
+          *(f"round_patience(false, {s}) == 64" for s in (1, 2, 3, 4, 32, 65536)),
+          *(f"round_patience(true, {s}) == {p}" for s, p in ((1, 1), (2, 4), (3, 16), (4, 64), (5, 64), (65536, 64))))
 
 
 def shifted_tile(mem, t, epoch, patience, stats):
