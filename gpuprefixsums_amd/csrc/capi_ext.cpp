@@ -398,22 +398,18 @@ int gps_inclusive_scan_fp_per_segment(gps_handle* h, const void* d_in, float* d_
 
 // A replay of one kernel is that kernel's launch: 3.1 us of the host against
 // 14 for hipGraphLaunch, whose packets also put 4 us between kernels (50.9 M
-// elements 75.6 against 79.7 us a replay). On another device than the
-// graph's, on a stream that is being captured, and where an error of an earlier
-// HIP call is pending, which the launch would return as its own, the graph is
-// launched.
+// elements 75.6 against 79.7 us a replay). A stream that is being captured
+// records it, where hipGraphLaunch reports success and records nothing. The
+// graph is launched where another device is current than its own, or an error
+// of an earlier HIP call is pending, which the launch would return as its own.
 int gps_graph_launch(gps_graph* g, void* stream) {
     if (!g || !g->exec) return fail(GPS_ERR_INVALID, "null graph");
     const hipStream_t s = static_cast<hipStream_t>(stream);
     int device = -1;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
-    const bool pending = hipPeekAtLastError() != hipSuccess;
-    if (!pending && hipGetDevice(&device) == hipSuccess && device == g->device &&
-        hipStreamIsCapturing(s, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone) {
+    if (hipPeekAtLastError() == hipSuccess && hipGetDevice(&device) == hipSuccess && device == g->device) {
         HIP_TRY(g->launch(s));
         return GPS_OK;
     }
-    if (!pending) (void)hipGetLastError();  // a refused query is no error of the replay
     HIP_TRY(hipGraphLaunch(g->exec, s));
     return GPS_OK;
 }

@@ -1,5 +1,6 @@
-"""gps_graph_launch with an error of an earlier HIP call pending: one graph per
-kernel that a replay can launch (a single tile, one round, persistent)."""
+"""gps_graph_launch into a stream that is being captured, and with an error of
+an earlier HIP call pending: one graph per kernel that a replay can launch (a
+single tile, one round, persistent)."""
 import ctypes
 
 import numpy as np
@@ -44,6 +45,25 @@ class Replay:
         self.g.close()
         assert self.h.device_error() == 0
         self.h.close()
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_replay_recorded_by_a_capture(n):
+    r = Replay(n)
+    s = torch.cuda.Stream()
+    outer = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(outer, stream=s):
+        r.out.fill_(-7)
+        r.g.launch(s)
+    for _ in range(4):
+        outer.replay()
+        assert r.right()
+        r.out.fill_(-7)
+        torch.cuda.synchronize()
+        r.g.launch(s)  # between the replays, on its own
+        assert r.right()
+    del outer
+    r.close()
 
 
 @pytest.mark.parametrize("n", SIZES)
