@@ -21,13 +21,16 @@ handles are kept open, so earlier captures stay valid.
 
 An ordinary call on the device (contiguous, on the current device, no gradient
 asked for, the stream's handle in place) runs in csrc/torch_ops.cpp, which
-falls back to the implementations here for all others.
+falls back to the implementations here for all others. Where that library is
+absent or does not load (it is built against one PyTorch), they serve every call,
+12 us slower each.
 """
 from __future__ import annotations
 
 import ctypes
 import threading
-from typing import Dict, List, Tuple
+import warnings
+from typing import Dict, List, Optional, Tuple
 
 import torch
 
@@ -43,12 +46,15 @@ _retired: List[ScanHandle] = []
 _lock = threading.Lock()
 
 
-def _load_kernels() -> ctypes.CDLL:
+def _load_kernels() -> Optional[ctypes.CDLL]:
     """Loads libgps_torch.so, which registers the operators' device kernels."""
     path = _lib.LIB_PATH.with_name("libgps_torch.so")
-    if not path.exists():
-        raise ImportError(f"{path} is not built; run `python -m gpuprefixsums_amd.build`")
-    lib = ctypes.CDLL(str(path))
+    try:
+        lib = ctypes.CDLL(str(path))
+    except OSError as e:
+        warnings.warn(f"gps: the operators run through Python, 12 us slower a call: {e} "
+                      "(`python -m gpuprefixsums_amd.build` builds them for this PyTorch)", RuntimeWarning)
+        return None
     lib.gps_torch_set_handle.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint64]
     lib.gps_torch_set_handle.restype = None
     return lib
@@ -75,8 +81,9 @@ def _handle(x: torch.Tensor, n: int) -> ScanHandle:
             with torch.cuda.device(x.device):
                 h = ScanHandle(ALGO_CSDL, max(n, 1 << 20))
             _handles[key] = h
-            _lib.kept_open.append(h)
-            _kernels.gps_torch_set_handle(*key, h.handle, h.max_n)
+            if _kernels is not None:
+                _lib.kept_open.append(h)
+                _kernels.gps_torch_set_handle(*key, h.handle, h.max_n)
         return h
 
 
