@@ -1292,6 +1292,12 @@ uint32_t pp_resident_workgroups(TileShape s, bool inclusive) {
     return 0;
 }
 
+// From 512 threads on at most 1024 threads per CU, as for csdl_pp_u32: with more
+// workgroups waiting on lookbacks the rate falls apart or not with small changes
+// of the code around them (1024 x 4 at 2^28: 385 us so, 566 to 1790 with two per
+// CU; 1024 x 2 at 2^26 152, 300 to 757; 512 x 4 at 2^28 600, 614 to 776; 512 x 2
+// 1296, 1111 to 1555). Smaller workgroups gain up to 2^26 elements and lose 7-14%
+// at 2^28, so they keep what fits.
 template <int DW, int V, bool I>
 static hipError_t launch_cw(const ScanParams& p, hipStream_t stream) {
     struct Residency {
@@ -1303,6 +1309,7 @@ static hipError_t launch_cw(const ScanParams& p, hipStream_t stream) {
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, csdl_cw_u32<DW, V, I>, 64 * (DW + 1), 0) !=
                 hipSuccess)
                 return;
+            if (DW + 1 >= 8 && per_cu > 16 / (DW + 1)) per_cu = 16 / (DW + 1);
             workgroups = (uint32_t)(cus > 0 ? cus : 1) * (uint32_t)(per_cu > 0 ? per_cu : 1);
         }
     };
