@@ -752,7 +752,7 @@ __device__ __forceinline__ void publish_own_word(const ScanParams& p, uint32_t t
     if (tile != 0 && status_flag(old, epoch) == (uint32_t)kFlagIncl) raise_device_error(p.err, kErrLookbackWatchdog);
 }
 
-template <int BLOCK, int VEC, bool INCL>
+template <int BLOCK, int VEC, bool INCL, int FB>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(VEC >= 8 ? 4 : GPS_WAVES_PER_EU))) void
 csdldf_pp_u32(ScanParams p) {
     using C = TileCfg<BLOCK, VEC>;
@@ -913,10 +913,9 @@ csdldf_pp_u32(ScanParams p) {
 
             // Workgroup-wide redundant reduction of tile j (a full tile: only
             // the last tile is partial and it is nobody's predecessor), FB
-            // vectors per round so that it fits beside the two live tiles.
+            // vectors per round beside the two live tiles.
             const uint32_t j = __builtin_amdgcn_readfirstlane(s_fb_tile);
             {
-                constexpr int FB = VEC < 2 ? VEC : 2;
                 const u32x4_any* v =
                     reinterpret_cast<const u32x4_any*>(p.in + (uint64_t)j * C::kTile + thread_offset<VEC>());
                 uint32_t tsum = 0;
@@ -1373,13 +1372,22 @@ hipError_t launch_csdldf_split_u32(TileShape s, bool inclusive, const ScanParams
     return launch_csdldf_grid(s, inclusive, q, split_tile_count(p.num_tiles, p.stall_period, 2u), stream);
 }
 
-template <int B, int V, bool I>
+// Vectors per round of a fallback: two of them spill 16 of VEC 4's 64 VGPRs,
+// which costs up to 2^25 elements (1024 x 4: 65536 6.0 us, 5.5 with one; 2^25 63.8
+// and 60.2; with period 7 88.2 and 86.0); above, one is slower (2^28 398 and 420;
+// with period 7 655 and 653).
+template <int B, int V, bool I, int FB>
 static hipError_t launch_df_pp(const ScanParams& p, hipStream_t stream) {
-    const uint32_t resident = resident_workgroups<csdldf_pp_u32<B, V, I>, B>();
+    const uint32_t resident = resident_workgroups<csdldf_pp_u32<B, V, I, FB>, B>();
     if (resident == 0) return hipErrorInvalidDevice;
     const uint32_t grid = p.num_tiles < resident ? p.num_tiles : resident;
-    hipLaunchKernelGGL((csdldf_pp_u32<B, V, I>), dim3(grid), dim3(B), 0, stream, p);
+    hipLaunchKernelGGL((csdldf_pp_u32<B, V, I, FB>), dim3(grid), dim3(B), 0, stream, p);
     return hipGetLastError();
+}
+template <int B, int V, bool I>
+static hipError_t launch_df_pp(const ScanParams& p, hipStream_t stream) {
+    return V == 4 && p.n <= (1ull << 25) ? launch_df_pp<B, V, I, V == 4 ? 1 : 2>(p, stream)
+                                         : launch_df_pp<B, V, I, 2>(p, stream);
 }
 
 hipError_t launch_csdldf_pp_u32(TileShape s, bool inclusive, const ScanParams& p, hipStream_t stream) {
