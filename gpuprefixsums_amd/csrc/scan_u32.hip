@@ -1334,13 +1334,22 @@ hipError_t launch_csdl_cw_u32(TileShape s, bool inclusive, const ScanParams& p, 
 // Tiles that stall in place, above 3 * 2^25 elements: half of a 1024 x 8 tile
 // waits in LDS (periods 7 / 2: 2^25 73.5 / 77.5 us so, 72.5 / 76.4 without; 2^26 129 /
 // 146 so, 135 / 141 without; 2^27 235 / 264 so, 259 / 276 without).
+//
+// VEC 4 takes 64 VGPRs, eight waves per SIMD, and is faster with seven: one
+// workgroup less per CU waits on its predecessors. Dynamic LDS, 82 bytes per
+// thread, keeps it out (512 x 4: 2^25 74.6 us so, 79.5 with eight, split period 2
+// 143 and 153; 256 x 4 135 and 139; 1024 x 4, one per CU: 12,345,677 21.4 and
+// 24.2, 2^25 56.9 and 58.5). At 1024 x 4 two are faster above 2^25 (2^28 386
+// against 414) and under stalls, where what is resident sets the pace (2^28
+// period 7: 507, 669 so).
 template <int B, int V, bool I>
 static hipError_t launch_df(const ScanParams& p, uint32_t grid, hipStream_t stream) {
     constexpr int kStash = B == 1024 && V == 8 ? 4 : 0;
+    const bool seven = V == 4 && (B < 1024 || (!p.stall_period && p.n <= (1ull << 25)));
     if (kStash && p.stall_period && !p.split_pass && p.n > (3ull << 25))
         hipLaunchKernelGGL((csdldf_u32<B, V, I, kStash>), dim3(grid), dim3(B), 0, stream, p);
     else
-        hipLaunchKernelGGL((csdldf_u32<B, V, I, 0>), dim3(grid), dim3(B), 0, stream, p);
+        hipLaunchKernelGGL((csdldf_u32<B, V, I, 0>), dim3(grid), dim3(B), seven ? 82 * B : 0, stream, p);
     return hipGetLastError();
 }
 
