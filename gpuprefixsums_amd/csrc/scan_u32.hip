@@ -993,7 +993,10 @@ csdldf_pp_u32(ScanParams p) {
 // carry-in. Reads the input twice (12 B/elem of traffic against 8 B
 // algorithmic), which is what bounds it: 7.1 TB/s over those 12 B at 2^26. Up
 // to kRtsDirect tiles the rescan adds up the sums before its tile by itself (a
-// load per thread and 512 tiles, from L2, beside the tile's own loads);
+// load per thread and BLOCK tiles, from L2, beside the tile's own loads), while
+// those loads are at most sixteen times the tile's vectors (256 x 2 at 2^25, 64
+// sums against 2 vectors: 82.8 us so, 59.7 with a spine; 2^24, 32 sums: 33.4,
+// 34.2 with a narrower one);
 // beyond, one workgroup scans them in between. The reduce loads with the
 // ordinary cache policy, so that the rescan finds part of the input in the
 // Infinity Cache, and the rescan streams past it. Against a spine of 4096
@@ -1413,7 +1416,7 @@ template <int B, int V, bool I>
 static hipError_t launch_rts(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t num_tiles, uint32_t* tile_sums,
                              hipStream_t stream) {
     hipLaunchKernelGGL((rts_reduce_u32<B, V>), dim3(num_tiles), dim3(B), 0, stream, in, n, tile_sums);
-    if (num_tiles <= kRtsDirect) {
+    if (num_tiles <= kRtsDirect && num_tiles <= 16u * B * V) {
         hipLaunchKernelGGL((rts_downsweep_u32<B, V, I, true>), dim3(num_tiles), dim3(B), 0, stream, in, out, n,
                            (const uint32_t*)tile_sums);
         return hipGetLastError();
