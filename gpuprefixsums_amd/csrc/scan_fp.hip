@@ -308,7 +308,12 @@ __device__ __forceinline__ void blocked_to_striped(f32x4 (&x)[VEC], float* slice
 template <int BLOCK, int VEC, bool COMP>
 struct FpTile {
     using C = TileCfg<BLOCK, VEC>;
-    static constexpr uint32_t kSliceFloats = COMP ? C::kWaves * BlockedSlice<VEC>::kFloats : 1u;
+    // At 1024 threads a slice's last row goes without its padding: two
+    // workgroups of 1024 x 4 then fit the 160 KB of a CU, which 256 bytes more
+    // left to one (scan_fp at 2^27 FP32 pairs 225 -> 202 us, BF16 at 2^25 48.3 ->
+    // 42.0). Not at 256 threads, where an eighth workgroup per CU costs 3%.
+    static constexpr uint32_t kSlice = BlockedSlice<VEC>::kFloats - (BLOCK == 1024 ? 4u : 0u);
+    static constexpr uint32_t kSliceFloats = COMP ? C::kWaves * kSlice : 1u;
     f32x4 x[VEC];
     ff lane_carry[COMP ? 1 : VEC];
     ff wave_pre, total;
