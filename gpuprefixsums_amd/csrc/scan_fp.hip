@@ -413,7 +413,7 @@ __global__ __launch_bounds__(BLOCK) void scan_fp(FpParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// One-round FP scan (device_common.hpp): the tile schedule up to kRoundTiles
+// One-round FP scan (device_common.hpp): the tile schedule up to fp_round_tiles()
 // tiles; a single tile takes no ticket and publishes nothing. Back to back,
 // FP32 pairs, against tickets and a chained lookback over lane-striped tiles:
 // 1000 elements 2.6 us (4.1), 2^16 4.6 (4.6), 2^20 6.7 (8.1), 2^22 9.0 (11.5),
@@ -1542,12 +1542,25 @@ static hipError_t launch_fp_pp_carry(int carry, const FpParams& p, hipStream_t s
     return launch_fp_pp<B, V, BF16, PairCarry<false>>(p, stream);
 }
 
+// Most tiles of a one-round scan. Workgroups of 1024 threads are one per CU with
+// pairs (LDS) and at 1024 x 8 (registers), so beyond 256 tiles a second round of
+// them would wait for the first to end, where the ticketed kernel's wait for
+// their predecessors only. FP32 pairs, one round / ticketed: 1024 x 4 300 tiles
+// 13.8 / 12.1 us, 512 16.5 / 17.4, 1024 35.3 / 29.4; 1024 x 8 300 20.4 / 20.1, 800
+// 53.5 / 47.5, 1024 60.0 / 54.9. Plain at 1024 x 8: 512 tiles 26.0 / 27.0, 611
+// 36.0 / 36.9, 800 48.5 / 45.7. The rest gain up to 1024 (plain 1024 x 4 BF16 800 tiles
+// 18.9 / 20.2; 512 x 8 pairs 1024 31.2 / 35.1).
+template <int B, int V, bool COMP>
+constexpr uint32_t fp_round_tiles() {
+    return B < 1024 ? kRoundTiles : COMP ? 256u : V == 8 ? 640u : kRoundTiles;
+}
+
 // One workgroup per tile.
 template <int B, int V, bool BF16, bool COMP>
 static void launch_fp_tile(const FpParams& p, hipStream_t stream) {
     if (p.num_tiles == 1)
         hipLaunchKernelGGL((scan_fp_round<B, V, BF16, COMP, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (p.num_tiles <= kRoundTiles && round_buffers(p.in, (BF16 ? 2u : 4u) * p.n, p.out, 4u * p.n))
+    else if (p.num_tiles <= fp_round_tiles<B, V, COMP>() && round_buffers(p.in, (BF16 ? 2u : 4u) * p.n, p.out, 4u * p.n))
         hipLaunchKernelGGL((scan_fp_round<B, V, BF16, COMP, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((scan_fp<B, V, BF16, COMP>), dim3(p.num_tiles), dim3(B), 0, stream, p);

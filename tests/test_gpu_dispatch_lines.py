@@ -49,3 +49,23 @@ def test_fallback_vec4(words, block, schedule, period):
                         stall_period=period) as h:
         for k, m in enumerate((n, n + 1, n + 5)):
             scan_and_validate(h, words, m, k % 2 == 0)
+
+
+@pytest.mark.parametrize("block,vec", [(1024, 4), (1024, 8)])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("comp", [gps.FP_PAIR, gps.FP_PLAIN], ids=["pair", "plain"])
+def test_fp_round_tiles(block, vec, bf16, comp):
+    """1024 threads: pairs take one round up to 256 tiles, plain ones up to 640 or
+    1024. Sums of -1, 0 and 1 are exact in any order."""
+    tile = block * vec * 4
+    lines = [256] if comp == gps.FP_PAIR else [640 if vec == 8 else 1024]
+    x = torch.randint(-1, 2, ((lines[-1] + 1) * tile,), device="cuda").to(torch.bfloat16 if bf16 else torch.float32)
+    want, out = torch.cumsum(x.double(), 0), torch.empty(x.numel(), device="cuda")
+    with gps.ScanHandle(gps.ALGO_CSDL, x.numel(), block_threads=block, vec_per_thread=vec,
+                        schedule=gps.SCHEDULE_TILE) as h:
+        for k in lines:
+            for n in (k * tile, k * tile + 1, (k + 1) * tile - 3):
+                out.fill_(-7)
+                (h.inclusive_bf16_f32 if bf16 else h.inclusive_f32)(x, out, n, comp)
+                assert torch.equal(out[:n].double(), want[:n]), n
+        assert h.device_error() == 0
