@@ -1516,10 +1516,15 @@ bool fp_shape_supported(TileShape s) {
     return false;
 }
 
+// At most seven waves per SIMD: at VEC 4, where eight fit, one workgroup less per
+// CU is faster, as for csdl_pp_u32 (1024 x 4, one instead of two: 2^23 FP32 15.0 us
+// instead of 20.2, 2^25 52.7 and 56.1; 256 x 4 2^23 53.7 and 58.6, 2^27 437 and 440).
 template <int B, int V, bool BF16, class Ops>
 static hipError_t launch_fp_pp(const FpParams& p, hipStream_t stream) {
-    const uint32_t resident = resident_workgroups<scan_fp_pp<B, V, BF16, Ops>, B>();
-    if (resident == 0) return hipErrorInvalidDevice;
+    const uint32_t fit = resident_workgroups<scan_fp_pp<B, V, BF16, Ops>, B>();
+    if (fit == 0) return hipErrorInvalidDevice;
+    const uint32_t most = device_cus() * (28u / (B / 64));
+    const uint32_t resident = most && most < fit ? most : fit;
     const uint32_t grid = persistent_grid(p.num_tiles, resident);
     hipLaunchKernelGGL((scan_fp_pp<B, V, BF16, Ops>), dim3(grid), dim3(B), 0, stream, p);
     return hipGetLastError();
