@@ -210,7 +210,7 @@ __global__ __launch_bounds__(BLOCK) void csdl_u32x4(V4Params p) {
 
 // ---------------------------------------------------------------------------
 // One-round struct scan (device_common.hpp): the tile schedule up to
-// kRoundTiles tiles; a single tile takes no ticket and publishes nothing.
+// kRoundTiles tiles and kRoundStructs structs; a single tile takes no ticket and publishes nothing.
 // Back to back, against tickets and csdl_u32x4's lookback over 16-tile windows:
 // 1000 structs 3.1 us (4.0), 2^16 5.2 (5.6), 2^18 5.9 (7.3), 1,000,003 8.5
 // (10.8), 2,000,000 12.4 (13.9). Up to some 2^16 structs the 24 DPP steps and
@@ -410,12 +410,17 @@ uint32_t v4_resident_workgroups(TileShape s, bool inclusive) {
     return 0;
 }
 
-// One workgroup per tile.
+// One workgroup per tile; one round up to kRoundTiles tiles and 2^22 structs,
+// where the input is as large as the caches serve (1024 x 8, one workgroup per CU:
+// 512 tiles, 2^22 structs, 27.2 us against 27.1 with tickets, 611 36.3 and 35.6, 1024
+// 57.2 and 52.4; 1024 x 4 and 512 x 8 end at 2^22 with their 1024 tiles, 29.4 and 28.6
+// against 32.0 and 32.2).
+constexpr uint64_t kRoundStructs = 1ull << 22;
 template <int B, int V, bool I>
 static hipError_t launch_tile_v4(const V4Params& p, hipStream_t stream) {
     if (p.num_tiles == 1)
         hipLaunchKernelGGL((csdl_round_u32x4<B, V, I, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (p.num_tiles <= kRoundTiles && round_buffers(p.in, 16u * p.n, p.out, 16u * p.n))
+    else if (p.num_tiles <= kRoundTiles && p.n <= kRoundStructs && round_buffers(p.in, 16u * p.n, p.out, 16u * p.n))
         hipLaunchKernelGGL((csdl_round_u32x4<B, V, I, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((csdl_u32x4<B, V, I>), dim3(p.num_tiles), dim3(B), 0, stream, p);

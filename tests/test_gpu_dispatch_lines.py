@@ -69,3 +69,22 @@ def test_fp_round_tiles(block, vec, bf16, comp):
                 (h.inclusive_bf16_f32 if bf16 else h.inclusive_f32)(x, out, n, comp)
                 assert torch.equal(out[:n].double(), want[:n]), n
         assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("block,vec", [(512, 8), (1024, 4), (1024, 8)])
+@pytest.mark.parametrize("inclusive", [False, True], ids=["excl", "incl"])
+def test_struct_round(words, block, vec, inclusive):
+    """Structs take one round up to 2^22 of them."""
+    x, out = words
+    with gps.ScanHandle(gps.ALGO_CSDL, (1 << 22) + 5, block_threads=block, vec_per_thread=vec,
+                        schedule=gps.SCHEDULE_TILE) as h:
+        for n in (1 << 22, (1 << 22) + 1, (1 << 22) + 5):
+            v = x[:4 * n].view(n, 4).long() & 0xFFFFFFFF
+            want = torch.cumsum(v, 0)
+            if not inclusive:
+                want -= v
+            out.fill_(-7)
+            h.scan_u32x4(x, out, n, inclusive)
+            assert torch.equal(out[:4 * n].view(n, 4).long() & 0xFFFFFFFF, want & 0xFFFFFFFF), n
+            assert bool((out[4 * n:4 * n + 64] == -7).all())
+        assert h.device_error() == 0
