@@ -523,12 +523,22 @@ hipError_t prepare_segscan_u32(TileShape s, bool inclusive, bool persistent) {
     return hipErrorInvalidValue;
 }
 
+// Most tiles of a one-round scan: those that a workgroup's B / 64 waves cover with
+// 64 each and its own. At 1024 x 8 the kernel's 70 and more registers leave one
+// workgroup per CU, and a second round of them would wait for the first to end (257
+// tiles in 100000 segments 24.3 us, 17.7 with tickets, 512 34.3 and 28.9, 1024 68.8
+// and 59.8); at 1024 threads 1025 tiles are slower too (1024 x 2 28.3 and 26.0).
+template <int B, int V>
+constexpr uint32_t seg_round_tiles() {
+    return B == 1024 ? (V == 8 ? 256u : 1024u) : (uint32_t)B + 1u;
+}
+
 // One workgroup per tile.
 template <int B, int V, bool I>
 static hipError_t launch_seg_tile(const SegParams& p, hipStream_t stream) {
     if (p.num_tiles == 1)
         hipLaunchKernelGGL((segscan_round_u32<B, V, I, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (p.num_tiles <= (uint32_t)B + 1u)  // B / 64 waves x 64 tiles
+    else if (p.num_tiles <= seg_round_tiles<B, V>())
         hipLaunchKernelGGL((segscan_round_u32<B, V, I, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((segscan_u32<B, V, I>), dim3(p.num_tiles), dim3(B), 0, stream, p);

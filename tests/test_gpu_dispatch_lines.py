@@ -1,5 +1,8 @@
 """Explicit handles on both sides of the lines where a scan changes its kernel."""
+import numpy as np
 import pytest
+
+import oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -87,4 +90,22 @@ def test_struct_round(words, block, vec, inclusive):
             h.scan_u32x4(x, out, n, inclusive)
             assert torch.equal(out[:4 * n].view(n, 4).long() & 0xFFFFFFFF, want & 0xFFFFFFFF), n
             assert bool((out[4 * n:4 * n + 64] == -7).all())
+        assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("block,vec,line", [(256, 4, 257), (512, 4, 513), (1024, 2, 1024), (1024, 4, 1024), (1024, 8, 256)])
+@pytest.mark.parametrize("segments", [1, 3000])
+def test_segmented_round_tiles(words, block, vec, line, segments):
+    """Segmented scans take one round up to `line` tiles."""
+    x, out = words
+    tile = block * vec * 4
+    with gps.ScanHandle(gps.ALGO_CSDL, (line + 1) * tile, block_threads=block, vec_per_thread=vec,
+                        schedule=gps.SCHEDULE_TILE) as h:
+        for k, n in enumerate((line * tile, line * tile + 1, (line + 1) * tile - 3)):
+            cuts = np.linspace(0, n, segments + 1).astype(np.uint64)
+            off = torch.from_numpy(cuts.view(np.int64)).cuda()
+            out.fill_(-7)
+            h.segmented(x, out, off, segments, n, k % 2 == 0)
+            want = oracle.segmented_scan_u32(x[:n].cpu().numpy().view(np.uint32), cuts, k % 2 == 0)
+            assert np.array_equal(out[:n].cpu().numpy().view(np.uint32), want), n
         assert h.device_error() == 0
