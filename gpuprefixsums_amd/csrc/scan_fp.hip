@@ -1621,12 +1621,23 @@ static hipError_t launch_segfp_pp(const SegFpParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Most tiles of a one-round scan with pairs: those that a workgroup's B / 64 waves
+// cover with 64 each and its own. Workgroups of 1024 threads are one per CU (LDS):
+// at 1024 x 4, of which the ticketed kernel runs two, that one is faster beyond two
+// rounds (16000 segments, one round / ticketed: 512 tiles 21.8 / 23.5 us, 800 40.8 /
+// 35.0, 1025 54.7 / 41.8); 1024 x 8 loses only at 1025 tiles in few segments (75.0 /
+// 68.6 in one; 1024 in 16000 72.6 / 75.2).
+template <int B, int V>
+constexpr uint32_t segfp_round_tiles() {
+    return B == 1024 ? (V == 4 ? 512u : 1024u) : (uint32_t)B + 1u;
+}
+
 // One workgroup per tile.
 template <int B, int V, bool BF16, bool COMP>
 static void launch_segfp_tile(const SegFpParams& p, hipStream_t stream) {
     if (COMP && p.num_tiles == 1)
         hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (COMP && p.num_tiles <= (uint32_t)B + 1u)  // B / 64 waves x 64 tiles
+    else if (COMP && p.num_tiles <= segfp_round_tiles<B, V>())
         hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((segscan_fp<B, V, BF16, COMP>), dim3(p.num_tiles), dim3(B), 0, stream, p);

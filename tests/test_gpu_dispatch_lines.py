@@ -109,3 +109,22 @@ def test_segmented_round_tiles(words, block, vec, line, segments):
             want = oracle.segmented_scan_u32(x[:n].cpu().numpy().view(np.uint32), cuts, k % 2 == 0)
             assert np.array_equal(out[:n].cpu().numpy().view(np.uint32), want), n
         assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("block,vec,line", [(256, 4, 257), (512, 8, 513), (1024, 4, 512), (1024, 8, 1024)])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_segmented_fp_round_tiles(block, vec, line, bf16):
+    """Segmented pair scans take one round up to `line` tiles."""
+    tile, segments = block * vec * 4, 3000
+    x = torch.randint(-1, 2, ((line + 1) * tile,), device="cuda").to(torch.bfloat16 if bf16 else torch.float32)
+    c, out = torch.cumsum(x.double(), 0), torch.empty(x.numel(), device="cuda")
+    with gps.ScanHandle(gps.ALGO_CSDL, x.numel(), block_threads=block, vec_per_thread=vec,
+                        schedule=gps.SCHEDULE_TILE) as h:
+        for n in (line * tile, line * tile + 1, (line + 1) * tile - 3):
+            off = torch.linspace(0, n, segments + 1, dtype=torch.float64, device="cuda").long()
+            before = torch.where(off[:-1] > 0, c[(off[:-1] - 1).clamp(min=0)], torch.zeros_like(c[:segments]))
+            want = c[:n] - torch.repeat_interleave(before, off.diff())
+            out.fill_(-7)
+            h.segmented_fp(x, out, off, segments, n, bf16=bf16, compensated=True)
+            assert torch.equal(out[:n].double(), want), n
+        assert h.device_error() == 0
