@@ -21,7 +21,7 @@ from typing import Optional
 
 import numpy as np
 
-from .space import Config, Workload, candidates, default_config, features, gated_choice
+from .space import Config, Workload, candidates, default_config, features, gated_choice, with_default
 
 DATA = Path(__file__).resolve().parent / "data"
 DEFAULT_MODEL = DATA / "mlp_mi355x.npz"
@@ -54,7 +54,8 @@ class Tuner:
             from .harness import Runner
             self._runner = Runner(max_n=max(w.n, 1 << 10))
         times = self._runner.time_all(w)
-        return Config.parse(min(times, key=times.get))
+        fastest = Config.parse(min(times, key=times.get))
+        return with_default([fastest], default_config(w.dtype, w.segments, w.n, w.stall_period))[0]
 
 
 __all__ = ["Tuner", "Config", "Workload", "candidates", "default_config"]

@@ -20,7 +20,8 @@ import time
 from pathlib import Path
 from typing import Dict
 
-from .space import Config, Workload, c5_workloads, candidates, extra_workloads, stall_workloads
+from .space import (Config, Workload, c5_workloads, candidates, default_config, extra_workloads, stall_workloads,
+                    with_default)
 
 
 class Runner:
@@ -41,12 +42,12 @@ class Runner:
         self.bf16 = self.f32.to(torch.bfloat16).view(torch.int16)
         self.out = torch.empty(max_n, dtype=torch.int32, device=dev)
         self.off = torch.empty(max_segments + 1, dtype=torch.int64, device=dev)
-        self.handles: Dict[Config, object] = {}
+        self.handles: Dict[tuple, object] = {}
         torch.cuda.synchronize()
 
     def handle(self, c: Config, stall_period: int = 0):
         gps = self.gps
-        key = (c, stall_period)
+        key = (c, c.plain, stall_period)
         h = self.handles.get(key)
         if h is None:
             algo, kw = c.handle_args()
@@ -95,16 +96,18 @@ class Runner:
         return statistics.median(out)
 
     def time_all(self, w: Workload, only=None, passes: int = 2) -> Dict[str, float]:
-        """Times every candidate of w (or only those named in `only`): the
-        lower of `passes` medians, each pass over all candidates in turn, so
-        a transient slowdown of the device during one configuration's timing
-        (seen once to make a 20.8 us configuration read 36.9 us) is not taken
-        for its speed."""
+        """Times every candidate of w (or only those named in `only`), the one
+        that stands for the default as a default handle: the lower of `passes`
+        medians, each pass over all candidates in turn, so a transient slowdown
+        of the device during one configuration's timing (seen once to make a
+        20.8 us configuration read 36.9 us) is not taken for its speed."""
         self.stage(w)
         res: Dict[str, float] = {}
         best = float("inf")
+        cands = with_default(candidates(w.dtype, w.stall_period),
+                             default_config(w.dtype, w.segments, w.n, w.stall_period))
         for _ in range(passes):
-            for c in candidates(w.dtype, w.stall_period):
+            for c in cands:
                 if only is not None and c.name not in only:
                     continue
                 t = self.time(w, c, best)

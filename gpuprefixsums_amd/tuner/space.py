@@ -17,6 +17,11 @@ loop_csdl persistent (loop_csdl ":tile": one workgroup per tile, what a
 default handle runs below 2^24 elements), loop_rts and loop_csdldf one
 workgroup per tile.
 
+At each workload the configuration named as the default stands for a default
+handle, which picks kernel, shape and schedule by its own rules
+(Config.plain): it is timed as one and chosen as one, and its name only says
+which of the candidates it resembles.
+
 A second sweep covers the decoupled-fallback scan under emulated deadlock
 (every stall_period-th tile stalled until a successor inserts its
 aggregate): there the choice is the tile shape and the lookback spin limit of
@@ -31,7 +36,7 @@ MAX_SPIN_COUNT (GPUPrefixSumsCUDA/EmulatedDeadlocking.cuh:15).
 from __future__ import annotations
 
 import math
-from dataclasses import dataclass
+from dataclasses import dataclass, field, replace
 from typing import List
 
 import numpy as np
@@ -48,6 +53,7 @@ class Config:
     spin: int = 0
     persistent: bool = False  # FP kinds: the persistent pipelined kernel
     tile: bool = False        # loop_csdl: one workgroup per tile instead of the persistent kernel
+    plain: bool = field(default=False, compare=False)  # run by a default handle, whatever the name says
 
     @property
     def name(self) -> str:
@@ -61,6 +67,8 @@ class Config:
         import gpuprefixsums_amd as gps
         algo = {"batched": gps.ALGO_CSDL, "loop_csdl": gps.ALGO_CSDL, "loop_rts": gps.ALGO_RTS,
                 "loop_csdldf": gps.ALGO_CSDLDF, "loop_fp": gps.ALGO_CSDL, "batched_fp": gps.ALGO_CSDL}[self.kind]
+        if self.plain:
+            return algo, {}
         kw = dict(block_threads=self.block, vec_per_thread=self.vec)
         if self.kind == "loop_csdldf":
             kw["spin_limit"] = self.spin
@@ -105,14 +113,16 @@ def candidates(dtype: str, stall_period: int = 0) -> List[Config]:
 
 
 def default_config(dtype: str, segments: int, n: int = 1 << 30, stall_period: int = 0) -> Config:
-    """What the library does without the tuner: a default handle's choice for
-    n elements (the same rules as libgps's size-adaptive defaults, but for three
-    things: segmented uint32 scans run one workgroup per tile up to 2^23 elements, pair scans run persistent above 2^23 elements, and the segmented FP
-    kernel has 512 x 4 tiles, no candidate, between 2^20 and 9 * 2^18). Under
+    """What the library does without the tuner: a default handle, under the
+    name of the candidate that resembles its choice for n elements. Under
     emulated deadlock it is the default decoupled-fallback handle (1024 x 8,
     spin limit 4)."""
     if stall_period:
         return Config("loop_csdldf", 1024, 8, 4)
+    return replace(_default_name(dtype, segments, n), plain=True)
+
+
+def _default_name(dtype: str, segments: int, n: int) -> Config:
     if dtype != "u32":
         if segments == 1:
             b, v = (256, 4) if n <= 1 << 19 else (1024, 4) if n <= 1 << 22 else (1024, 8)
@@ -131,6 +141,11 @@ def default_config(dtype: str, segments: int, n: int = 1 << 30, stall_period: in
         return Config("loop_csdl", 1024, 8)
     b, v = (1024, 2) if n < 1 << 20 else (1024, 4) if n < 1 << 22 else (1024, 8)
     return Config("batched", b, v)
+
+
+def with_default(cands: List[Config], default: Config) -> List[Config]:
+    """The candidates, with the default in the place of the one it resembles."""
+    return [default if c == default else c for c in cands]
 
 
 def fixed_default_config(dtype: str, segments: int, stall_period: int = 0) -> Config:
