@@ -7,8 +7,8 @@ is the fallback.
                                               [--configs name,name,...]
 
 One JSON line per workload: {"wid", "n", "dtype", "segments", "times_ms": {config: ms}}.
-Each time is the median of a few back-to-back runs bracketed by events on the
-launch stream (fewer repetitions for long runs).
+Each time is the median of a few brackets of events on the launch stream, each
+around enough back-to-back runs to last BRACKET_MS (fewer for long runs).
 """
 from __future__ import annotations
 
@@ -22,6 +22,12 @@ from typing import Dict
 
 from .space import (Config, Workload, c5_workloads, candidates, default_config, extra_workloads, stall_workloads,
                     with_default)
+
+
+# A single run between two events reads up to 2 us too long or too short, more
+# than most configurations differ at a few microseconds.
+BRACKET_MS = 0.2
+MAX_RUNS = 32
 
 
 class Runner:
@@ -78,15 +84,21 @@ class Runner:
     def time(self, w: Workload, c: Config, best_so_far: float = float("inf")) -> float:
         torch = self.torch
         st = torch.cuda.current_stream()
-        self.run(w, c)  # warm-up
-        reps, out = 5, []
-        for r in range(reps):
-            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+
+        def bracket(runs: int) -> float:
             e0.record(st)
-            self.run(w, c)
+            for _ in range(runs):
+                self.run(w, c)
             e1.record(st)
             e1.synchronize()
-            ms = e0.elapsed_time(e1)
+            return e0.elapsed_time(e1) / runs
+
+        self.run(w, c)  # warm-up
+        runs = min(max(int(BRACKET_MS / max(bracket(1), 1e-3)), 1), MAX_RUNS)
+        reps, out = 5, []
+        for r in range(reps):
+            ms = bracket(runs)
             out.append(ms)
             # long or clearly losing configurations need fewer repetitions;
             # "clearly losing" is judged on the fastest run so far, so one
