@@ -81,6 +81,66 @@ def test_small_network_kernels_at_their_edges(D, H, B):
         m.close()
 
 
+def in_order(acc, *terms):
+    """acc + terms[0] + terms[1] + ..., each sum rounded to FP32."""
+    for t in terms:
+        acc = acc + t
+        assert acc.dtype == np.float32
+    return acc
+
+
+def by_chunks(rows, chunk=128):
+    """Sum of rows: each chunk's in increasing row, then the chunks'."""
+    zero = np.zeros_like(rows[0])
+    return in_order(zero, *(in_order(zero, *rows[c:c + chunk]) for c in range(0, len(rows), chunk)))
+
+
+def loss_grad_f32(p, x, t, D, H):
+    """Forward, loss and gradients in FP32, one multiply and one add a term, in
+    the documented order: a unit's inputs, then a chunk's samples, increasing;
+    squared errors per 256 by halves, then those sums in order."""
+    f = np.float32
+    at = np.cumsum([0, H * D, H, H * H, H, H, 1])
+    W1, b1, W2, b2, W3, b3 = (p[a:b] for a, b in zip(at, at[1:]))
+    W1, W2, B = W1.reshape(H, D), W2.reshape(H, H), len(x)
+    z1 = in_order(np.broadcast_to(b1, (B, H)), *(W1[:, i] * x[:, i:i + 1] for i in range(D)))
+    a1 = np.maximum(z1, f(0))
+    z2 = in_order(np.broadcast_to(b2, (B, H)), *(W2[:, i] * a1[:, i:i + 1] for i in range(H)))
+    a2 = np.maximum(z2, f(0))
+    y = in_order(np.broadcast_to(b3, (B,)), *(W3[i] * a2[:, i] for i in range(H)))
+    d = y - t
+    dy = f(2) * d / f(B)
+    e = np.zeros((B + 255) // 256 * 256, f)
+    e[:B] = d * d
+    e = e.reshape(-1, 256)
+    while e.shape[1] > 1:
+        e = e[:, :e.shape[1] // 2] + e[:, e.shape[1] // 2:]
+    loss = in_order(f(0), *e[:, 0]) * (f(1) / f(B))
+    dz2 = np.where(z2 > 0, dy[:, None] * W3, f(0))
+    dz1 = np.where(z1 > 0, in_order(np.zeros((B, H), f), *(dz2[:, o:o + 1] * W2[o] for o in range(H))), f(0))
+    g = [by_chunks(dz1[:, :, None] * x[:, None, :]), by_chunks(dz1), by_chunks(dz2[:, :, None] * a1[:, None, :]),
+         by_chunks(dz2), by_chunks(dy[:, None] * a2), by_chunks(dy)]
+    return y, loss, np.concatenate([np.ravel(a) for a in g])
+
+
+@pytest.mark.parametrize("D,H,B", [(1, 1, 5), (18, 64, 129), (18, 64, 1500), (33, 40, 31), (20, 112, 300), (64, 128, 257),
+                                   (65, 16, 300), (10, 129, 300)])
+def test_order_and_rounding_of_every_sum(D, H, B):
+    """Exactly the FP32 sums of the documented order, from the kernels of small
+    networks and, in the last two sizes, from those of one layer each."""
+    p, x, t = problem(D, H, B, seed=11 * D + H + B)
+    want_y, want_loss, want_g = loss_grad_f32(p, x, t, D, H)
+    m = GpuMlp(D, H, B)
+    try:
+        m.set_params(p)
+        assert np.array_equal(m.forward(x), want_y)
+        loss, g = m.loss_grad(x, t)
+        assert np.float32(loss) == want_loss
+        assert np.array_equal(g, want_g), np.flatnonzero(g != want_g)[:8]
+    finally:
+        m.close()
+
+
 def test_training_reduces_loss_and_fits():
     rng = np.random.default_rng(3)
     X = rng.uniform(-2, 2, size=(4000, 6))
