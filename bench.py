@@ -15,7 +15,7 @@ periods 0/7/8, one workgroup per tile and persistent), copy (the read-n + write-
 (copies and one-way streams of the same 2 GiB with other access patterns, the
 runtime's copy and fill), vendor (rocPRIM's device
 scan, the reference's CUB comparator on ROCm), n2p20 (latency at 2^20),
-segmented (4096 log-normal segments in one graph-launched pass) and
+segmented (4096 log-normal segments in one launch, and that launch replayed) and
 segmented_loop (the same as one launch per segment), segmented_fp and
 segmented_fp_loop (the same segments over FP32: one segmented FP launch, and
 one launch per segment), fp (n = 2^27 FP32/BF16 with and without compensated carries,
@@ -226,8 +226,9 @@ class Legs:
 
     def segmented(self, out):
         """C3: 4096 log-normal segments of values uniform in [0, 1023] (seed 3),
-        exclusive, in one launch: launched directly, and replayed from a
-        hipGraph (the form a serving loop would use)."""
+        exclusive, in one launch: through the call, and as a replay of the
+        recorded launch (gps_graph_launch, which launches the kernel itself;
+        the form a serving loop would use)."""
         gps, torch, oracle, np = self.gps, self.torch, self.oracle, self.np
         S, off, n, d_off = self._c3_segments()
         x = torch.from_numpy(oracle.gen_u32(3, n, 10).view(np.int32)).to("cuda")

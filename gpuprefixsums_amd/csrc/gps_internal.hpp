@@ -100,9 +100,13 @@ bool shape_supported(TileShape s);
 // persistent grid, which has too few tiles per workgroup to pay for its ramp;
 // up to 3 * 2^20 smaller tiles also occupy more of the chip (2,500,000: 6.0
 // against 6.9 us for 1024 x 8; 3,500,000 6.7 against 7.2, with three inputs in
-// turn 8.1 against 7.9). 2^20: 5.1 us; 2^23:
-// 11.4 against 14.5; 12,345,677: 17.9 against 18.2; just below 2^24 24.1
-// against 23.0. Leaves shape and schedule unchanged there.
+// turn 8.1 against 7.9). 2^20: 5.1 us; 2^23: 11.4 against 14.5 persistent;
+// 12,345,677: 17.6 against 18.0. From there to 2^24 it depends on where the input
+// is: one input again and again, from the Infinity Cache, is faster on the
+// persistent grid (13,500,000 19.0 against 20.6 us, just below 2^24 22.6 against
+// 23.9), six inputs in turn, from memory, in one round (21.7 against 22.6, 25.7
+// against 25.8). The line is drawn for the latter. Leaves shape and schedule
+// unchanged from 2^24 on.
 inline void size_adaptive_config(uint64_t n, TileShape& shape, uint32_t& schedule) {
     constexpr uint32_t kTile = 1;  // GPS_SCHEDULE_TILE
     if (n <= (1ull << 18)) {

@@ -527,8 +527,9 @@ __global__ __launch_bounds__(BLOCK) void scan_fp_round(FpParams p) {
 // resident workgroups loop over ticketed tiles; with tile i scanned and its
 // aggregate published, a workgroup takes its next ticket and issues tile
 // i+1's loads, then resolves tile i's lookback and stores tile i. The carry
-// arithmetic comes from a policy, PairCarry<COMP> (pair or plain floats),
-// with the same per-level operations and order as scan_fp.
+// arithmetic comes from a policy, PairCarry<COMP> (pair or plain floats);
+// launched with plain ones, whose per-level operations and order are scan_fp's
+// (pairs run scan_fp_bl).
 //
 // 2^27 FP32 / BF16 elements at 1024 x 8: pairs 4998 / 4433 GB/s against
 // 4787 / 4009 for one workgroup per tile, plain 5567 / 5285 against 5383 /
@@ -1038,7 +1039,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
 
 // ---------------------------------------------------------------------------
 // Persistent FP scan over lane-blocked runs (GPS_SCHEDULE_PERSISTENT with
-// pair carries; the default above 2^24 elements).
+// pair carries; the default for them above 2^23 elements).
 //
 // scan_fp_pp pays one pair wave scan per uint4 vector: VEC scans of 64 lane
 // totals per wave run, about 60 VALU instructions each, most of the pair
