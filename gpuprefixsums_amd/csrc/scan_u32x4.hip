@@ -210,12 +210,14 @@ __global__ __launch_bounds__(BLOCK) void csdl_u32x4(V4Params p) {
 
 // ---------------------------------------------------------------------------
 // One-round struct scan (device_common.hpp): the tile schedule up to
-// kRoundTiles tiles and kRoundStructs structs; a single tile takes no ticket and publishes nothing.
+// kRoundTiles tiles and kRoundStructs structs; a single tile takes no ticket and
+// publishes nothing.
 // Back to back, against tickets and csdl_u32x4's lookback over 16-tile windows:
 // 1000 structs 3.1 us (3.4), 2^16 4.9 (5.6), 2^18 5.7 (7.9), 1,000,003 8.4
-// (11.3), 2,000,000 12.0 (14.6); six inputs in turn 9.3 (11.4) and 13.9 (14.9). Up to some 2^16 structs the 24 DPP steps and
-// 12 adds of every vector, 1 us of each CU, weigh as much as the memory;
-// runs of whole structs per lane would trade them for as many LDS cycles.
+// (11.3), 2,000,000 12.0 (14.6); six inputs in turn 9.3 (11.4) and 13.9 (14.9).
+// Up to some 2^16 structs the 24 DPP steps and 12 adds of every vector, 1 us of
+// each CU, weigh as much as the memory; runs of whole structs per lane would
+// trade them for as many LDS cycles.
 // ---------------------------------------------------------------------------
 // Member sums of tile j (a full one of TILE structs) by one wave; lane l
 // returns member l % 4.
