@@ -401,7 +401,8 @@ int gps_inclusive_scan_fp_per_segment(gps_handle* h, const void* d_in, float* d_
 // elements 75.6 against 79.7 us a replay). A stream that is being captured
 // records it, where hipGraphLaunch reports success and records nothing. The
 // graph is launched where another device is current than its own, or an error
-// of an earlier HIP call is pending, which the launch would return as its own.
+// of an earlier HIP call is pending, which the launch would return as its own;
+// into a capture such a replay is refused.
 int gps_graph_launch(gps_graph* g, void* stream) {
     if (!g || !g->exec) return fail(GPS_ERR_INVALID, "null graph");
     const hipStream_t s = static_cast<hipStream_t>(stream);
@@ -410,6 +411,10 @@ int gps_graph_launch(gps_graph* g, void* stream) {
         HIP_TRY(g->launch(s));
         return GPS_OK;
     }
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
+        return fail(GPS_ERR_HIP, "a capture cannot record the replay: another device is current or an earlier HIP "
+                                 "call's error is pending");
     HIP_TRY(hipGraphLaunch(g->exec, s));
     return GPS_OK;
 }

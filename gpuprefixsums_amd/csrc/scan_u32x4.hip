@@ -174,8 +174,8 @@ __global__ __launch_bounds__(BLOCK) void csdl_u32x4(V4Params p) {
     const uint32_t tile = __builtin_amdgcn_readfirstlane(s_ticket[0]),
                    epoch = __builtin_amdgcn_readfirstlane(s_ticket[1]);
     u32x4 d[VEC];
-    // More than kRoundTiles tiles stream past the caches, and structs are 16-byte
-    // aligned. Through load_tile's streaming path, whose instructions differ in
+    // What is too large for one round streams past the caches, and structs are
+    // 16-byte aligned. Through load_tile's streaming path, whose instructions differ in
     // their addresses only, 1024 x 4 takes 442 us at 2^26, 361 so (2^23: 62, 56.6).
     if ((uint64_t)(tile + 1u) * (BLOCK * VEC) <= p.n) {
         const u32x4* const v = reinterpret_cast<const u32x4*>(p.in) +

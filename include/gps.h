@@ -151,7 +151,8 @@ int gps_segmented_scan_u32_per_segment(gps_handle* h, const uint32_t* d_in, uint
 
 /* A hipGraph holding one gps_segmented_scan_u32 call with fixed arguments
  * (captured on a private stream); a replay on its device launches that one
- * kernel itself, also into a stream that is being captured. Replays reuse the handle's status words
+ * kernel itself, also into a stream that is being captured (not with an earlier
+ * HIP call's error pending). Replays reuse the handle's status words
  * through their epochs; after 2^30 - 1 replays call gps_reset first. */
 typedef struct gps_graph gps_graph;
 int gps_segmented_graph_create(gps_handle* h, const uint32_t* d_in, uint32_t* d_out, const uint64_t* d_offsets,

@@ -80,3 +80,23 @@ def test_replay_with_an_error_pending(n):
         assert hip.hipGetLastError() == pending  # still the caller's
         assert r.right()
     r.close()
+
+
+def test_capture_with_an_error_pending_is_refused():
+    """hipGraphLaunch would record nothing and report success."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    r = Replay(SIZES[0])
+    s = torch.cuda.Stream()
+    outer = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(outer, stream=s):
+        r.out.fill_(-7)
+        assert hip.hipSetDevice(999) != 0
+        pending = hip.hipPeekAtLastError()
+        with pytest.raises(gps.GpsError, match="pending"):
+            r.g.launch(s)
+        assert hip.hipGetLastError() == pending
+        r.g.launch(s)
+    outer.replay()
+    assert r.right()
+    del outer
+    r.close()
