@@ -1638,7 +1638,8 @@ template <int B, int V, bool BF16, bool COMP>
 static void launch_segfp_tile(const SegFpParams& p, hipStream_t stream) {
     if (COMP && p.num_tiles == 1)
         hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (COMP && p.num_tiles <= segfp_round_tiles<B, V>())
+    else if (COMP && p.num_tiles <= segfp_round_tiles<B, V>() &&
+             round_buffers(p.in, (BF16 ? 2u : 4u) * p.n, p.out, 4u * p.n))
         hipLaunchKernelGGL((segscan_fp_round<B, V, BF16, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((segscan_fp<B, V, BF16, COMP>), dim3(p.num_tiles), dim3(B), 0, stream, p);

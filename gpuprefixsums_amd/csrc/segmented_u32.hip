@@ -538,7 +538,7 @@ template <int B, int V, bool I>
 static hipError_t launch_seg_tile(const SegParams& p, hipStream_t stream) {
     if (p.num_tiles == 1)
         hipLaunchKernelGGL((segscan_round_u32<B, V, I, true>), dim3(1), dim3(B), 0, stream, p);
-    else if (p.num_tiles <= seg_round_tiles<B, V>())
+    else if (p.num_tiles <= seg_round_tiles<B, V>() && round_buffers(p.in, 4u * p.n, p.out, 4u * p.n))
         hipLaunchKernelGGL((segscan_round_u32<B, V, I, false>), dim3(p.num_tiles), dim3(B), 0, stream, p);
     else
         hipLaunchKernelGGL((segscan_u32<B, V, I>), dim3(p.num_tiles), dim3(B), 0, stream, p);

@@ -83,3 +83,37 @@ def test_carry_in_inside_the_output(name, place):
             assert np.array_equal(got, want), (n, first_mismatch(got, want))
             assert int(after.item()) & 0xFFFFFFFF == int(want[-1])
         assert h.device_error() == 0
+
+
+def cuts_of(n):
+    """Segments none of which begins where a tile does, so that every tile
+    waits for the one before it."""
+    return np.array([0, *(c for c in (3, 5000, 8191, 100001, 700001) if c < n), n], dtype=np.uint64)
+
+
+@pytest.mark.parametrize("name", HANDLES)
+@pytest.mark.parametrize("whole", [True, False], ids=["one", "several"])
+def test_shifted_segmented_u32(name, whole):
+    with gps.ScanHandle(gps.ALGO_CSDL, max(SIZES), **HANDLES[name]) as h:
+        for k, n in enumerate(SIZES):
+            x, inclusive = oracle.gen_u32(k, n, 32), k % 2 == 0
+            off = np.array([0, n], np.uint64) if whole else cuts_of(n)
+            buf = to_dev(np.r_[np.zeros(1, np.uint32), x])
+            h.segmented(buf[1:], buf[:-1], to_dev(off), off.size - 1, n, inclusive)
+            got, want = u32(buf[:-1]), oracle.segmented_scan_u32(x, off, inclusive)
+            assert np.array_equal(got, want), (n, first_mismatch(got, want))
+        assert h.device_error() == 0
+
+
+@pytest.mark.parametrize("name", HANDLES)
+@pytest.mark.parametrize("comp", [gps.FP_PAIR, gps.FP_PLAIN], ids=["pair", "plain"])
+def test_shifted_segmented_f32(name, comp):
+    with gps.ScanHandle(gps.ALGO_CSDL, max(SIZES), **HANDLES[name]) as h:
+        for k, n in enumerate(SIZES):
+            x, off = np.random.default_rng(k).integers(-1, 2, n).astype(np.float32), cuts_of(n)
+            buf = to_dev(np.r_[np.zeros(1, np.float32), x])
+            h.segmented_fp(buf[1:], buf[:-1], to_dev(off), off.size - 1, n, False, comp)
+            torch.cuda.synchronize()
+            want = np.concatenate([np.cumsum(x[int(a):int(b)], dtype=np.float64) for a, b in zip(off, off[1:])])
+            assert np.array_equal(buf[:-1].cpu().numpy(), want), n
+        assert h.device_error() == 0
